@@ -4,51 +4,62 @@
 // products, :761-879 near field, :911 and :928 the switch) stores U only and
 // evaluates every coupling block B_ij and near-field block D_ij from the
 // shell pairs at each matvec, through H2ERI_calc_ERI_pairs_to_mat
-// (src/CMS.c:387-451).  Here the same blocks are evaluated on the device:
+// (src/CMS.c:387-451).  Here the blocks' products with their inputs are
+// evaluated on the device without ever forming an integral:
 //
-//  * Row tasks.  Every output row has one writer: a task owns one shell pair
-//    a of one node n on one side (the node's full leaf rows, or its skeleton
-//    rows, J_row) and walks every partner block of that side, evaluating each
-//    shell quartet (a|b) and contracting it with the partner's input at once.
-//    Side rules of the reference's three coupling cases
-//    (src/H2ERI_matvec.c:455-545): node n is on its skeleton side against an
-//    admissible partner m when level(n) >= level(m), else on its full side
-//    (n is then a leaf).  Full rows are x-indexed and receive the near field
-//    (the leaf itself and its inadmissible partners, both orientations) and
-//    the coupling products of case (2)/(3) leaves; skeleton rows are y1 of
-//    the node.  A block (n, m) is so evaluated once from each side, against
-//    the reference's once with a bi-GEMV: twice the integrals, in exchange
-//    for no atomics and a fixed summation order (bit-reproducible results).
-//  * The integrals: McMurchie-Davidson (Helgaker, Jorgensen & Olsen,
-//    Molecular Electronic-Structure Theory, eqs. 9.5.x and 9.9.33),
+//  * Sides.  A list of shell pairs is one side of a node: its full leaf rows,
+//    or its skeleton rows (J_row).  Side rules of the reference's three
+//    coupling cases (src/H2ERI_matvec.c:455-545): node n is on its skeleton
+//    side against an admissible partner m when level(n) >= level(m), else on
+//    its full side (n is then a leaf).  Full rows are x-indexed and receive
+//    the near field (the leaf itself and its inadmissible partners, both
+//    orientations) and the coupling products of case (2)/(3) leaves;
+//    skeleton rows are y1 of the node.  Every output row has one writer: a
+//    block (n, m) is evaluated once from each side, against the reference's
+//    once with a bi-GEMV, in exchange for no atomics and a fixed summation
+//    order (bit-reproducible results).
+//  * The product of a block with its input in a Hermite Gaussian basis.  In
+//    McMurchie-Davidson form (Helgaker, Jorgensen & Olsen, Molecular
+//    Electronic-Structure Theory, eqs. 9.5.x and 9.9.33)
 //    (ab|cd) = sum_{ij} 2 pi^{5/2} / (p q sqrt(p+q)) K_i K_j
 //              sum_{tuv} E^{ab}_{tuv} sum_{tau nu phi} (-1)^{tau+nu+phi}
-//              E^{cd}_{tau nu phi} R_{t+tau, u+nu, v+phi}(alpha, PQ)
-//    with Hermite coefficients E from their two-term recurrences, Hermite
-//    Coulomb integrals R from R^{(n)}_{000} = (-2 alpha)^n F_n(alpha |PQ|^2)
-//    and R^{(n)}_{t+1,u,v} = t R^{(n+1)}_{t-1,u,v} + X_PQ R^{(n+1)}_{t,u,v},
-//    and the Boys function of the host engine (the same table).  One wave
-//    evaluates one quartet, or a few kets of one class against its bra pair
-//    (jit_task): lanes over primitive quartets for the E and R tables (in
-//    LDS), then lanes over the Cartesian components, each summing its
-//    component over the primitive quartets in a fixed order.  Shells up to
-//    d (cc-pVDZ); the primitive pairs, centres and conventions are the host
-//    engine's (first shell of a pair = N, row index n * nbf(M) + m,
-//    lexicographic Cartesians).
+//              E^{cd}_{tau nu phi} R_{t+tau, u+nu, v+phi}(alpha, PQ),
+//    and sum_cd (ab|cd) x_cd separates: the input is first contracted with
+//    the ket's E into a Hermite density H_j per primitive (once per side,
+//    not once per bra), each bra primitive i collects the Hermite potential
+//    V_i = sum_j R H_j / sqrt(p+q), and the rows are E^{ab} V_i (the density
+//    form of the J build: Ahmadi & Almlof, Chem. Phys. Lett. 246, 364 (1995);
+//    White & Head-Gordon, J. Chem. Phys. 104, 2620 (1996)).  A primitive
+//    quartet costs its Boys values, the R recursion and one product of
+//    nherm(L_ab) x nherm(L_cd) terms; no Cartesian component is formed.
+//  * Centres.  The primitives of a side with equal exponent sum, centre and
+//    total order are one Hermite centre (contracted s shells of one atom
+//    share their exponents: 289 s-s primitives of a C-C pair in cc-pVDZ are
+//    81 centres).
+//  * R^{(n)}_{000} = (-2 alpha)^n F_n(alpha |PQ|^2), R^{(n)}_{t+1,u,v} =
+//    t R^{(n+1)}_{t-1,u,v} + X_PQ R^{(n+1)}_{t,u,v}, in registers, with the
+//    Boys function from a table in LDS.  Shells up to d (cc-pVDZ); the
+//    primitive pairs, centres and conventions are the host engine's (first
+//    shell of a pair = N, row index n * nbf(M) + m, lexicographic
+//    Cartesians).
 //  * Sweeps: the up sweep (y0 = U^T x, children first) and the down sweep
 //    (parents first) are one launch per tree level over the nodes of that
 //    level, with U in FP64.
 //
-// Sequence of one matvec: zero y1 and the row outputs, up sweep, the row
-// tasks (they need y0), down sweep (it needs y1), y = down-sweep rows + row
-// task rows.
+// Sequence of one matvec: zero y1 and the row outputs, up sweep, Hermite
+// densities of every side (they need y0), potentials, rows, down sweep (it
+// needs y1), y = down-sweep rows + block rows.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cmath>
+#include <cstring>
+#include <map>
 #include <numeric>
 #include <thread>
+#include <unordered_map>
 #include <utility>
 #include <vector>
 
@@ -56,147 +67,77 @@
 
 namespace h2e {
 
-static const int JIT_LMAX = 2;     // shell angular momentum (d)
-static const int JIT_LDS = 2048;   // LDS doubles of a task with a bra or ket pair of la + lb >= 3
-static const int JIT_LDS_S = 1280; // LDS doubles of a task whose pairs all have la + lb <= 2
-static const int JIT_NAB = 36;     // Cartesian rows of a shell pair, at most
-static const int JIT_KMAX = 4;     // kets per pass, at most (8 and 16: 1% slower)
-static const int JIT_PASSQ = 64;   // primitive quartets of a multi-ket pass, at most
+static const int JIT_LMAX = 2;      // shell angular momentum (d)
+static const int JIT_OMAX = 4;      // order of a pair (la + lb)
+static const int JIT_NORD = JIT_OMAX + 1;
+static const int JIT_NLT = 2 * JIT_OMAX + 1;   // total orders of a quartet
+static const int JIT_WPG = 4;       // waves (tasks) per workgroup of the potential kernels
 
-// Everything a row task reads or writes; the pointers are device or, in the
+// Boys table: T in [0, 40) in 640 intervals of 1/16; per interval eight
+// doubles, the seven coefficients of F_m in powers of (T0 - T), T0 the
+// interval's midpoint, and exp(-T0).  40,960 bytes per order, four tables to
+// the 160 KB of LDS of a CU.
+static const int JIT_BGRID = 640;
+static const int JIT_BROW = 8;
+static const double JIT_BTMAX = 40.0;
+
+// One wave's work: the potential of n centres (from global centre c0, order
+// la) against the centres of order lb in segments [s0, s1), bw = 2^lbw lanes
+// per centre group (64 / bw slices share the segments' centres); partial
+// potentials nherm(la) x bw into part[poff].
+struct JitTask {
+    int cls;        // la * JIT_NORD + lb
+    int c0, n, lbw;
+    int s0, s1;
+    long long poff;
+};
+// Centres [c0, c0 + n) of order la: the sum of its tasks' partials, in order.
+struct JitChunk {
+    int la, c0, n, lbw;
+    int t0, t1;     // in ctask
+};
+
+// Everything the kernels read or write; the pointers are device or, in the
 // emulator, host arrays.
 struct JitView {
-    int N;
+    int N, ncen, nent;
     const int *pinfo;     // per shell pair: la, lb, primitive pairs, first primitive
     const double *pgeo;   // per shell pair: A (3), B (3)
     const double *prim;   // per primitive pair: p, P (3), K, 1/(2p)
-    const double *boys;   // Boys table [grid][bcol]
-    int bgrid, bcol;
-    double bstep, btmax, inv_bstep;
-    const int *kl_pair, *kl_moff;     // per partner-list entry: shell pair, its input map
-    const int *kmap;                  // input index per column (-1: not used)
-    const int *t_pair, *t_e0, *t_e1;  // per task: bra pair, its range of gent
-    const int *gent;                  // partner list entries of the tasks
-    double *part;                     // per task: the partial rows (JIT_NAB doubles)
-    // output rows of one bra pair on one side = the sum of its tasks' partials
-    const int *r_pair, *r_omap, *r_t0, *r_t1, *r_tasks;
-    const int *omap;                  // output index per row (-1: not written)
+    const double *boys;   // Boys tables by total order
+    const int *kl_pair, *kl_moff;     // per side entry: shell pair, its row map
+    const int *kmap;                  // index per row (< N: x / y, else y0 / y1; -1: not used)
+    const int *e_c0, *ecen;           // per entry: first of its primitives' centres in ecen
+    const int *cptr, *cent, *cprim;   // per centre: its contributions (entry, primitive)
+    const double *cgeo;               // per centre: p, P (3)
+    int coff[JIT_NORD + 1];           // first centre of each order
+    long long hoff[JIT_NORD];         // its first Hermite coefficient
+    double *H, *V;                    // Hermite densities and potentials by centre
+    const JitTask *tasks;
+    const int *segs;                  // (first, end) centre per segment
+    const JitChunk *chunks;
+    const long long *cpoff;           // per chunk and task: its partials in part
+    double *part;
+    const int *oent;                  // entries with output rows, by class
     const double *X, *Y0;             // inputs: index < N in X, else Y0[index - N]
     double *YJ, *Y1;                  // outputs: index < N in YJ, else Y1[index - N]
 };
 
-__host__ __device__ inline void jit_sync() {
-#ifdef __HIP_DEVICE_COMPILE__
-    __syncthreads();
-#endif
-}
-
-__host__ __device__ inline int jit_ncart(int L) { return (L + 1) * (L + 2) / 2; }
+__host__ __device__ constexpr int jit_ncart(int L) { return (L + 1) * (L + 2) / 2; }
 __host__ __device__ constexpr int jit_nherm(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
-// index of the Hermite (or Cartesian) triple (t, u, v) among all triples of
-// total order <= t+u+v, lexicographic within an order
+// index of the Hermite triple (t, u, v) among all triples of total order
+// <= t+u+v, lexicographic within an order
 __host__ __device__ constexpr int jit_herm(int t, int u, int v) {
     const int k = t + u + v, a = k - t;
     return k * (k + 1) * (k + 2) / 6 + a * (a + 1) / 2 + v;
 }
-// exponents of the k-th lexicographic Cartesian component of order L
-__host__ __device__ constexpr void jit_cart(int L, int k, int &lx, int &ly, int &lz) {
+// exponent in direction dir of the k-th lexicographic Cartesian component of order L
+__host__ __device__ constexpr int jit_cexp(int L, int k, int dir) {
     int a = 0;
     while ((a + 1) * (a + 2) / 2 <= k) a++;
-    lx = L - a;
-    ly = a - (k - a * (a + 1) / 2);
-    lz = L - lx - ly;
+    const int lx = L - a, ly = a - (k - a * (a + 1) / 2);
+    return dir == 0 ? lx : (dir == 1 ? ly : L - lx - ly);
 }
-
-// Index tables of the Hermite recursion, fixed at compile time: for each
-// Hermite triple h = 1..nherm(8)-1 in jit_herm order, the step that builds
-// it (R^{(n)}_h = X_dir R^{(n+1)}_{h1} + c R^{(n+1)}_{h2}); jit_herm of every
-// triple of order <= 8 (-1 above); 1/k! and 1/(2m-1).
-// Also: for each pair class (la, lb) and Cartesian pair index ab, the
-// offsets of its E rows in the pair's table (x, y, z) and its orders per
-// direction (packed 4 bits each); and magic[d] = ceil(2^32 / d) (2^32 for
-// d = 1, so 64 bits), so that x / d = (x magic[d]) >> 32 exactly for
-// x d < 2^32.
-struct JitTabs {
-    int rstep[165][4];   // h1, h2 (-1: none), c, direction
-    short herm[9][9][9];
-    double inv_fact[8];
-    double inv_odd[10];
-    short eoff[100][4];  // pair classes in (la, lb) order, each nab rows
-    short pcoff[9];      // first eoff row of pair class la * 3 + lb
-    unsigned long long magic[1297];
-    constexpr JitTabs() : rstep{}, herm{}, inv_fact{}, inv_odd{}, eoff{}, pcoff{}, magic{} {
-        int row = 0;
-        for (int la = 0; la <= 2; la++)
-            for (int lb = 0; lb <= 2; lb++) {
-                pcoff[la * 3 + lb] = (short)row;
-                const int L = la + lb, esd = (la + 1) * (lb + 1) * (L + 1);
-                const int na = (la + 1) * (la + 2) / 2, nb = (lb + 1) * (lb + 2) / 2;
-                for (int ia = 0; ia < na; ia++)
-                    for (int ib = 0; ib < nb; ib++, row++) {
-                        int ax = 0, ay = 0, az = 0, bx = 0, by = 0, bz = 0;
-                        jit_cart(la, ia, ax, ay, az);
-                        jit_cart(lb, ib, bx, by, bz);
-                        eoff[row][0] = (short)((ax * (lb + 1) + bx) * (L + 1));
-                        eoff[row][1] = (short)((ay * (lb + 1) + by) * (L + 1) + esd);
-                        eoff[row][2] = (short)((az * (lb + 1) + bz) * (L + 1) + 2 * esd);
-                        eoff[row][3] = (short)((ax + bx) | ((ay + by) << 4) | ((az + bz) << 8));
-                    }
-            }
-        for (int d = 1; d < 1297; d++) magic[d] = (0x100000000ULL + (unsigned long long)d - 1) / (unsigned long long)d;
-        for (int t = 0; t < 9; t++)
-            for (int u = 0; u < 9; u++)
-                for (int w = 0; w < 9; w++) herm[t][u][w] = (short)(t + u + w <= 8 ? jit_herm(t, u, w) : -1);
-        for (int k = 1; k <= 8; k++)
-            for (int t = k; t >= 0; t--)
-                for (int u = k - t; u >= 0; u--) {
-                    const int w = k - t - u, h = jit_herm(t, u, w);
-                    int h1 = 0, h2 = -1, c = 0, d = 0;
-                    if (t > 0) { h1 = jit_herm(t - 1, u, w); c = t - 1; d = 0; if (c > 0) h2 = jit_herm(t - 2, u, w); }
-                    else if (u > 0) { h1 = jit_herm(t, u - 1, w); c = u - 1; d = 1; if (c > 0) h2 = jit_herm(t, u - 2, w); }
-                    else { h1 = jit_herm(t, u, w - 1); c = w - 1; d = 2; if (c > 0) h2 = jit_herm(t, u, w - 2); }
-                    rstep[h][0] = h1; rstep[h][1] = h2; rstep[h][2] = c; rstep[h][3] = d;
-                }
-        double f = 1.0;
-        for (int k = 0; k < 8; k++) { inv_fact[k] = 1.0 / f; f *= (double)(k + 1); }
-        inv_odd[0] = 0.0;
-        for (int m = 1; m < 10; m++) inv_odd[m] = 1.0 / (double)(2 * m - 1);
-    }
-};
-__constant__ JitTabs jit_tabs_dev = JitTabs();
-static constexpr JitTabs jit_tabs_host = JitTabs();
-__host__ __device__ inline const JitTabs &jit_tabs() {
-#ifdef __HIP_DEVICE_COMPILE__
-    return jit_tabs_dev;
-#else
-    return jit_tabs_host;
-#endif
-}
-
-// F_m(T) for m = 0..mmax into out[m * stride]: the host engine's method
-// (Taylor expansion of the tabulated grid for T <= tmax, downward
-// recursion; erf and upward recursion above).
-__host__ __device__ inline void jit_boys(const JitView &v, int mmax, double T, double *out, int stride) {
-    if (T <= v.btmax) {
-        const int gi = (int)(T * v.inv_bstep + 0.5);
-        const double dT = gi * v.bstep - T;
-        const double *row = v.boys + (size_t)gi * v.bcol;
-        const JitTabs &tb = jit_tabs();
-        double f = 0.0, pw = 1.0;
-        for (int k = 0; k < 8; k++) {
-            f += row[mmax + k] * pw * tb.inv_fact[k];
-            pw *= dT;
-        }
-        out[mmax * stride] = f;
-        const double eT = exp(-T);
-        for (int m = mmax; m > 0; m--) out[(m - 1) * stride] = (2.0 * T * out[m * stride] + eT) * tb.inv_odd[m];
-    } else {
-        const double eT = exp(-T), inv2T = 0.5 / T;
-        out[0] = 0.5 * sqrt(M_PI / T) * erf(sqrt(T));
-        for (int m = 0; m < mmax; m++) out[(m + 1) * stride] = ((2 * m + 1) * out[m * stride] - eT) * inv2T;
-    }
-}
-
 // Components of the Hermite triple of index h (inverse of jit_herm).
 __host__ __device__ constexpr int jit_hcomp(int h, int which) {
     for (int k = 0; k <= 8; k++)
@@ -212,127 +153,65 @@ struct JitSum {   // index of the triple sum and the sign of the ket triple
     static constexpr int idx = jit_herm(t1 + t2, u1 + u2, w1 + w2);
     static constexpr bool neg = ((t2 + u2 + w2) & 1) != 0;
 };
-template <int H1, int... H2>
-__host__ __device__ inline double jit_inner(const double *R, const double *ec, std::integer_sequence<int, H2...>) {
-    return (0.0 + ... + (ec[H2] * R[JitSum<H1, H2>::idx]));
-}
-template <int... H2>
-__host__ __device__ inline void jit_ket_e(const double *Eb, int px, int py, int pz, double *ec,
-                                          std::integer_sequence<int, H2...>) {
-    ((ec[H2] = (JitSum<0, H2>::neg ? -1.0 : 1.0) * Eb[px + JitSum<0, H2>::t2] * Eb[py + JitSum<0, H2>::u2] *
-               Eb[pz + JitSum<0, H2>::w2]),
-     ...);
-}
-template <int LCD, int... H1>
-__host__ __device__ inline double jit_outer(const double *Ea, int ox, int oy, int oz, const double *R, const double *ec,
-                                            std::integer_sequence<int, H1...>) {
-    return (0.0 + ... +
-            (Ea[ox + JitSum<H1, 0>::t1] * Ea[oy + JitSum<H1, 0>::u1] * Ea[oz + JitSum<H1, 0>::w1] *
-             jit_inner<H1>(R, ec, std::make_integer_sequence<int, jit_nherm(LCD)>{})));
-}
-// One component on one primitive quartet: sum over the bra Hermite triples
-// of total order <= LAB and the ket triples of order <= LCD, every R index a
-// compile-time constant.  The E rows hold zeros beyond each component's own
-// order, so the triples outside a component's box add nothing.
-template <int LAB, int LCD>
-__host__ __device__ inline double jit_comp(const double *Ea, int ox, int oy, int oz, const double *Eb, int px, int py,
-                                           int pz, const double *R) {
-    double ec[jit_nherm(LCD)];
-    jit_ket_e(Eb, px, py, pz, ec, std::make_integer_sequence<int, jit_nherm(LCD)>{});
-    return jit_outer<LCD>(Ea, ox, oy, oz, R, ec, std::make_integer_sequence<int, jit_nherm(LAB)>{});
-}
-template <int LAB, int TMAX>
-__host__ __device__ inline double jit_comp_l(int Lcd, const double *Ea, int ox, int oy, int oz, const double *Eb, int px,
-                                             int py, int pz, const double *R) {
-    if constexpr (TMAX >= 3 && LAB <= 2)
-        if (Lcd == 3) return jit_comp<LAB, 3>(Ea, ox, oy, oz, Eb, px, py, pz, R);
-    switch (Lcd) {
-    case 0: return jit_comp<LAB, 0>(Ea, ox, oy, oz, Eb, px, py, pz, R);
-    case 1: return jit_comp<LAB, 1>(Ea, ox, oy, oz, Eb, px, py, pz, R);
-    default: return jit_comp<LAB, 2>(Ea, ox, oy, oz, Eb, px, py, pz, R);
-    }
-}
-// The same sum for the larger classes (either side of total order 3 or 4):
-// each component's own box of Hermite terms, lane-dependent loop bounds and
-// indices through the LDS copy hm of jit_herm.
-__host__ __device__ inline double jit_comp_box(const double *Ea, int ox, int oy, int oz, int ex, int ey, int ez,
-                                               const double *Eb, int px, int py, int pz, int fx, int fy, int fz,
-                                               const double *R, const short *hm) {
-    double val = 0.0;
-    for (int t = 0; t <= ex; t++)
-        for (int u = 0; u <= ey; u++)
-            for (int w = 0; w <= ez; w++) {
-                const double eab = Ea[ox + t] * Ea[oy + u] * Ea[oz + w];
-                double inner = 0.0;
-                for (int tt = 0; tt <= fx; tt++)
-                    for (int uu = 0; uu <= fy; uu++)
-                        for (int ww = 0; ww <= fz; ww++) {
-                            const double ecd = Eb[px + tt] * Eb[py + uu] * Eb[pz + ww];
-                            const double r = R[hm[((t + tt) * 9 + (u + uu)) * 9 + (w + ww)]];
-                            inner += ((tt + uu + ww) & 1) ? -ecd * r : ecd * r;
-                        }
-                val += eab * inner;
-            }
-    return val;
+
+// 1 / sqrt(x), x > 0.  On the device one third-order step from v_rsq_f64
+// (good to 2^-23): with e = 1 - x y^2, y (1 + e/2 + 3 e^2 / 8) is off by
+// e^3 (2^-66) besides its rounding.
+__host__ __device__ inline double jit_rsqrt(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+#else
+    return 1.0 / sqrt(x);
+#endif
 }
 
-// Hermite expansion coefficients of one primitive pair along one direction,
-// for a fixed (LA, LB), unrolled: E[(i * (LB + 1) + j) * (LA + LB + 1) + t],
-// i <= LA, j <= LB, every t written (zero for t > i + j, so the rows can be
-// summed to the class's full order).  E^{00}_0 = 1: the exponential factor
-// is in the pair prefactor K.  Two-term recurrences
-// E^{i+1,j}_t = E^{ij}_{t-1} / (2p) + X_PA E^{ij}_t + (t+1) E^{ij}_{t+1}, and
-// the same in j with X_PB.
-template <int LA, int LB>
-__host__ __device__ inline void jit_hermite_e_t(double xpa, double xpb, double i2p, double *E) {
-    constexpr int NT = LA + LB + 1;
-    double e[LA + 1][LB + 1][NT];
+// Position of coefficient pair k (0..3) of interval gi in its table: the
+// pairs of a row are permuted by the row number, so that lanes at different
+// rows read different LDS banks (rows are 16 of the 64 banks wide; unpermuted,
+// a pair of every row would sit in the same 16 banks).
+__host__ __device__ inline int jit_bpos(int gi, int k) { return gi * JIT_BROW + ((2 * k) ^ (((gi >> 2) & 3) * 2)); }
+
+// F_0..F_M at T into F: the table's polynomial for F_M and downward
+// recursion F_{m-1} = (2T F_m + e^-T) / (2m - 1) below T = 40; above, F_0 =
+// sqrt(pi/T)/2 (erfc(sqrt 40) is 4e-19) and upward recursion.  There e^-T is
+// 3e-10 of F_8 at T = 40 and 4e-19 of it at 64, and below an ulp of F_0 and
+// F_1 throughout.
+template <int M>
+__host__ __device__ inline void jit_boys(double T, const double *bt, double *F) {
+    if (T < JIT_BTMAX) {
+        const int gi = (int)(T * 16.0);
+        const double d = fma((double)gi, 0.0625, 0.03125) - T;
+        struct D2 { double x, y; };
+        const D2 a = *reinterpret_cast<const D2 *>(bt + jit_bpos(gi, 0)), b = *reinterpret_cast<const D2 *>(bt + jit_bpos(gi, 1));
+        const D2 c = *reinterpret_cast<const D2 *>(bt + jit_bpos(gi, 2)), e = *reinterpret_cast<const D2 *>(bt + jit_bpos(gi, 3));
+        F[M] = fma(fma(fma(fma(fma(fma(e.x, d, c.y), d, c.x), d, b.y), d, b.x), d, a.y), d, a.x);
+        if constexpr (M > 0) {
+            // e^-T = e^-T0 e^d, |d| <= 1/32: the omitted d^8/8! is 2e-17
+            const double ed = fma(fma(fma(fma(fma(fma(fma(d, 1.0 / 5040, 1.0 / 720), d, 1.0 / 120), d, 1.0 / 24), d,
+                                          1.0 / 6), d, 0.5), d, 1.0), d, 1.0);
+            const double eT = e.y * ed, T2 = 2.0 * T;
 #pragma unroll
-    for (int i = 0; i <= LA; i++)
+            for (int m = M; m > 0; m--) F[m - 1] = fma(T2, F[m], eT) * (1.0 / (2 * m - 1));
+        }
+    } else {
+        const double r = jit_rsqrt(T);
+        F[0] = 0.88622692545275801365 * r;   // sqrt(pi) / 2
+        if constexpr (M > 0) {
+            const double i2T = 0.5 * r * r;
+            double eT = 0.0;
+            if constexpr (M > 1)
+                if (T < 64.0) eT = exp(-T);
 #pragma unroll
-        for (int j = 0; j <= LB; j++)
-#pragma unroll
-            for (int t = 0; t < NT; t++) e[i][j][t] = 0.0;
-    e[0][0][0] = 1.0;
-#pragma unroll
-    for (int i = 0; i < LA; i++)
-#pragma unroll
-        for (int t = 0; t <= i + 1; t++)
-            e[i + 1][0][t] = (t > 0 ? i2p * e[i][0][t - 1] : 0.0) + (t <= i ? xpa * e[i][0][t] : 0.0) +
-                             (t + 1 <= i ? (t + 1) * e[i][0][t + 1] : 0.0);
-#pragma unroll
-    for (int i = 0; i <= LA; i++)
-#pragma unroll
-        for (int j = 0; j < LB; j++)
-#pragma unroll
-            for (int t = 0; t <= i + j + 1; t++)
-                e[i][j + 1][t] = (t > 0 ? i2p * e[i][j][t - 1] : 0.0) + (t <= i + j ? xpb * e[i][j][t] : 0.0) +
-                                 (t + 1 <= i + j ? (t + 1) * e[i][j][t + 1] : 0.0);
-#pragma unroll
-    for (int i = 0; i <= LA; i++)
-#pragma unroll
-        for (int j = 0; j <= LB; j++)
-#pragma unroll
-            for (int t = 0; t < NT; t++) E[(i * (LB + 1) + j) * NT + t] = e[i][j][t];
-}
-__host__ __device__ inline void jit_hermite_e_any(int la, int lb, double xpa, double xpb, double i2p, double *E) {
-    switch (la * 3 + lb) {
-    case 0: jit_hermite_e_t<0, 0>(xpa, xpb, i2p, E); break;
-    case 1: jit_hermite_e_t<0, 1>(xpa, xpb, i2p, E); break;
-    case 2: jit_hermite_e_t<0, 2>(xpa, xpb, i2p, E); break;
-    case 3: jit_hermite_e_t<1, 0>(xpa, xpb, i2p, E); break;
-    case 4: jit_hermite_e_t<1, 1>(xpa, xpb, i2p, E); break;
-    case 5: jit_hermite_e_t<1, 2>(xpa, xpb, i2p, E); break;
-    case 6: jit_hermite_e_t<2, 0>(xpa, xpb, i2p, E); break;
-    case 7: jit_hermite_e_t<2, 1>(xpa, xpb, i2p, E); break;
-    default: jit_hermite_e_t<2, 2>(xpa, xpb, i2p, E); break;
+            for (int m = 0; m < M; m++) F[m + 1] = fma((double)(2 * m + 1), F[m], -eT) * i2T;
+        }
     }
 }
 
 // The in-place Hermite recursion for a fixed total order LT, in registers:
 // for n = LT-1 .. 0 the entries of order <= LT-n in decreasing index (so
-// the orders an entry reads still hold R^{(n+1)}), then R^{(n)}_{000};
-// R^{(0)} written out at the end.
+// the orders an entry reads still hold R^{(n+1)}), then R^{(n)}_{000}.
 template <int H>
 struct JitStep {   // R_h = X_dir R_{h1} + c R_{h2}
     static constexpr int t = jit_hcomp(H, 0), u = jit_hcomp(H, 1), w = jit_hcomp(H, 2);
@@ -345,7 +224,7 @@ template <int H>
 __host__ __device__ inline void jit_rdesc(double *r, const double *xyz) {
     if constexpr (H >= 1) {
         using S = JitStep<H>;
-        if constexpr (S::h2 >= 0) r[H] = xyz[S::dir] * r[S::h1] + (double)S::c * r[S::h2];
+        if constexpr (S::h2 >= 0) r[H] = fma(xyz[S::dir], r[S::h1], (double)S::c * r[S::h2]);
         else r[H] = xyz[S::dir] * r[S::h1];
         jit_rdesc<H - 1>(r, xyz);
     }
@@ -358,358 +237,423 @@ __host__ __device__ inline void jit_rlevel(double *r, const double *xyz, const d
         jit_rlevel<LT, N - 1>(r, xyz, Fs);
     }
 }
-template <int LT>
-__host__ __device__ inline void jit_rrec(double X, double Y, double Z, const double *Fs, double *R) {
-    double r[jit_nherm(LT)];
-    const double xyz[3] = {X, Y, Z};
-    r[0] = Fs[LT];
-    jit_rlevel<LT, LT - 1>(r, xyz, Fs);
+
+template <int H1, int... H2>
+__host__ __device__ inline void jit_vrow(const double *R, const double *H, double &V, std::integer_sequence<int, H2...>) {
+    ((V = fma(R[JitSum<H1, H2>::idx], H[H2], V)), ...);
+}
+template <int LB, int... H1>
+__host__ __device__ inline void jit_vall(const double *R, const double *H, double *V, std::integer_sequence<int, H1...>) {
+    (jit_vrow<H1>(R, H, V[H1], std::make_integer_sequence<int, jit_nherm(LB)>{}), ...);
+}
+// V += R H / sqrt(p+q) of one bra centre (exponent p, position P, order LA)
+// and one ket centre (kg: q, Q; Hermite density Hk, order LB).
+template <int LA, int LB>
+__host__ __device__ inline void jit_pair(double p, double Px, double Py, double Pz, double q, double Qx, double Qy,
+                                         double Qz, const double *Hk, const double *bt, double *V) {
+    constexpr int LT = LA + LB;
+    const double xyz[3] = {Px - Qx, Py - Qy, Pz - Qz};
+    const double s = jit_rsqrt(p + q);
+    const double alpha = p * q * (s * s);
+    const double T = alpha * fma(xyz[0], xyz[0], fma(xyz[1], xyz[1], xyz[2] * xyz[2]));
+    double F[LT + 1];
+    jit_boys<LT>(T, bt, F);
+    double f = s;
 #pragma unroll
-    for (int h = 0; h < jit_nherm(LT); h++) R[h] = r[h];
+    for (int n = 0; n <= LT; n++) { F[n] *= f; f *= -2.0 * alpha; }
+    double R[jit_nherm(LT)];
+    R[0] = F[LT];
+    jit_rlevel<LT, LT - 1>(R, xyz, F);
+    jit_vall<LB>(R, Hk, V, std::make_integer_sequence<int, jit_nherm(LA)>{});
 }
 
-// x / d for x d < 2^32, with m = magic[d].
-__host__ __device__ inline int jit_div(int x, unsigned long long m) {
-    return (int)(((unsigned long long)(unsigned)x * m) >> 32);
+// Hermite expansion coefficients of one primitive pair along one direction,
+// for a fixed (LA, LB): e[i][j][t], zero for t > i + j.  E^{00}_0 = 1: the
+// exponential factor is in the pair prefactor K.  Two-term recurrences
+// E^{i+1,j}_t = E^{ij}_{t-1} / (2p) + X_PA E^{ij}_t + (t+1) E^{ij}_{t+1}, and
+// the same in j with X_PB.  (Trip counts are constant, so that every index is
+// one after unrolling.)
+template <int LA, int LB>
+__host__ __device__ inline void jit_hermite_e(double xpa, double xpb, double i2p, double (&e)[LA + 1][LB + 1][LA + LB + 1]) {
+    constexpr int NT = LA + LB + 1;
+#pragma unroll
+    for (int i = 0; i <= LA; i++)
+#pragma unroll
+        for (int j = 0; j <= LB; j++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) e[i][j][t] = 0.0;
+    e[0][0][0] = 1.0;
+#pragma unroll
+    for (int i = 0; i < LA; i++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            if (t <= i + 1)
+                e[i + 1][0][t] = (t > 0 ? i2p * e[i][0][t > 0 ? t - 1 : 0] : 0.0) + (t <= i ? xpa * e[i][0][t] : 0.0) +
+                                 (t + 1 <= i ? (t + 1) * e[i][0][t + 1 < NT ? t + 1 : 0] : 0.0);
+#pragma unroll
+    for (int i = 0; i <= LA; i++)
+#pragma unroll
+        for (int j = 0; j < LB; j++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                if (t <= i + j + 1)
+                    e[i][j + 1][t] = (t > 0 ? i2p * e[i][j][t > 0 ? t - 1 : 0] : 0.0) + (t <= i + j ? xpb * e[i][j][t] : 0.0) +
+                                     (t + 1 <= i + j ? (t + 1) * e[i][j][t + 1 < NT ? t + 1 : 0] : 0.0);
 }
-
-// Input value of index k (k < 0: none).
-__host__ __device__ inline double jit_in(const JitView &v, int k) {
-    return k < 0 ? 0.0 : (k < v.N ? v.X[k] : v.Y0[k - v.N]);
-}
-
-// One row task on NL lanes (64 on the device, 1 in the emulator), lds of
-// LDSN doubles (enough for every ket class against the task's bra class):
-// bra pair a against the partner entries gent[t_e0, t_e1), its partial rows
-// into part[task].
-// Per quartet: the partial sums of each component over the primitive
-// quartets live in nsl slices (NL / ncomp of them when a quartet has fewer
-// components than lanes, so that the lanes left over share the primitive
-// loop), added in slice order at the end of the quartet.
-// E tables of both pairs and the Hermite integrals R of one primitive
-// quartet (bra primitive pair pi, ket primitive pair pj) into Ea (esa
-// doubles), Eb = Ea + esa (esb) and R = Eb + esb (nH(Lt) + Lt + 1).
-__host__ __device__ inline void jit_prim(const JitView &v, int la, int lb, int lc, int ld, int esa_d, int esb_d,
-                                         const double *pi, const double *pj, const double *Ag, const double *Cg,
-                                         double *Ea) {
-    const int Lt = la + lb + lc + ld, nH = jit_nherm(Lt);
-    double *Eb = Ea + 3 * esa_d, *R = Eb + 3 * esb_d;
-    const double p = pi[0], qq = pj[0];
-    for (int d = 0; d < 3; d++) {
-        jit_hermite_e_any(la, lb, pi[1 + d] - Ag[d], pi[1 + d] - Ag[3 + d], pi[5], Ea + d * esa_d);
-        jit_hermite_e_any(lc, ld, pj[1 + d] - Cg[d], pj[1 + d] - Cg[3 + d], pj[5], Eb + d * esb_d);
+template <int LA, int LB>
+struct JitE {
+    double x[LA + 1][LB + 1][LA + LB + 1], y[LA + 1][LB + 1][LA + LB + 1], z[LA + 1][LB + 1][LA + LB + 1];
+    // E tables of primitive pr of the pair at geo, the x table times f
+    __host__ __device__ inline void make(const double *pr, const double *geo, double f) {
+        jit_hermite_e<LA, LB>(pr[1] - geo[0], pr[1] - geo[3], pr[5], x);
+        jit_hermite_e<LA, LB>(pr[2] - geo[1], pr[2] - geo[4], pr[5], y);
+        jit_hermite_e<LA, LB>(pr[3] - geo[2], pr[3] - geo[5], pr[5], z);
+#pragma unroll
+        for (int i = 0; i <= LA; i++)
+#pragma unroll
+            for (int j = 0; j <= LB; j++)
+#pragma unroll
+                for (int t = 0; t <= LA + LB; t++) x[i][j][t] *= f;
     }
-    const double pq = p + qq, inv_pq = 1.0 / pq, alpha = p * qq * inv_pq;
-    const double X = pi[1] - pj[1], Y = pi[2] - pj[2], Z = pi[3] - pj[3];
-    const double T = alpha * (X * X + Y * Y + Z * Z);
-    // 2 pi^{5/2} / (p q sqrt(p + q)) K_i K_j, with 1/p = 2 pi[5]
-    const double pre = 2.0 * M_PI * M_PI * sqrt(M_PI) * (4.0 * pi[5] * pj[5]) * sqrt(inv_pq) * pi[4] * pj[4];
-    double *Fs = R + nH;   // pre (-2 alpha)^n F_n
-    jit_boys(v, Lt, T, Fs, 1);
-    double s = pre;
-    for (int n = 0; n <= Lt; n++) { Fs[n] *= s; s *= -2.0 * alpha; }
-    // R^{(n)} from R^{(n+1)} in place, n = Lt-1 .. 0: orders from the
-    // highest down, so that the orders k-1 and k-2 an order-k entry reads
-    // still hold R^{(n+1)}
-    switch (Lt) {
-    case 0: R[0] = Fs[0]; break;
-    case 1: jit_rrec<1>(X, Y, Z, Fs, R); break;
-    case 2: jit_rrec<2>(X, Y, Z, Fs, R); break;
-    case 3: jit_rrec<3>(X, Y, Z, Fs, R); break;
-    case 4: jit_rrec<4>(X, Y, Z, Fs, R); break;
-    default: break;
-    }
-    const JitTabs &tb = jit_tabs();
-    if (Lt > 4) R[0] = Fs[Lt];
-    for (int n = Lt > 4 ? Lt - 1 : -1; n >= 0; n--) {
-        for (int k = Lt - n; k >= 1; k--) {
-            const int hb = k * (k + 1) * (k + 2) / 6, he = (k + 1) * (k + 2) * (k + 3) / 6;
-            for (int h = hb; h < he; h++) {
-                const int h1 = tb.rstep[h][0], h2 = tb.rstep[h][1], d = tb.rstep[h][3];
-                const double xx = d == 0 ? X : (d == 1 ? Y : Z);
-                R[h] = h2 >= 0 ? xx * R[h1] + (double)tb.rstep[h][2] * R[h2] : xx * R[h1];
-            }
+};
+// Cartesian component AB of class (LA, LB) and Hermite triple H: whether H is
+// in the component's box, and its E product.
+template <int LA, int LB, int AB, int H>
+struct JitBox {
+    static constexpr int ia = AB / jit_ncart(LB), ib = AB % jit_ncart(LB);
+    static constexpr int ax = jit_cexp(LA, ia, 0), ay = jit_cexp(LA, ia, 1), az = jit_cexp(LA, ia, 2);
+    static constexpr int bx = jit_cexp(LB, ib, 0), by = jit_cexp(LB, ib, 1), bz = jit_cexp(LB, ib, 2);
+    static constexpr int t = jit_hcomp(H, 0), u = jit_hcomp(H, 1), w = jit_hcomp(H, 2);
+    static constexpr bool in = t <= ax + bx && u <= ay + by && w <= az + bz;
+    static constexpr bool neg = ((t + u + w) & 1) != 0;
+    static __host__ __device__ inline double e(const JitE<LA, LB> &E) { return E.x[ax][bx][t] * E.y[ay][by][u] * E.z[az][bz][w]; }
+};
+template <int LA, int LB, int AB, int... H>
+__host__ __device__ inline void jit_dens_ab(const JitE<LA, LB> &E, double x, double *Hc, std::integer_sequence<int, H...>) {
+    ([&] {
+        using B = JitBox<LA, LB, AB, H>;
+        if constexpr (B::in) Hc[H] = fma(B::neg ? -x : x, B::e(E), Hc[H]);
+    }(), ...);
+}
+template <int LA, int LB, int... AB>
+__host__ __device__ inline void jit_dens_all(const JitE<LA, LB> &E, const JitView &v, const int *km, double *Hc,
+                                             std::integer_sequence<int, AB...>) {
+    ([&] {
+        const int k = km[AB];   // k < 0: the row is not used
+        const double x = k < 0 ? 0.0 : (k < v.N ? v.X[k] : v.Y0[k - v.N]);
+        jit_dens_ab<LA, LB, AB>(E, x, Hc, std::make_integer_sequence<int, jit_nherm(LA + LB)>{});
+    }(), ...);
+}
+// Hermite density of one contribution: entry e (class LA, LB), primitive pr;
+// 2 pi^{5/2} K / q and the ket's signs are in it.
+template <int LA, int LB>
+__host__ __device__ inline void jit_dens(const JitView &v, int e, int b, const double *pr, double *Hc) {
+    JitE<LA, LB> E;
+    E.make(pr, v.pgeo + 6 * (size_t)b, 4.0 * M_PI * M_PI * sqrt(M_PI) * pr[5] * pr[4]);
+    jit_dens_all<LA, LB>(E, v, v.kmap + v.kl_moff[e], Hc, std::make_integer_sequence<int, jit_ncart(LA) * jit_ncart(LB)>{});
+}
+// Hermite density of centre c of order L: its contributions in order.
+template <int L>
+__host__ __device__ inline void jit_density(const JitView &v, int c) {
+    double Hc[jit_nherm(L)];
+#pragma unroll
+    for (int h = 0; h < jit_nherm(L); h++) Hc[h] = 0.0;
+    for (int k = v.cptr[c]; k < v.cptr[c + 1]; k++) {
+        const int e = v.cent[k], b = v.kl_pair[e];
+        const double *pr = v.prim + 6 * (size_t)v.cprim[k];
+        if constexpr (L == 0) jit_dens<0, 0>(v, e, b, pr, Hc);
+        if constexpr (L == 1) { if (v.pinfo[4 * b] == 0) jit_dens<0, 1>(v, e, b, pr, Hc); else jit_dens<1, 0>(v, e, b, pr, Hc); }
+        if constexpr (L == 2) {
+            const int la = v.pinfo[4 * b];
+            if (la == 0) jit_dens<0, 2>(v, e, b, pr, Hc);
+            else if (la == 1) jit_dens<1, 1>(v, e, b, pr, Hc);
+            else jit_dens<2, 0>(v, e, b, pr, Hc);
         }
-        R[0] = Fs[n];
+        if constexpr (L == 3) { if (v.pinfo[4 * b] == 1) jit_dens<1, 2>(v, e, b, pr, Hc); else jit_dens<2, 1>(v, e, b, pr, Hc); }
+        if constexpr (L == 4) jit_dens<2, 2>(v, e, b, pr, Hc);
     }
+    double *o = v.H + v.hoff[L] + (long long)(c - v.coff[L]) * jit_nherm(L);
+#pragma unroll
+    for (int h = 0; h < jit_nherm(L); h++) o[h] = Hc[h];
 }
 
-// One component (E-row offsets and orders ea, ec) on one primitive quartet.
-template <int TMAX>
-__host__ __device__ inline double jit_cval(int Lab, int Lcd, const double *Ea, const double *Eb, const double *R,
-                                           const short *ea, const short *ec, const short *hm) {
-    const int ox = ea[0], oy = ea[1], oz = ea[2], px = ec[0], py = ec[1], pz = ec[2];
-    if (Lab > TMAX || Lcd > TMAX || Lab + Lcd > 5)
-        return jit_comp_box(Ea, ox, oy, oz, ea[3] & 15, (ea[3] >> 4) & 15, ea[3] >> 8, Eb, px, py, pz, ec[3] & 15,
-                            (ec[3] >> 4) & 15, ec[3] >> 8, R, hm);
-    if (Lab == 0) return jit_comp_l<0, TMAX>(Lcd, Ea, ox, oy, oz, Eb, px, py, pz, R);
-    if (Lab == 1) return jit_comp_l<1, TMAX>(Lcd, Ea, ox, oy, oz, Eb, px, py, pz, R);
-    if (Lab == 2) return jit_comp_l<2, TMAX>(Lcd, Ea, ox, oy, oz, Eb, px, py, pz, R);
-    if constexpr (TMAX >= 3) return jit_comp_l<3, TMAX>(Lcd, Ea, ox, oy, oz, Eb, px, py, pz, R);
-    return 0.0;
-}
-
-// One row task on NL lanes (64 on the device, 1 in the emulator), lds of
-// LDSN doubles (enough for every ket class against the task's bra class):
-// bra pair a against the partner entries gent[t_e0, t_e1), its partial rows
-// into part[task].
-//
-// Entries are taken in passes.  A pass is either one ket (its primitive
-// quartets in batches of up to NL, each component's sum over them split
-// into NL / ncomp slices when a quartet has fewer components than lanes,
-// the slices added in order), or up to JIT_KMAX consecutive kets of one
-// class whose primitive quartets number at most JIT_PASSQ together: their
-// E/R work shares the lanes, each (ket, component) sums its own primitive
-// quartets in order (in the small-LDS launch).  The pass boundaries depend
-// only on the task, so the summation order is fixed.  pk holds 6 * (JIT_KMAX + 1) integers of
-// per-ket data (LDS on the device).
-template <int NL, int LDSN, int TMAX>
-__host__ __device__ void jit_task(const JitView &v, int task, int lane, double *lds, const short *hm, const short *eo,
-                                  long long *pk) {
-    const int a = v.t_pair[task];
-    const int la = v.pinfo[4 * a], lb = v.pinfo[4 * a + 1], npa = v.pinfo[4 * a + 2], pa0 = v.pinfo[4 * a + 3];
-    const double *Ag = v.pgeo + 6 * a;
-    const int na = jit_ncart(la), nb = jit_ncart(lb), nab = na * nb, Lab = la + lb;
-    const int esa_d = (la + 1) * (lb + 1) * (Lab + 1), esa = 3 * esa_d;
-    constexpr int RPL = NL >= JIT_NAB ? 1 : JIT_NAB;   // rows per lane
-    constexpr int S = JIT_KMAX + 1;                   // pk block stride
-    double racc[RPL];
-    for (int k = 0; k < RPL; k++) racc[k] = 0.0;
-    const int te1 = v.t_e1[task];
-    for (int ge = v.t_e0[task]; ge < te1;) {
-        const int e = v.gent[ge];
-        const int b = v.kl_pair[e];
-        const int *km = v.kmap + v.kl_moff[e];
-        const int lc = v.pinfo[4 * b], ld = v.pinfo[4 * b + 1], npb = v.pinfo[4 * b + 2], pb0 = v.pinfo[4 * b + 3];
-        const double *Cg = v.pgeo + 6 * b;
-        const int nc = jit_ncart(lc), nd = jit_ncart(ld), ncd = nc * nd, Lcd = lc + ld, Lt = Lab + Lcd;
-        const int esb_d = (lc + 1) * (ld + 1) * (Lcd + 1), esb = 3 * esb_d;
-        const int rsz = jit_nherm(Lt) + Lt + 1;   // R^{(0)} and the scaled Boys values
-        const int ncomp = nab * ncd;
-        const int perq = esa + esb + rsz;
-        const JitTabs &tb = jit_tabs();
-        const unsigned long long m_comp = tb.magic[ncomp], m_cd = tb.magic[ncd], m_b = tb.magic[npb];
-        const short *eo_a = eo + 4 * tb.pcoff[la * 3 + lb], *eo_c = eo + 4 * tb.pcoff[lc * 3 + ld];
-        // ---- the pass: kets ge .. ge + K - 1 of this class
-        // (the small-LDS launch only: in the other the extra path costs spills)
-        int K = 1, sq = npa * npb;
-        if (LDSN == JIT_LDS_S && sq <= JIT_PASSQ)
-            while (ge + K < te1 && K < JIT_KMAX) {
-                const int bn = v.kl_pair[v.gent[ge + K]];
-                if (v.pinfo[4 * bn] != lc || v.pinfo[4 * bn + 1] != ld) break;
-                const int nq2 = npa * v.pinfo[4 * bn + 2];
-                if (sq + nq2 > JIT_PASSQ || (K + 1) * (ncomp + ncd) + (sq + nq2) * perq > LDSN) break;
-                sq += nq2;
-                K++;
-            }
-        if (K > 1) {
-            jit_sync();   // the previous pass's readers of pk are done
-            if (lane == 0) {
-                int q = 0;
-                for (int k = 0; k < K; k++) {
-                    const int ek = v.gent[ge + k], bk = v.kl_pair[ek], npk = v.pinfo[4 * bk + 2];
-                    pk[k] = bk;
-                    pk[S + k] = npk;
-                    pk[2 * S + k] = v.pinfo[4 * bk + 3];
-                    pk[3 * S + k] = v.kl_moff[ek];
-                    pk[4 * S + k] = q;
-                    pk[5 * S + k] = (long long)tb.magic[npk];
-                    q += npa * npk;
-                }
-                pk[4 * S + K] = q;
-            }
-            double *acc = lds, *vin = lds + K * ncomp, *qb = vin + K * ncd;
-            for (int c = lane; c < K * ncomp; c += NL) acc[c] = 0.0;
-            jit_sync();
-            for (int it = lane; it < K * ncd; it += NL) {   // every ket's input
-                const int k = jit_div(it, m_cd), c = it - k * ncd;
-                vin[it] = jit_in(v, v.kmap[pk[3 * S + k] + c]);
-            }
-            for (int qf = lane; qf < sq; qf += NL) {   // E and R of every primitive quartet of the pass
-                int k = 0;
-                while (k + 1 < K && qf >= (int)pk[4 * S + k + 1]) k++;
-                const int q = qf - (int)pk[4 * S + k];
-                const int i = jit_div(q, (unsigned long long)pk[5 * S + k]), j = q - i * (int)pk[S + k];
-                const int bk = (int)pk[k];
-                jit_prim(v, la, lb, lc, ld, esa_d, esb_d, v.prim + 6 * (size_t)(pa0 + i),
-                         v.prim + 6 * (size_t)(pk[2 * S + k] + j), Ag, v.pgeo + 6 * bk, qb + (size_t)qf * perq);
-            }
-            jit_sync();
-            for (int it = lane; it < K * ncomp; it += NL) {   // (ket, component) over its primitive quartets
-                const int k = jit_div(it, m_comp), cmp = it - k * ncomp;
-                const int ab = jit_div(cmp, m_cd), cd = cmp - ab * ncd;
-                const short *ea = eo_a + 4 * ab, *ec = eo_c + 4 * cd;
-                double sum = 0.0;
-                for (int qf = (int)pk[4 * S + k]; qf < (int)pk[4 * S + k + 1]; qf++) {
-                    const double *Ea = qb + (size_t)qf * perq;
-                    sum += jit_cval<TMAX>(Lab, Lcd, Ea, Ea + esa, Ea + esa + esb, ea, ec, hm);
-                }
-                acc[it] = sum;
-            }
-            jit_sync();
-            for (int k = 0; k < RPL; k++) {   // contract with every ket's input, kets in order
-                const int r = lane + k * NL;
-                if (r < nab)
-                    for (int kk = 0; kk < K; kk++) {
-                        double s = 0.0;
-                        for (int c = 0; c < ncd; c++) s += acc[kk * ncomp + r * ncd + c] * vin[kk * ncd + c];
-                        racc[k] += s;
-                    }
-            }
-            jit_sync();
-            ge += K;
-            continue;
-        }
-        // ---- one ket
-        const int nsl = ncomp >= NL ? 1 : jit_div(NL, m_comp), npart = nsl * ncomp;
-        const int preg = ncomp > 64 ? ncomp : 64;   // partial-sum region (npart <= preg)
-        double *acc = lds, *vin = lds + preg, *qb = vin + ncd;
-        int bq = jit_div(LDSN - preg - ncd, tb.magic[perq]);
-        if (bq > NL) bq = NL;
-        for (int c = lane; c < npart; c += NL) acc[c] = 0.0;
-        // the partner's input: on the device one value per lane, held in a
-        // register and stored after the first batch's E/R work, so the
-        // global load's latency hides behind it
-        double vreg = 0.0;
-        if constexpr (NL >= JIT_NAB) {
-            if (lane < ncd) vreg = jit_in(v, km[lane]);
-        } else {
-            for (int c = lane; c < ncd; c += NL) vin[c] = jit_in(v, km[c]);
-        }
-        const int nq = npa * npb;
-        for (int q0 = 0; q0 < nq; q0 += bq) {
-            const int nqb = nq - q0 < bq ? nq - q0 : bq;
-            jit_sync();
-            for (int q = lane; q < nqb; q += NL) {   // E tables and R of one primitive quartet
-                const int i = jit_div(q0 + q, m_b), j = q0 + q - i * npb;
-                jit_prim(v, la, lb, lc, ld, esa_d, esb_d, v.prim + 6 * (size_t)(pa0 + i), v.prim + 6 * (size_t)(pb0 + j),
-                         Ag, Cg, qb + (size_t)q * perq);
-            }
-            if constexpr (NL >= JIT_NAB)
-                if (q0 == 0 && lane < ncd) vin[lane] = vreg;
-            jit_sync();
-            for (int it = lane; it < npart; it += NL) {   // components over the primitive quartets
-                const int sl = jit_div(it, m_comp), cmp = it - sl * ncomp;
-                const int ab = jit_div(cmp, m_cd), cd = cmp - ab * ncd;
-                const short *ea = eo_a + 4 * ab, *ec = eo_c + 4 * cd;
-                double sum = acc[it];
-                for (int q = sl; q < nqb; q += nsl) {
-                    const double *Ea = qb + (size_t)q * perq;
-                    sum += jit_cval<TMAX>(Lab, Lcd, Ea, Ea + esa, Ea + esa + esb, ea, ec, hm);
-                }
-                acc[it] = sum;
-            }
-        }
-        jit_sync();
-        if (nsl > 1) {   // slices in order; lane cmp alone reads and writes column cmp
-            for (int cmp = lane; cmp < ncomp; cmp += NL) {
-                double t = acc[cmp];
-                for (int sl = 1; sl < nsl; sl++) t += acc[sl * ncomp + cmp];
-                acc[cmp] = t;
-            }
-            jit_sync();
-        }
-        for (int k = 0; k < RPL; k++) {   // contract the quartet with the partner's input
-            const int r = lane + k * NL;
-            if (r < nab) {
-                double s = 0.0;
-                for (int c = 0; c < ncd; c++) s += acc[r * ncd + c] * vin[c];
-                racc[k] += s;
-            }
-        }
-        jit_sync();
-        ge++;
+// One thread per centre, workgroups of one order, the highest (and slowest)
+// first.  The E tables of order 4 take 256 VGPRs, two waves per SIMD; the
+// centres are too few to use more (C30H62: 77,249, 1,207 waves of the
+// 2,048 that fit).
+__global__ void __launch_bounds__(256) jit_density_kernel(JitView v) {
+    int b = blockIdx.x, L = JIT_OMAX;
+    for (; L > 0; L--) {
+        const int nb = (v.coff[L + 1] - v.coff[L] + 255) / 256;
+        if (b < nb) break;
+        b -= nb;
     }
-    for (int k = 0; k < RPL; k++) {
-        const int r = lane + k * NL;
-        if (r < nab) v.part[(size_t)task * JIT_NAB + r] = racc[k];
+    const int c = v.coff[L] + b * 256 + threadIdx.x;
+    if (c >= v.coff[L + 1]) return;
+    switch (L) {
+    case 0: jit_density<0>(v, c); break;
+    case 1: jit_density<1>(v, c); break;
+    case 2: jit_density<2>(v, c); break;
+    case 3: jit_density<3>(v, c); break;
+    default: jit_density<4>(v, c); break;
     }
 }
 
-// Output rows of group g: the partials of its tasks, added in entry order.
-__host__ __device__ inline void jit_reduce(const JitView &v, int g) {
-    const int a = v.r_pair[g];
-    const int nab = jit_ncart(v.pinfo[4 * a]) * jit_ncart(v.pinfo[4 * a + 1]);
-    const int *om = v.omap + v.r_omap[g];
-    for (int r = 0; r < nab; r++) {
-        const int o = om[r];
-        if (o < 0) continue;
-        double s = 0.0;
-        for (int k = v.r_t0[g]; k < v.r_t1[g]; k++) s += v.part[(size_t)v.r_tasks[k] * JIT_NAB + r];
-        if (o < v.N) v.YJ[o] = s;
-        else v.Y1[o - v.N] = s;
+// Rows of entry e (class LA, LB) from the potentials of its primitives'
+// centres: primitives sub, sub + NS, ... on this lane; NS lanes share an
+// entry and add their rows in a fixed order.
+template <int LA, int LB, int AB, int... H>
+__host__ __device__ inline double jit_row_ab(const JitE<LA, LB> &E, const double *Vc, std::integer_sequence<int, H...>) {
+    double s = 0.0;
+    ([&] {
+        using B = JitBox<LA, LB, AB, H>;
+        if constexpr (B::in) s = fma(B::e(E), Vc[H], s);
+    }(), ...);
+    return s;
+}
+template <int LA, int LB, int... AB>
+__host__ __device__ inline void jit_row_all(const JitE<LA, LB> &E, const double *Vc, double *acc, std::integer_sequence<int, AB...>) {
+    ((acc[AB] += jit_row_ab<LA, LB, AB>(E, Vc, std::make_integer_sequence<int, jit_nherm(LA + LB)>{})), ...);
+}
+template <int LA, int LB, int NS>
+__host__ __device__ inline void jit_rows(const JitView &v, int e, int b, int sub) {
+    constexpr int L = LA + LB, NAB = jit_ncart(LA) * jit_ncart(LB), NH = jit_nherm(L);
+    double acc[NAB];
+#pragma unroll
+    for (int k = 0; k < NAB; k++) acc[k] = 0.0;
+    const int np = v.pinfo[4 * b + 2], p0 = v.pinfo[4 * b + 3], ec = v.e_c0[e];
+    for (int k = sub; k < np; k += NS) {
+        const double *pr = v.prim + 6 * (size_t)(p0 + k);
+        const double *Vp = v.V + v.hoff[L] + (long long)(v.ecen[ec + k] - v.coff[L]) * NH;
+        double Vc[NH];
+#pragma unroll
+        for (int h = 0; h < NH; h++) Vc[h] = Vp[h];
+        JitE<LA, LB> E;
+        E.make(pr, v.pgeo + 6 * (size_t)b, 2.0 * pr[5] * pr[4]);
+        jit_row_all<LA, LB>(E, Vc, acc, std::make_integer_sequence<int, NAB>{});
+    }
+    const int *om = v.kmap + v.kl_moff[e];
+#pragma unroll
+    for (int k = 0; k < NAB; k++) {
+        double a = acc[k];
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+        for (int s = 1; s < NS; s <<= 1) a += __shfl_xor(a, s, NS);
+#endif
+        if (k % NS == sub) {
+            const int o = om[k];
+            if (o >= 0) {
+                if (o < v.N) v.YJ[o] = a;
+                else v.Y1[o - v.N] = a;
+            }
+        }
+    }
+}
+template <int NS>
+__host__ __device__ inline void jit_rows_any(const JitView &v, int e, int sub) {
+    const int b = v.kl_pair[e];
+    switch (v.pinfo[4 * b] * 3 + v.pinfo[4 * b + 1]) {
+    case 0: jit_rows<0, 0, NS>(v, e, b, sub); break;
+    case 1: jit_rows<0, 1, NS>(v, e, b, sub); break;
+    case 2: jit_rows<0, 2, NS>(v, e, b, sub); break;
+    case 3: jit_rows<1, 0, NS>(v, e, b, sub); break;
+    case 4: jit_rows<1, 1, NS>(v, e, b, sub); break;
+    case 5: jit_rows<1, 2, NS>(v, e, b, sub); break;
+    case 6: jit_rows<2, 0, NS>(v, e, b, sub); break;
+    case 7: jit_rows<2, 1, NS>(v, e, b, sub); break;
+    default: jit_rows<2, 2, NS>(v, e, b, sub); break;
+    }
+}
+// Eight lanes per entry; entries are sorted by class, so a wave's eight
+// entries take one path.
+static const int JIT_RLANES = 8;
+__global__ void __launch_bounds__(256) jit_rows_kernel(JitView v, int nout) {
+    const int i = (blockIdx.x * 256 + threadIdx.x) / JIT_RLANES;
+    // whole lane groups leave together: the shuffles stay within a group
+    if (i < nout) jit_rows_any<JIT_RLANES>(v, v.oent[i], threadIdx.x % JIT_RLANES);
+}
+
+// The potential kernels, bound by FP64 vector issue: C30H62 has 5.4e8 pairs
+// of centres (1.08e9 primitive quartets), 45 to 250 vector instructions each,
+// 1.2 ms at one instruction per SIMD and four cycles; the three launches take
+// 2.1 ms together, in place of 255 ms when every quartet formed its Cartesian
+// components.  One wave per task, lanes over bra centres (their
+// exponent, position and potential in registers), a loop over the ket
+// centres, which are the same for every lane: their data come through scalar
+// loads and feed the FMAs from scalar registers.  A task whose centres fill
+// less than half a wave gives each centre 64 / bw lanes, which take the ket
+// centres in turn and add their potentials at the end in a fixed order.
+template <int LA, int LB, bool UNI>
+__device__ __forceinline__ void jit_potential(const JitView &v, const JitTask &t, const double *__restrict__ cgeo,
+                                              const double *__restrict__ Hall, const int *__restrict__ segs,
+                                              const double *bt) {
+    constexpr int NA = jit_nherm(LA), NB = jit_nherm(LB);
+    const int lane = threadIdx.x & 63, bw = 1 << t.lbw;
+    const int b = lane & (bw - 1), sl = UNI ? 0 : lane >> t.lbw, ns = UNI ? 1 : 64 >> t.lbw;
+    const double *bg = cgeo + 4 * (long long)(t.c0 + min(b, t.n - 1));   // lanes past the tile repeat its last centre
+    const double p = bg[0], Px = bg[1], Py = bg[2], Pz = bg[3];
+    double V[NA];
+#pragma unroll
+    for (int h = 0; h < NA; h++) V[h] = 0.0;
+    const double *Hb = Hall + v.hoff[LB] - (long long)v.coff[LB] * NB;
+    for (int sg = t.s0; sg < t.s1; sg++) {
+        const int k0 = segs[2 * sg], k1 = segs[2 * sg + 1];
+        for (int j = k0 + sl; j < k1; j += ns) {
+            const double *g = cgeo + 4 * (long long)j;
+            jit_pair<LA, LB>(p, Px, Py, Pz, g[0], g[1], g[2], g[3], Hb + (long long)j * NB, bt, V);
+        }
+    }
+    if constexpr (!UNI) {
+#pragma unroll
+        for (int h = 0; h < NA; h++)
+            for (int s = bw; s < 64; s <<= 1) V[h] += __shfl_xor(V[h], s, 64);
+    }
+    if (lane < t.n) {
+        double *o = v.part + t.poff + lane;
+#pragma unroll
+        for (int h = 0; h < NA; h++) o[(long long)h * bw] = V[h];
     }
 }
 
-__global__ void jit_reduce_kernel(JitView v, int ngroup) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < ngroup) jit_reduce(v, g);
+// Groups of classes by total order LT, one kernel each: 0 LT <= 2, 1 LT 3 and
+// 4, 2 LT >= 5 (up to 165 Hermite integrals per lane).  The tasks of a
+// workgroup share a class, so its Boys table is one order's.
+__host__ __device__ constexpr int jit_group(int LT) { return LT <= 2 ? 0 : (LT <= 4 ? 1 : 2); }
+template <int G, int LA, int LB>
+__device__ __forceinline__ void jit_run(const JitView &v, const JitTask &t, const double *__restrict__ cgeo,
+                                        const double *__restrict__ H, const int *__restrict__ segs, const double *bt) {
+    if constexpr (jit_group(LA + LB) == G) {
+        if (G < 2 && t.lbw == 6) jit_potential<LA, LB, true>(v, t, cgeo, H, segs, bt);
+        else jit_potential<LA, LB, false>(v, t, cgeo, H, segs, bt);
+    }
 }
-
-// The small-LDS launch asks for 3 waves per SIMD (168 VGPRs); the other is
-// held to 2 by its LDS anyway.
-template <int LDSN>
-__global__ void __launch_bounds__(64, LDSN == JIT_LDS_S ? 3 : 2) jit_task_kernel(JitView v, int t0, int t1) {
-    __shared__ double lds[LDSN];
-    __shared__ short hm[729];   // jit_herm by (t, u, w), for lane-dependent lookups
-    __shared__ short eo[400];   // E-row offsets by pair class and Cartesian pair
-    __shared__ long long pk[6 * (JIT_KMAX + 1)];   // per-ket data of a multi-ket pass
-    const int task = t0 + blockIdx.x;
-    if (task >= t1) return;
-    for (int k = threadIdx.x; k < 729; k += 64) hm[k] = (&jit_tabs_dev.herm[0][0][0])[k];
-    for (int k = threadIdx.x; k < 400; k += 64) eo[k] = (&jit_tabs_dev.eoff[0][0])[k];
+template <int G, int... C>
+__device__ __forceinline__ void jit_dispatch(const JitView &v, const JitTask &t, const double *__restrict__ cgeo,
+                                             const double *__restrict__ H, const int *__restrict__ segs,
+                                             const double *bt, std::integer_sequence<int, C...>) {
+    ([&] { if constexpr (jit_group(C / JIT_NORD + C % JIT_NORD) == G) {
+        if (t.cls == C) jit_run<G, C / JIT_NORD, C % JIT_NORD>(v, t, cgeo, H, segs, bt);
+    } }(), ...);
+}
+template <int G> constexpr int jit_waves() { return G == 0 ? 4 : (G == 1 ? 2 : 1); }
+template <int G>
+__global__ void __launch_bounds__(64 * JIT_WPG, jit_waves<G>())
+jit_potential_kernel(JitView v, const JitTask *__restrict__ tasks, const double *__restrict__ cgeo,
+                     const double *__restrict__ H, const int *__restrict__ segs, const double *__restrict__ boys) {
+    __shared__ double2 bt[JIT_BGRID * JIT_BROW / 2];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const JitTask t = tasks[JIT_WPG * blockIdx.x + wave];
+    const int LT = t.cls / JIT_NORD + t.cls % JIT_NORD;
+    const double2 *src = reinterpret_cast<const double2 *>(boys + (long long)LT * JIT_BGRID * JIT_BROW);
+#pragma unroll
+    for (int k = threadIdx.x; k < JIT_BGRID * JIT_BROW / 2; k += 64 * JIT_WPG) bt[k] = src[k];
     __syncthreads();
-    jit_task<64, LDSN, LDSN == JIT_LDS_S ? 2 : 3>(v, task, threadIdx.x, lds, hm, eo, pk);
+    if (t.n == 0) return;   // padding of the workgroup
+    jit_dispatch<G>(v, t, cgeo, H, segs, reinterpret_cast<const double *>(bt),
+                    std::make_integer_sequence<int, JIT_NORD * JIT_NORD>{});
 }
 
-// Up sweep of one level: y0[n] = U_n^T in_n for the listed nodes, where the
-// input rows come from x (leaves) or from the children's y0 (index map uin).
-// Four waves split the rows, lanes the columns; partial sums added in a fixed
-// order.
-__global__ void __launch_bounds__(256) jit_up_kernel(const int *__restrict__ nodes, const long long *__restrict__ uoff,
-                                                     const int *__restrict__ unr, const int *__restrict__ unc,
-                                                     const int *__restrict__ uin0, const int *__restrict__ y0off,
-                                                     const int *__restrict__ uin, const double *__restrict__ U,
-                                                     const double *__restrict__ X, double *__restrict__ Y0, int N) {
-    __shared__ double red[4][64];
-    const int n = nodes[blockIdx.x];
-    const int nr = unr[n], ncl = unc[n], w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const double *Un = U + uoff[n];
-    const int *in = uin + uin0[n];
-    for (int c0 = 0; c0 < ncl; c0 += 64) {
-        const int c = c0 + lane;
+// V of the centres of chunk g: the partials of its tasks, in order.
+__host__ __device__ inline void jit_reduce(const JitView &v, const JitChunk &g, int lane, int NL) {
+    const int nh = jit_nherm(g.la), bw = 1 << g.lbw;
+    double *o = v.V + v.hoff[g.la] + (long long)(g.c0 - v.coff[g.la]) * nh;
+    for (int q = lane; q < nh * bw; q += NL) {
+        const int h = q >> g.lbw, b = q & (bw - 1);
+        if (b >= g.n) continue;
         double s = 0.0;
-        if (c < ncl)
-            for (int r = w; r < nr; r += 4) {
-                const int k = in[r];
-                const double xv = k < N ? X[k] : Y0[k - N];
-                s += Un[(size_t)r * ncl + c] * xv;
-            }
-        red[w][lane] = s;
-        __syncthreads();
-        if (w == 0 && c < ncl) Y0[y0off[n] + c] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
-        __syncthreads();
+        #pragma unroll 8
+        for (int k = g.t0; k < g.t1; k++) s += v.part[v.cpoff[k] + q];
+        o[(long long)b * nh + h] = s;
     }
 }
+__global__ void __launch_bounds__(256) jit_reduce_kernel(JitView v) { jit_reduce(v, v.chunks[blockIdx.x], threadIdx.x, 256); }
 
-// Down sweep of one level: t = U_n y1[n]; row r goes to its leaf row of yd
-// (index < N) or is added to the child's y1 (index - N).
-__global__ void __launch_bounds__(256) jit_down_kernel(const int *__restrict__ nodes, const long long *__restrict__ uoff,
+// The sweeps, one launch per tree level.  They are bound by the read of U
+// (once each); a level near the root has few nodes, so a node is spread over
+// workgroups by columns (up) and rows (down).
+//
+// Up sweep: y0[n] = U_n^T in_n, the input rows from x (leaves) or from the
+// children's y0 (index map uin).  A workgroup takes 64 columns of a node
+// (lanes; a wave reads 512 bytes of a row), its 16 waves split the rows with
+// eight loads in flight, inputs staged in LDS; partial sums added in a fixed
+// order.  C30H62 (4 levels, 128 MB of U): 4 x 13.5 us; with one workgroup
+// of four waves per node 4 x 190 us.
+static const int JIT_URB = 1024;   // input rows staged at a time
+__global__ void __launch_bounds__(1024) jit_up_kernel(const int *__restrict__ items, const long long *__restrict__ uoff,
+                                                      const int *__restrict__ unr, const int *__restrict__ unc,
+                                                      const int *__restrict__ uin0, const int *__restrict__ y0off,
+                                                      const int *__restrict__ uin, const double *__restrict__ U,
+                                                      const double *__restrict__ X, double *__restrict__ Y0, int N) {
+    __shared__ double xin[JIT_URB];
+    __shared__ double red[16][64];
+    const int n = items[2 * blockIdx.x], c0 = items[2 * blockIdx.x + 1];
+    const int nr = unr[n], ncl = unc[n], w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const double *Un = U + uoff[n] + min(c0 + lane, ncl - 1);   // lanes past the last column repeat it
+    const int *in = uin + uin0[n];
+    double s = 0.0;
+    for (int rb = 0; rb < nr; rb += JIT_URB) {
+        const int m = min(JIT_URB, nr - rb);
+        __syncthreads();
+        for (int r = threadIdx.x; r < m; r += 1024) {
+            const int k = in[rb + r];
+            xin[r] = k < N ? X[k] : Y0[k - N];
+        }
+        __syncthreads();
+        int r = w;
+        for (; r + 7 * 16 < m; r += 8 * 16) {
+            double u[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) u[k] = Un[(size_t)(rb + r + 16 * k) * ncl];
+#pragma unroll
+            for (int k = 0; k < 8; k++) s = fma(u[k], xin[r + 16 * k], s);
+        }
+        for (; r < m; r += 16) s = fma(Un[(size_t)(rb + r) * ncl], xin[r], s);
+    }
+    red[w][lane] = s;
+    __syncthreads();
+    for (int h = 8; h > 0; h >>= 1) {
+        if (w < h) red[w][lane] += red[w + h][lane];
+        __syncthreads();
+    }
+    if (w == 0 && c0 + lane < ncl) Y0[y0off[n] + c0 + lane] = red[0][lane];
+}
+
+// Down sweep: t = U_n y1[n]; row r goes to its leaf row of yd (index < N) or
+// is added to the child's y1 (index - N; a child has one parent).  A
+// workgroup takes 64 rows of a node, a wave four rows at a time with its
+// lanes over the columns.  C30H62: 4 x 12.7 us; with a thread per row 4 x 133 us.
+static const int JIT_DROWS = 64;
+__global__ void __launch_bounds__(256) jit_down_kernel(const int *__restrict__ items, const long long *__restrict__ uoff,
                                                        const int *__restrict__ unr, const int *__restrict__ unc,
                                                        const int *__restrict__ uin0, const int *__restrict__ y0off,
                                                        const int *__restrict__ uin, const double *__restrict__ U,
                                                        double *__restrict__ YD, double *__restrict__ Y1, int N) {
-    const int n = nodes[blockIdx.x];
-    const int nr = unr[n], ncl = unc[n];
+    const int n = items[2 * blockIdx.x], r0 = items[2 * blockIdx.x + 1];
+    const int nr = unr[n], ncl = unc[n], w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const double *Un = U + uoff[n];
     const double *y1 = Y1 + y0off[n];
     const int *out = uin + uin0[n];
-    for (int r = threadIdx.x; r < nr; r += 256) {
-        double s = 0.0;
-        for (int c = 0; c < ncl; c++) s += Un[(size_t)r * ncl + c] * y1[c];
-        const int k = out[r];
-        if (k < N) YD[k] = s;
-        else Y1[k - N] += s;
+    const int re = min(r0 + JIT_DROWS, nr);
+    for (int r = r0 + 4 * w; r < re; r += 16) {
+        const double *row[4];
+        double s[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) { row[k] = Un + (size_t)min(r + k, re - 1) * ncl; s[k] = 0.0; }
+        for (int c = lane; c < ncl; c += 64) {
+            const double y = y1[c];
+#pragma unroll
+            for (int k = 0; k < 4; k++) s[k] = fma(row[k][c], y, s[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) s[k] += __shfl_xor(s[k], d, 64);
+        if (lane < 4 && r + lane < re) {
+            const double v = lane == 0 ? s[0] : (lane == 1 ? s[1] : (lane == 2 ? s[2] : s[3]));
+            const int k = out[r + lane];
+            if (k < N) YD[k] = v;
+            else Y1[k - N] += v;
+        }
     }
 }
 
@@ -731,8 +675,20 @@ struct JitPlan {
     std::vector<int> pinfo;
     std::vector<double> pgeo, prim;
     std::vector<int> kl_start, kl_count, kl_pair, kl_moff, kmap;
-    std::vector<int> t_pair, t_e0, t_e1, gent, omap;
-    std::vector<int> r_pair, r_omap, r_t0, r_t1, r_tasks;
+    // Hermite centres, order by order, and their contributions
+    std::vector<int> e_c0, ecen, cptr, cent, cprim;
+    std::vector<double> cgeo;
+    int coff[JIT_NORD + 1] = {};
+    long long hoff[JIT_NORD] = {}, nherm = 0;
+    // tasks: group g in [gtask[g], gtask[g + 1]), whole workgroups
+    std::vector<JitTask> tasks;
+    std::vector<JitChunk> chunks;
+    std::vector<int> segs, ctask, oent;
+    std::vector<long long> cpoff;
+    int gtask[4] = {};
+    long long npart = 0;
+    int ntask = 0;   // without the padding
+    std::vector<double> boys;
     // sweeps
     std::vector<long long> uoff;
     std::vector<int> unr, unc, uin0, y0off, uin;
@@ -740,12 +696,43 @@ struct JitPlan {
     std::vector<std::vector<int>> level_nodes;   // nodes with a non-empty U, per level
     // work per matvec
     double quartets = 0, prim_quartets = 0, eri_values = 0;
-    double cost_b = 0, cost_d = 0;   // planned task cost of coupling and near-field entries
-    int n_big = 0;   // tasks [0, n_big) have a bra or ket pair with la + lb >= 3
-    const double *boys = nullptr;
-    int bgrid = 0, bcol = 0;
-    double bstep = 0, btmax = 0;
+    double cost_b = 0, cost_d = 0;   // planned task cost of coupling and near-field blocks
 };
+
+// The Boys tables of the potential kernels (JIT_BROW): per order M and
+// interval the Taylor coefficients F_{M+k}(T0) / k!, k = 0..8, with the last
+// two replaced by their best lower-degree polynomials on |d| <= 1/32 (from
+// the Chebyshev polynomials T_8 and T_7); what is left out is below
+// (1/32)^7 / (64 7!) F_{M+7}, 1e-16 of F_M for M <= 8.
+static void jit_boys_tables(std::vector<double> &out) {
+    const int top = 2 * JIT_OMAX + 8;
+    out.assign((size_t)JIT_NLT * JIT_BGRID * JIT_BROW, 0.0);
+    for (int gi = 0; gi < JIT_BGRID; gi++) {
+        const long double T = (gi + 0.5L) / 16.0L, eT = expl(-T);
+        long double F[2 * JIT_OMAX + 9];
+        long double term = 1.0L / (2 * top + 1), sum = term;
+        for (int k = 1; k < 2000 && term >= sum * 1e-21L; k++) {
+            term *= 2.0L * T / (long double)(2 * top + 2 * k + 1);
+            sum += term;
+        }
+        F[top] = eT * sum;
+        for (int m = top; m > 0; m--) F[m - 1] = (2.0L * T * F[m] + eT) / (long double)(2 * m - 1);
+        for (int M = 0; M < JIT_NLT; M++) {
+            long double c[9], fact = 1.0L;
+            for (int k = 0; k <= 8; k++) { c[k] = F[M + k] / fact; fact *= (long double)(k + 1); }
+            const long double r = 1.0L / 32.0L, r2 = r * r;
+            c[6] += c[8] * r2 * 2.0L;
+            c[4] -= c[8] * r2 * r2 * 160.0L / 128.0L;
+            c[2] += c[8] * r2 * r2 * r2 * 32.0L / 128.0L;
+            c[0] -= c[8] * r2 * r2 * r2 * r2 / 128.0L;
+            c[5] += c[7] * r2 * 112.0L / 64.0L;
+            c[3] -= c[7] * r2 * r2 * 56.0L / 64.0L;
+            c[1] += c[7] * r2 * r2 * r2 * 7.0L / 64.0L;
+            double *tab = out.data() + (size_t)M * JIT_BGRID * JIT_BROW;
+            for (int k = 0; k < 8; k++) tab[jit_bpos(gi, k >> 1) + (k & 1)] = (double)(k < 7 ? c[k] : eT);
+        }
+    }
+}
 
 static bool jit_plan(H2ERI_p h, JitPlan &J) {
     HostState *hs = host_state(h);
@@ -770,7 +757,7 @@ static bool jit_plan(H2ERI_p h, JitPlan &J) {
             set_error(ERR_UNSUPPORTED, "on-the-fly B/D: shell pair %d has angular momentum above d", i);
             return false;
         }
-        if (pv.np > 1296) {   // the multiply-high divisions by the primitive-pair count
+        if (pv.np > 1296) {   // 36 x 36 primitives: the interface's limit
             set_error(ERR_UNSUPPORTED, "on-the-fly B/D: shell pair %d has %d primitive pairs (at most 1296)", i, pv.np);
             return false;
         }
@@ -897,230 +884,305 @@ static bool jit_plan(H2ERI_p h, JitPlan &J) {
         nearf[n1].push_back(n0);
     }
     auto lv = [&](int n) { return h->node_level[n]; };
-    // output groups: one bra pair on one side against the side's partner
-    // entries gent[e0, e1); split into tasks of bounded cost below
-    struct GroupRec { int pair, omap, e0, e1; };
-    std::vector<GroupRec> groups;
-    // cost of one quartet in rough lane-steps: per primitive quartet, the
-    // Hermite terms of all its components and the R table, over the 64
-    // lanes, plus a fixed cost (loads, barriers)
-    double cls[3][3][3][3];
-    for (int la = 0; la <= JIT_LMAX; la++)
-        for (int lb = 0; lb <= JIT_LMAX; lb++)
-            for (int lc = 0; lc <= JIT_LMAX; lc++)
-                for (int ld = 0; ld <= JIT_LMAX; ld++) {
-                    double terms = 0;
-                    int e[4][3];
-                    for (int ia = 0; ia < jit_ncart(la); ia++)
-                        for (int ib = 0; ib < jit_ncart(lb); ib++)
-                            for (int ic = 0; ic < jit_ncart(lc); ic++)
-                                for (int id = 0; id < jit_ncart(ld); id++) {
-                                    jit_cart(la, ia, e[0][0], e[0][1], e[0][2]);
-                                    jit_cart(lb, ib, e[1][0], e[1][1], e[1][2]);
-                                    jit_cart(lc, ic, e[2][0], e[2][1], e[2][2]);
-                                    jit_cart(ld, id, e[3][0], e[3][1], e[3][2]);
-                                    double t = 1;
-                                    for (int d = 0; d < 3; d++) t *= (e[0][d] + e[1][d] + 1) * (e[2][d] + e[3][d] + 1);
-                                    terms += t;
-                                }
-                    const int Lt = la + lb + lc + ld;
-                    cls[la][lb][lc][ld] = (3.0 * terms + 40.0 + (Lt + 1) * jit_nherm(Lt)) / 64.0;
-                }
-    auto qcost = [&](int a, int b) {
-        return (double)J.pinfo[4 * a + 2] * J.pinfo[4 * b + 2] *
-                   cls[J.pinfo[4 * a]][J.pinfo[4 * a + 1]][J.pinfo[4 * b]][J.pinfo[4 * b + 1]] + 40.0;
-    };
-    int side_e0 = 0, side_e1 = 0;
-    std::vector<char> gent_d;   // per gent entry: from a near-field (D) list
-    // ket pairs of total order 3 or 4 last in each side's entries: tasks are
-    // cut where they start and run in the large-LDS launch
-    auto high_ket = [&](int e) { return J.pinfo[4 * J.kl_pair[e]] + J.pinfo[4 * J.kl_pair[e] + 1] >= 3; };
-    // and within each part grouped by pair class (la, lb), so that runs of
-    // one class form multi-ket passes
-    auto open_side = [&](const std::vector<int> &lists, int n_near) {   // the first n_near lists are near field
-        side_e0 = (int)J.gent.size();
-        for (int pass = 0; pass < 2; pass++)
-            for (int cls = 0; cls < 9; cls++)
-                for (size_t li = 0; li < lists.size(); li++) {
-                    const int L = lists[li];
-                    for (int e = J.kl_start[L]; e < J.kl_start[L] + J.kl_count[L]; e++) {
-                        const int bb = J.kl_pair[e];
-                        if (high_ket(e) == (pass == 1) && J.pinfo[4 * bb] * 3 + J.pinfo[4 * bb + 1] == cls) {
-                            J.gent.push_back(e);
-                            gent_d.push_back((int)li < n_near ? 1 : 0);
-                        }
-                    }
-                }
-        side_e1 = (int)J.gent.size();
-    };
-    auto add_tasks = [&](const std::vector<int> &, int a, const std::vector<int> &om) {
-        GroupRec g;
-        g.pair = a;
-        g.omap = (int)J.omap.size();
-        J.omap.insert(J.omap.end(), om.begin(), om.end());
-        g.e0 = side_e0;
-        g.e1 = side_e1;
-        groups.push_back(g);
-        for (int ge = g.e0; ge < g.e1; ge++) {
-            const int b = J.kl_pair[J.gent[ge]];
-            J.quartets += 1;
-            J.prim_quartets += (double)J.pinfo[4 * a + 2] * J.pinfo[4 * b + 2];
-            J.eri_values += (double)h->sp_nbfp[a] * h->sp_nbfp[b];
-        }
-    };
+    // ---- target sides and the sides they take
+    struct Target { int list, n_near; std::vector<int> src; };   // the first n_near sources are near field
+    std::vector<Target> targets;
+    std::vector<char> used(2 * (size_t)n_node, 0);
     for (int n = 0; n < n_node; n++) {
         if (is_leaf(n)) {   // full rows: near field and case (2)/(3) coupling with n uncompressed
-            std::vector<int> lists;
+            Target t;
+            t.list = 2 * n;
             for (int m : nearf[n]) {
                 if (!is_leaf(m)) { set_error(ERR_ARG, "on-the-fly B/D: near-field partner %d is not a leaf", m); return false; }
-                lists.push_back(2 * m);
+                t.src.push_back(2 * m);
             }
-            const int n_near = (int)lists.size();
+            t.n_near = (int)t.src.size();
             for (int m : adm[n])
-                if (lv(n) < lv(m)) lists.push_back(2 * m + 1);
-            open_side(lists, n_near);
-            if (!lists.empty())
-                for (int a = h->pt_cluster[2 * n]; a <= h->pt_cluster[2 * n + 1]; a++) {
-                    std::vector<int> om(h->sp_nbfp[a]);
-                    for (int r = 0; r < h->sp_nbfp[a]; r++) om[r] = h->sp_bfp_sidx[a] + r;
-                    add_tasks(lists, a, om);
-                }
+                if (lv(n) < lv(m)) t.src.push_back(2 * m + 1);
+            if (!t.src.empty()) targets.push_back(t);
         }
-        std::vector<int> lists;   // skeleton rows: partners at the same or a coarser level
+        Target t;   // skeleton rows: partners at the same or a coarser level
+        t.list = 2 * n + 1;
+        t.n_near = 0;
         for (int m : adm[n]) {
             if (lv(n) < lv(m)) continue;
             if (lv(m) < lv(n) && !is_leaf(m)) {
                 set_error(ERR_ARG, "on-the-fly B/D: coarser admissible partner %d of %d is not a leaf", m, n);
                 return false;
             }
-            lists.push_back(lv(m) >= lv(n) ? 2 * m + 1 : 2 * m);
+            t.src.push_back(lv(m) >= lv(n) ? 2 * m + 1 : 2 * m);
         }
-        if (lists.empty()) continue;
-        open_side(lists, 0);
-        const H2E_int_vec_p jp = h->J_pair[n];
-        if (!jp || rank(n) == 0) { set_error(ERR_ARG, "on-the-fly B/D: node %d has coupling blocks and no skeleton", n); return false; }
-        int rr = 0;
-        for (int k = 0; k < jp->length; k++) {
-            const int a = jp->data[k];
-            std::vector<int> om(h->sp_nbfp[a], -1);
-            bool any = false;
-            for (int r = 0; r < h->sp_nbfp[a]; r++) {
-                const int j = skel_pos[n][rr + r];
-                if (j >= 0) { om[r] = N + J.y0off[n] + j; any = true; }
-            }
-            if (any) add_tasks(lists, a, om);
-            rr += h->sp_nbfp[a];
+        if (t.src.empty()) continue;
+        if (!h->J_pair[n] || rank(n) == 0) {
+            set_error(ERR_ARG, "on-the-fly B/D: node %d has coupling blocks and no skeleton", n);
+            return false;
         }
+        targets.push_back(t);
     }
-    // tasks: each group's entries cut into runs of at most `cap` cost, so that
-    // no task holds the whole pass (a bra pair of contracted s shells against
-    // a full near field is the longest); cap = total / 32768
-    double total = 0;
-    for (const GroupRec &g : groups)
-        for (int ge = g.e0; ge < g.e1; ge++) {
-            const double c = qcost(g.pair, J.kl_pair[J.gent[ge]]);
-            total += c;
-            (gent_d[ge] ? J.cost_d : J.cost_b) += c;
-        }
-    const double cap = std::max(total / 32768.0, 256.0);
-    struct TaskRec { int pair, e0, e1, group; double cost; bool high; };
-    std::vector<TaskRec> tasks;
-    for (int gi = 0; gi < (int)groups.size(); gi++) {
-        const GroupRec &g = groups[gi];
-        int e0 = g.e0;
-        double c = 0;
-        for (int ge = g.e0; ge < g.e1; ge++) {
-            c += qcost(g.pair, J.kl_pair[J.gent[ge]]);
-            const bool cut = ge + 1 == g.e1 || high_ket(J.gent[ge + 1]) != high_ket(J.gent[ge]);
-            if (c >= cap || cut) {
-                tasks.push_back(TaskRec{g.pair, e0, ge + 1, gi, c, high_ket(J.gent[ge])});
-                e0 = ge + 1;
-                c = 0;
-            }
-        }
-        if (g.e0 == g.e1) tasks.push_back(TaskRec{g.pair, g.e0, g.e1, gi, 0.0, false});   // writes zero rows
+    for (const Target &t : targets) {
+        used[t.list] = 1;
+        for (int L : t.src) used[L] = 1;
     }
-    // tasks with a bra or ket pair of total order >= 3 first (the launch with
-    // the larger LDS), each launch longest tasks first
-    auto big = [&](int t) {
-        return tasks[t].high || J.pinfo[4 * tasks[t].pair] + J.pinfo[4 * tasks[t].pair + 1] >= 3;
+    // ---- Hermite centres: primitives of one side with equal order, exponent
+    // sum (bitwise) and centre (to rounding: (a A + b A) / p of one atom's
+    // primitives depends on their order) are one centre
+    const size_t ne = J.kl_pair.size();
+    J.e_c0.assign(ne + 1, 0);
+    for (size_t e = 0; e < ne; e++) J.e_c0[e + 1] = J.e_c0[e] + J.pinfo[4 * J.kl_pair[e] + 2];
+    J.ecen.assign((size_t)J.e_c0[ne], -1);
+    struct Cen { double g[4]; };
+    std::vector<Cen> cen[JIT_NORD];
+    std::vector<int> lc0[JIT_NORD];   // per list: its first centre of the order (lists in order, then the end)
+    struct Key {
+        long long a, x, y, z;
+        bool operator==(const Key &o) const { return a == o.a && x == o.x && y == o.y && z == o.z; }
     };
-    std::vector<int> order(tasks.size());
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        if (big(x) != big(y)) return big(x);
-        return tasks[x].cost > tasks[y].cost;
+    struct KeyHash {
+        size_t operator()(const Key &k) const {
+            unsigned long long s = (unsigned long long)k.a;
+            for (long long w : {k.x, k.y, k.z}) s = (s ^ (unsigned long long)w) * 0x9e3779b97f4a7c15ULL, s ^= s >> 29;
+            return (size_t)s;
+        }
+    };
+    for (int l = 0; l < JIT_NORD; l++) lc0[l].assign(2 * (size_t)n_node + 1, 0);
+    for (int L = 0; L < 2 * n_node; L++) {
+        for (int l = 0; l < JIT_NORD; l++) lc0[l][L] = (int)cen[l].size();
+        if (!used[L]) continue;
+        std::unordered_map<Key, int, KeyHash> at[JIT_NORD];
+        for (int e = J.kl_start[L]; e < J.kl_start[L] + J.kl_count[L]; e++) {
+            const int b = J.kl_pair[e], l = J.pinfo[4 * b] + J.pinfo[4 * b + 1];
+            for (int k = 0; k < J.pinfo[4 * b + 2]; k++) {
+                const double *pr = J.prim.data() + 6 * (size_t)(J.pinfo[4 * b + 3] + k);
+                Key key;
+                memcpy(&key.a, &pr[0], sizeof(double));
+                const double grid = 17592186044416.0;   // 2^44 per bohr
+                key.x = llround(pr[1] * grid);
+                key.y = llround(pr[2] * grid);
+                key.z = llround(pr[3] * grid);
+                auto it = at[l].find(key);
+                bool same = it != at[l].end();
+                if (same)
+                    for (int d = 0; d < 3; d++) {
+                        const double P = cen[l][it->second].g[1 + d];
+                        same = same && std::fabs(P - pr[1 + d]) <= 8 * 2.22e-16 * std::fabs(P);
+                    }
+                int id = same ? it->second : (int)cen[l].size();
+                if (!same) {
+                    if (it == at[l].end()) at[l].emplace(key, id);
+                    cen[l].push_back(Cen{{pr[0], pr[1], pr[2], pr[3]}});
+                }
+                J.ecen[J.e_c0[e] + k] = id;   // within its order, for now
+            }
+        }
+    }
+    long long nc = 0;
+    for (int l = 0; l < JIT_NORD; l++) {
+        lc0[l][2 * (size_t)n_node] = (int)cen[l].size();
+        J.coff[l] = (int)nc;
+        J.hoff[l] = J.nherm;
+        nc += (long long)cen[l].size();
+        J.nherm += (long long)cen[l].size() * jit_nherm(l);
+        if (nc >= INT32_MAX) { set_error(ERR_UNSUPPORTED, "on-the-fly B/D: too many primitives"); return false; }
+        for (const Cen &c : cen[l]) J.cgeo.insert(J.cgeo.end(), c.g, c.g + 4);
+    }
+    J.coff[JIT_NORD] = (int)nc;
+    // contributions of every centre, in entry order
+    J.cptr.assign((size_t)nc + 1, 0);
+    for (size_t e = 0; e < ne; e++) {
+        const int b = J.kl_pair[e], l = J.pinfo[4 * b] + J.pinfo[4 * b + 1];
+        for (int i = J.e_c0[e]; i < J.e_c0[e + 1]; i++)
+            if (J.ecen[i] >= 0) { J.ecen[i] += J.coff[l]; J.cptr[J.ecen[i] + 1]++; }
+    }
+    for (long long c = 0; c < nc; c++) J.cptr[c + 1] += J.cptr[c];
+    J.cent.resize((size_t)J.cptr[nc]);
+    J.cprim.resize((size_t)J.cptr[nc]);
+    {
+        std::vector<int> pos(J.cptr.begin(), J.cptr.end() - 1);
+        for (size_t e = 0; e < ne; e++)
+            for (int i = J.e_c0[e]; i < J.e_c0[e + 1]; i++)
+                if (J.ecen[i] >= 0) {
+                    const int q = pos[J.ecen[i]]++;
+                    J.cent[q] = (int)e;
+                    J.cprim[q] = J.pinfo[4 * J.kl_pair[e] + 3] + (i - J.e_c0[e]);
+                }
+    }
+    auto count = [&](int L, int l) { return lc0[l][L + 1] - lc0[l][L]; };
+    // ---- work
+    double cost[JIT_NORD][JIT_NORD];   // vector instructions of one pair of centres, roughly
+    for (int la = 0; la < JIT_NORD; la++)
+        for (int lb = 0; lb < JIT_NORD; lb++) {
+            const int LT = la + lb;
+            double rec = 0;
+            for (int n = 1; n <= LT; n++) rec += jit_nherm(n) - 1;
+            cost[la][lb] = (45.0 + (LT > 0 ? 12.0 + 3.0 * LT : 0.0) + 1.4 * rec + (double)jit_nherm(la) * jit_nherm(lb)) *
+                           (jit_group(LT) == 2 ? 1.3 : 1.0);
+        }
+    double total = 0;
+    std::vector<double> le(2 * (size_t)n_node), lp(2 * (size_t)n_node, 0.0), lr(2 * (size_t)n_node, 0.0);
+    for (int L = 0; L < 2 * n_node; L++) {
+        le[L] = J.kl_count[L];
+        for (int e = J.kl_start[L]; e < J.kl_start[L] + J.kl_count[L]; e++) {
+            lp[L] += J.pinfo[4 * J.kl_pair[e] + 2];
+            lr[L] += h->sp_nbfp[J.kl_pair[e]];
+        }
+    }
+    for (const Target &t : targets)
+        for (size_t i = 0; i < t.src.size(); i++) {
+            const int S = t.src[i];
+            J.quartets += le[t.list] * le[S];
+            J.prim_quartets += lp[t.list] * lp[S];
+            J.eri_values += lr[t.list] * lr[S];
+            double c = 0;
+            for (int la = 0; la < JIT_NORD; la++)
+                for (int lb = 0; lb < JIT_NORD; lb++) c += cost[la][lb] * count(t.list, la) / 64.0 * count(S, lb);
+            total += c;
+            ((int)i < t.n_near ? J.cost_d : J.cost_b) += c;
+        }
+    // ---- tasks: the centres of a target in chunks of 64, each against the
+    // sources' centres of one order, cut into runs of bounded cost: a wave's
+    // share of the pass when 16 waves of every CU take four tasks each, and at
+    // least 32 centres per lane (below that the table load and the first
+    // loads show)
+    const double cap = total / (256.0 * 16 * 4);
+    struct TaskRec { JitTask t; double cost; };
+    std::vector<TaskRec> recs;
+    for (const Target &t : targets)
+        for (int la = 0; la < JIT_NORD; la++) {
+            const int c0 = J.coff[la] + lc0[la][t.list], c1 = c0 + count(t.list, la);
+            std::map<std::pair<int, int>, std::vector<std::pair<int, int>>> cuts;   // (lb, lbw): its runs of segments
+            for (int c = c0; c < c1; c += 64) {
+                const int n = std::min(64, c1 - c);
+                int lbw = 2;
+                while ((1 << lbw) < n) lbw++;
+                JitChunk ch{la, c, n, lbw, (int)J.ctask.size(), 0};
+                const int ns = 64 >> lbw;
+                for (int lb = 0; lb < JIT_NORD; lb++) {
+                    auto key = std::make_pair(lb, lbw);
+                    auto it = cuts.find(key);
+                    if (it == cuts.end()) {
+                        std::vector<std::pair<int, int>> sg;   // contiguous sources joined
+                        long long tot = 0;
+                        for (int S : t.src) {
+                            const int k0 = J.coff[lb] + lc0[lb][S], k1 = k0 + count(S, lb);
+                            if (k0 == k1) continue;
+                            tot += k1 - k0;
+                            if (!sg.empty() && sg.back().second == k0) sg.back().second = k1;
+                            else sg.push_back({k0, k1});
+                        }
+                        std::vector<std::pair<int, int>> runs;
+                        const long long per_min = 32LL * ns;
+                        long long per = std::max((long long)(cap / cost[la][lb]) * ns, per_min);
+                        const long long nrun = std::max(1LL, (tot + per - 1) / per);
+                        per = (tot + nrun - 1) / nrun;
+                        per = (per + ns - 1) / ns * ns;
+                        long long left = per;
+                        int s0 = (int)J.segs.size() / 2;
+                        for (auto s : sg)
+                            while (s.first < s.second) {
+                                const int take = (int)std::min<long long>(left, s.second - s.first);
+                                J.segs.push_back(s.first);
+                                J.segs.push_back(s.first + take);
+                                s.first += take;
+                                left -= take;
+                                if (left == 0) {
+                                    runs.push_back({s0, (int)J.segs.size() / 2});
+                                    s0 = (int)J.segs.size() / 2;
+                                    left = per;
+                                }
+                            }
+                        if (s0 < (int)J.segs.size() / 2) runs.push_back({s0, (int)J.segs.size() / 2});
+                        it = cuts.emplace(key, runs).first;
+                    }
+                    for (const auto &r : it->second) {
+                        double iters = 0;
+                        for (int s = r.first; s < r.second; s++) iters += (J.segs[2 * s + 1] - J.segs[2 * s] + ns - 1) / ns;
+                        J.ctask.push_back((int)recs.size());
+                        recs.push_back(TaskRec{JitTask{la * JIT_NORD + lb, c, n, lbw, r.first, r.second, J.npart}, iters * cost[la][lb]});
+                        J.npart += (long long)jit_nherm(la) << lbw;
+                    }
+                }
+                ch.t1 = (int)J.ctask.size();
+                J.chunks.push_back(ch);
+            }
+        }
+    J.ntask = (int)recs.size();
+    // workgroups of four tasks of one class, longest first within each launch
+    std::vector<int> by(recs.size());
+    std::iota(by.begin(), by.end(), 0);
+    std::stable_sort(by.begin(), by.end(), [&](int x, int y) {
+        if (recs[x].t.cls != recs[y].t.cls) return recs[x].t.cls < recs[y].t.cls;
+        return recs[x].cost > recs[y].cost;
     });
-    J.n_big = 0;
-    std::vector<int> newid(tasks.size());
-    for (size_t k = 0; k < order.size(); k++) {
-        const TaskRec &t = tasks[order[k]];
-        newid[order[k]] = (int)k;
-        J.n_big += big(order[k]) ? 1 : 0;
-        J.t_pair.push_back(t.pair);
-        J.t_e0.push_back(t.e0);
-        J.t_e1.push_back(t.e1);
+    struct Wg { int first, n, group; double cost; };
+    std::vector<Wg> wgs;
+    for (size_t i = 0; i < by.size();) {
+        size_t e = i;
+        const int cls = recs[by[i]].t.cls;
+        while (e < by.size() && e - i < (size_t)JIT_WPG && recs[by[e]].t.cls == cls) e++;
+        wgs.push_back(Wg{(int)i, (int)(e - i), jit_group(cls / JIT_NORD + cls % JIT_NORD), recs[by[i]].cost});
+        i = e;
     }
-    // each group's tasks in entry order (they were created in that order)
-    std::vector<std::vector<int>> gtasks(groups.size());
-    for (size_t t = 0; t < tasks.size(); t++) gtasks[tasks[t].group].push_back(newid[t]);
-    for (size_t gi = 0; gi < groups.size(); gi++) {
-        J.r_pair.push_back(groups[gi].pair);
-        J.r_omap.push_back(groups[gi].omap);
-        J.r_t0.push_back((int)J.r_tasks.size());
-        J.r_tasks.insert(J.r_tasks.end(), gtasks[gi].begin(), gtasks[gi].end());
-        J.r_t1.push_back((int)J.r_tasks.size());
+    std::stable_sort(wgs.begin(), wgs.end(), [](const Wg &x, const Wg &y) {
+        return x.group != y.group ? x.group < y.group : x.cost > y.cost;
+    });
+    std::vector<int> newid(recs.size());
+    for (const Wg &w : wgs) {
+        for (int k = 0; k < JIT_WPG; k++) {
+            JitTask t = recs[by[w.first + std::min(k, w.n - 1)]].t;
+            if (k < w.n) newid[by[w.first + k]] = (int)J.tasks.size();
+            else t.n = 0;
+            J.tasks.push_back(t);
+        }
+        J.gtask[w.group + 1] = (int)J.tasks.size();
     }
+    for (int g = 0; g < 3; g++) J.gtask[g + 1] = std::max(J.gtask[g + 1], J.gtask[g]);
+    for (int &t : J.ctask) t = newid[t];
+    for (int t : J.ctask) J.cpoff.push_back(J.tasks[t].poff);
+    // ---- entries with output rows, by class, longest first
+    for (const Target &t : targets)
+        for (int e = J.kl_start[t.list]; e < J.kl_start[t.list] + J.kl_count[t.list]; e++) J.oent.push_back(e);
+    std::stable_sort(J.oent.begin(), J.oent.end(), [&](int x, int y) {
+        const int *a = &J.pinfo[4 * J.kl_pair[x]], *b = &J.pinfo[4 * J.kl_pair[y]];
+        if (a[0] * 3 + a[1] != b[0] * 3 + b[1]) return a[0] * 3 + a[1] < b[0] * 3 + b[1];
+        return a[2] > b[2];
+    });
     // ---- every index within its array
     const long long space = (long long)N + J.nY;
     for (int k : J.kmap)
-        if (k < -1 || k >= space) { set_error(ERR_ARG, "on-the-fly B/D: input index %d out of range", k); return false; }
-    for (int k : J.omap)
-        if (k < -1 || k >= space) { set_error(ERR_ARG, "on-the-fly B/D: output index %d out of range", k); return false; }
+        if (k < -1 || k >= space) { set_error(ERR_ARG, "on-the-fly B/D: row index %d out of range", k); return false; }
     for (int k : J.uin)
         if (k < 0 || k >= space) { set_error(ERR_ARG, "on-the-fly B/D: sweep index %d out of range", k); return false; }
-    for (size_t e = 0; e < J.kl_pair.size(); e++)
+    for (size_t e = 0; e < ne; e++)
         if (J.kl_pair[e] < 0 || J.kl_pair[e] >= np || J.kl_moff[e] + h->sp_nbfp[J.kl_pair[e]] > (long long)J.kmap.size()) {
             set_error(ERR_ARG, "on-the-fly B/D: partner entry %zu out of range", e);
             return false;
         }
-    for (size_t t = 0; t < J.t_pair.size(); t++)
-        if (J.t_e0[t] < 0 || J.t_e0[t] > J.t_e1[t] || J.t_e1[t] > (int)J.gent.size()) {
-            set_error(ERR_ARG, "on-the-fly B/D: task %zu out of range", t);
-            return false;
-        }
-    for (int e : J.gent)
-        if (e < 0 || e >= (int)J.kl_pair.size()) { set_error(ERR_ARG, "on-the-fly B/D: entry %d out of range", e); return false; }
-    for (size_t g = 0; g < J.r_pair.size(); g++)
-        if (J.r_omap[g] + h->sp_nbfp[J.r_pair[g]] > (long long)J.omap.size() || J.r_t1[g] > (int)J.r_tasks.size()) {
-            set_error(ERR_ARG, "on-the-fly B/D: output group %zu out of range", g);
-            return false;
-        }
-    for (int t : J.r_tasks)
-        if (t < 0 || t >= (int)J.t_pair.size()) { set_error(ERR_ARG, "on-the-fly B/D: task id %d out of range", t); return false; }
     for (int i = 0; i < np; i++)
         if ((size_t)(J.pinfo[4 * i + 3] + J.pinfo[4 * i + 2]) * 6 > J.prim.size()) {
             set_error(ERR_ARG, "on-the-fly B/D: primitives of pair %d out of range", i);
             return false;
         }
-    // every quartet class fits its launch's LDS with at least one primitive
-    // quartet per batch (shells up to d; both orders <= 2 in the small launch)
-    for (int la = 0; la <= JIT_LMAX; la++)
-        for (int lb = 0; lb <= JIT_LMAX; lb++)
-            for (int lc = 0; lc <= JIT_LMAX; lc++)
-                for (int ld = 0; ld <= JIT_LMAX; ld++) {
-                    const int ncomp = jit_ncart(la) * jit_ncart(lb) * jit_ncart(lc) * jit_ncart(ld);
-                    const int ncd = jit_ncart(lc) * jit_ncart(ld), Lt = la + lb + lc + ld;
-                    const int perq = 3 * (la + 1) * (lb + 1) * (la + lb + 1) + 3 * (lc + 1) * (ld + 1) * (lc + ld + 1) +
-                                     jit_nherm(Lt) + Lt + 1;
-                    const int need = (ncomp > 64 ? ncomp : 64) + ncd + perq;
-                    if (need > (la + lb >= 3 || lc + ld >= 3 ? JIT_LDS : JIT_LDS_S)) {
-                        set_error(ERR_ARG, "on-the-fly B/D: LDS budget of class (%d%d|%d%d)", la, lb, lc, ld);
-                        return false;
-                    }
-                }
-    J.boys = boys_table(&J.bgrid, &J.bcol, &J.bstep, &J.btmax);
-    if (J.bcol < 2 * JIT_LMAX * 2 + 8) { set_error(ERR_ARG, "on-the-fly B/D: Boys table has too few orders"); return false; }
+    for (const JitTask &t : J.tasks) {
+        const int la = t.cls / JIT_NORD, lb = t.cls % JIT_NORD;
+        bool ok = t.cls >= 0 && la < JIT_NORD && t.n >= 0 && t.n <= (1 << t.lbw) && t.lbw <= 6 && t.c0 >= J.coff[la] &&
+                  t.c0 + t.n <= J.coff[la + 1] && t.s0 >= 0 && t.s1 * 2 <= (int)J.segs.size() &&
+                  t.poff + ((long long)jit_nherm(la) << t.lbw) <= J.npart;
+        for (int s = t.s0; ok && s < t.s1; s++)
+            ok = J.segs[2 * s] >= J.coff[lb] && J.segs[2 * s] <= J.segs[2 * s + 1] && J.segs[2 * s + 1] <= J.coff[lb + 1];
+        if (!ok) { set_error(ERR_ARG, "on-the-fly B/D: task out of range"); return false; }
+    }
+    for (const JitChunk &c : J.chunks) {
+        bool ok = c.t0 >= 0 && c.t0 <= c.t1 && c.t1 <= (int)J.ctask.size() && c.c0 >= J.coff[c.la] && c.c0 + c.n <= J.coff[c.la + 1];
+        for (int k = c.t0; ok && k < c.t1; k++)
+            ok = J.ctask[k] >= 0 && J.ctask[k] < (int)J.tasks.size() && J.tasks[J.ctask[k]].c0 == c.c0 && J.tasks[J.ctask[k]].lbw == c.lbw;
+        if (!ok) { set_error(ERR_ARG, "on-the-fly B/D: chunk out of range"); return false; }
+    }
+    for (int e : J.oent)
+        for (int i = J.e_c0[e]; i < J.e_c0[e + 1]; i++) {
+            const int l = J.pinfo[4 * J.kl_pair[e]] + J.pinfo[4 * J.kl_pair[e] + 1];
+            if (J.ecen[i] < J.coff[l] || J.ecen[i] >= J.coff[l + 1]) { set_error(ERR_ARG, "on-the-fly B/D: centre out of range"); return false; }
+        }
+    jit_boys_tables(J.boys);
     return true;
 }
 
@@ -1131,14 +1193,17 @@ struct JitState {
     JitPlan P;
     bool ready = false;
     int *d_ints = nullptr;      // every int array, one allocation
-    double *d_dbls = nullptr;   // pgeo, prim, boys, U
+    double *d_dbls = nullptr;   // pgeo, prim, Boys tables, centres, U
     long long *d_uoff = nullptr;
-    double *Y0 = nullptr, *Y1 = nullptr, *YJ = nullptr, *YD = nullptr, *part = nullptr;
+    JitTask *d_tasks = nullptr;
+    JitChunk *d_chunks = nullptr;
+    double *Y0 = nullptr, *Y1 = nullptr, *YJ = nullptr, *YD = nullptr, *part = nullptr, *HV = nullptr;
     JitView view{};
     const int *d_unr = nullptr, *d_unc = nullptr, *d_uin0 = nullptr, *d_y0off = nullptr, *d_uin = nullptr;
     const double *d_U = nullptr;
-    std::vector<const int *> d_level;   // node lists per level
-    std::vector<int> level_off;
+    // work items per level: (node, first column) up, (node, first row) down
+    std::vector<const int *> d_up, d_down;
+    std::vector<int> n_up, n_down;
     size_t bytes = 0;   // device memory held
     std::vector<hipEvent_t> ev;   // phase timing: 6 per vector
 };
@@ -1155,7 +1220,7 @@ struct JitState {
 void jit_release(JitState *&js) {
     if (!js) return;
     for (hipEvent_t e : js->ev) (void)hipEventDestroy(e);
-    void *ps[] = {js->d_ints, js->d_dbls, js->d_uoff, js->Y0, js->Y1, js->YJ, js->YD, js->part};
+    void *ps[] = {js->d_ints, js->d_dbls, js->d_uoff, js->d_tasks, js->d_chunks, js->Y0, js->Y1, js->part, js->HV};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     delete js;
@@ -1164,6 +1229,15 @@ void jit_release(JitState *&js) {
 
 size_t jit_resident_bytes(const JitState *js) { return js ? js->bytes : 0; }
 
+// The plan's scalars and, at the given array bases, its pointers.
+static void jit_view_counts(const JitPlan &P, JitView &v) {
+    v.N = P.N;
+    v.ncen = P.coff[JIT_NORD];
+    v.nent = (int)P.kl_pair.size();
+    for (int l = 0; l <= JIT_NORD; l++) v.coff[l] = P.coff[l];
+    for (int l = 0; l < JIT_NORD; l++) v.hoff[l] = P.hoff[l];
+}
+
 bool jit_upload(H2ERI_p h, JitState *&js) {
     if (js && js->ready) return true;
     jit_release(js);
@@ -1171,79 +1245,100 @@ bool jit_upload(H2ERI_p h, JitState *&js) {
     JitPlan &P = js->P;
     if (!jit_plan(h, P)) { jit_release(js); return false; }
     // int arrays, concatenated
-    std::vector<const std::vector<int> *> iv = {&P.pinfo, &P.r_pair, &P.r_omap, &P.kl_pair, &P.kl_moff, &P.kmap,
-                                                &P.t_pair, &P.t_e0, &P.t_e1, &P.gent, &P.r_t0, &P.omap,
-                                                &P.unr, &P.unc, &P.uin0, &P.y0off, &P.uin, &P.r_t1, &P.r_tasks};
+    std::vector<const std::vector<int> *> iv = {&P.pinfo, &P.kl_pair, &P.kl_moff, &P.kmap, &P.e_c0, &P.ecen,
+                                                &P.cptr, &P.cent, &P.cprim, &P.segs, &P.oent,
+                                                &P.unr, &P.unc, &P.uin0, &P.y0off, &P.uin};
     std::vector<int> ints;
     std::vector<size_t> ioff;
     for (auto *v : iv) { ioff.push_back(ints.size()); ints.insert(ints.end(), v->begin(), v->end()); }
-    js->level_off.clear();
-    for (auto &l : P.level_nodes) { js->level_off.push_back((int)ints.size()); ints.insert(ints.end(), l.begin(), l.end()); }
+    std::vector<size_t> up_off, down_off;
+    for (auto &l : P.level_nodes) {
+        up_off.push_back(ints.size());
+        for (int n : l)
+            for (int c = 0; c < P.unc[n]; c += 64) { ints.push_back(n); ints.push_back(c); }
+        down_off.push_back(ints.size());
+        for (int n : l)
+            for (int r = 0; r < P.unr[n]; r += JIT_DROWS) { ints.push_back(n); ints.push_back(r); }
+        js->n_up.push_back((int)(down_off.back() - up_off.back()) / 2);
+        js->n_down.push_back((int)(ints.size() - down_off.back()) / 2);
+    }
     ints.push_back(0);
     std::vector<double> dbls;
-    const size_t o_geo = 0;
-    dbls.insert(dbls.end(), P.pgeo.begin(), P.pgeo.end());
-    const size_t o_prim = dbls.size();
-    dbls.insert(dbls.end(), P.prim.begin(), P.prim.end());
-    const size_t o_boys = dbls.size();
-    dbls.insert(dbls.end(), P.boys, P.boys + (size_t)P.bgrid * P.bcol);
-    const size_t o_U = dbls.size();
-    dbls.insert(dbls.end(), P.U.begin(), P.U.end());
+    auto put = [&](const std::vector<double> &a) {
+        dbls.resize((dbls.size() + 31) & ~(size_t)31, 0.0);   // 256-byte starts
+        const size_t o = dbls.size();
+        dbls.insert(dbls.end(), a.begin(), a.end());
+        return o;
+    };
+    const size_t o_geo = put(P.pgeo), o_prim = put(P.prim), o_boys = put(P.boys), o_cen = put(P.cgeo), o_U = put(P.U);
     dbls.push_back(0.0);
     JIT_HIP(hipMalloc(&js->d_ints, ints.size() * sizeof(int)));
     JIT_HIP(hipMemcpy(js->d_ints, ints.data(), ints.size() * sizeof(int), hipMemcpyHostToDevice));
     JIT_HIP(hipMalloc(&js->d_dbls, dbls.size() * sizeof(double)));
     JIT_HIP(hipMemcpy(js->d_dbls, dbls.data(), dbls.size() * sizeof(double), hipMemcpyHostToDevice));
-    JIT_HIP(hipMalloc(&js->d_uoff, (P.uoff.size() + 1) * sizeof(long long)));
-    JIT_HIP(hipMemcpy(js->d_uoff, P.uoff.data(), P.uoff.size() * sizeof(long long), hipMemcpyHostToDevice));
-    const size_t ny = (size_t)std::max(P.nY, 1), nn = (size_t)std::max(P.N, 1);
+    std::vector<long long> lls(P.uoff);   // U offsets, then the partials' offsets
+    lls.insert(lls.end(), P.cpoff.begin(), P.cpoff.end());
+    lls.push_back(0);
+    JIT_HIP(hipMalloc(&js->d_uoff, lls.size() * sizeof(long long)));
+    JIT_HIP(hipMemcpy(js->d_uoff, lls.data(), lls.size() * sizeof(long long), hipMemcpyHostToDevice));
+    JIT_HIP(hipMalloc(&js->d_tasks, (P.tasks.size() + 1) * sizeof(JitTask)));
+    JIT_HIP(hipMemcpy(js->d_tasks, P.tasks.data(), P.tasks.size() * sizeof(JitTask), hipMemcpyHostToDevice));
+    JIT_HIP(hipMalloc(&js->d_chunks, (P.chunks.size() + 1) * sizeof(JitChunk)));
+    JIT_HIP(hipMemcpy(js->d_chunks, P.chunks.data(), P.chunks.size() * sizeof(JitChunk), hipMemcpyHostToDevice));
+    const size_t ny = (size_t)std::max(P.nY, 1), nn = (size_t)std::max(P.N, 1), nh = (size_t)P.nherm + 1;
     JIT_HIP(hipMalloc(&js->Y0, ny * sizeof(double)));
-    JIT_HIP(hipMalloc(&js->Y1, ny * sizeof(double)));
-    JIT_HIP(hipMalloc(&js->YJ, nn * sizeof(double)));
-    JIT_HIP(hipMalloc(&js->YD, nn * sizeof(double)));
-    const size_t npart = (size_t)std::max<size_t>(P.t_pair.size(), 1) * JIT_NAB;
-    JIT_HIP(hipMalloc(&js->part, npart * sizeof(double)));
-    js->bytes = ints.size() * sizeof(int) + dbls.size() * sizeof(double) + (P.uoff.size() + 1) * sizeof(long long) +
-                (2 * ny + 2 * nn + npart) * sizeof(double);
+    JIT_HIP(hipMalloc(&js->Y1, (ny + 2 * nn) * sizeof(double)));   // Y1, YJ, YD: cleared together
+    js->YJ = js->Y1 + ny;
+    js->YD = js->YJ + nn;
+    JIT_HIP(hipMalloc(&js->HV, 2 * nh * sizeof(double)));
+    JIT_HIP(hipMalloc(&js->part, ((size_t)P.npart + 1) * sizeof(double)));
+    js->bytes = ints.size() * sizeof(int) + dbls.size() * sizeof(double) + lls.size() * sizeof(long long) +
+                P.tasks.size() * sizeof(JitTask) + P.chunks.size() * sizeof(JitChunk) +
+                (2 * ny + 2 * nn + 2 * nh + (size_t)P.npart) * sizeof(double);
     const int *I = js->d_ints;
     JitView &v = js->view;
-    v.N = P.N;
+    jit_view_counts(P, v);
     v.pinfo = I + ioff[0];
-    v.r_pair = I + ioff[1];
-    v.r_omap = I + ioff[2];
-    v.kl_pair = I + ioff[3];
-    v.kl_moff = I + ioff[4];
-    v.kmap = I + ioff[5];
-    v.t_pair = I + ioff[6];
-    v.t_e0 = I + ioff[7];
-    v.t_e1 = I + ioff[8];
-    v.gent = I + ioff[9];
-    v.r_t0 = I + ioff[10];
-    v.omap = I + ioff[11];
-    js->d_unr = I + ioff[12];
-    js->d_unc = I + ioff[13];
-    js->d_uin0 = I + ioff[14];
-    js->d_y0off = I + ioff[15];
-    js->d_uin = I + ioff[16];
-    v.r_t1 = I + ioff[17];
-    v.r_tasks = I + ioff[18];
-    v.part = js->part;
-    js->d_level.clear();
-    for (int o : js->level_off) js->d_level.push_back(I + o);
+    v.kl_pair = I + ioff[1];
+    v.kl_moff = I + ioff[2];
+    v.kmap = I + ioff[3];
+    v.e_c0 = I + ioff[4];
+    v.ecen = I + ioff[5];
+    v.cptr = I + ioff[6];
+    v.cent = I + ioff[7];
+    v.cprim = I + ioff[8];
+    v.segs = I + ioff[9];
+    v.oent = I + ioff[10];
+    js->d_unr = I + ioff[11];
+    js->d_unc = I + ioff[12];
+    js->d_uin0 = I + ioff[13];
+    js->d_y0off = I + ioff[14];
+    js->d_uin = I + ioff[15];
+    v.cpoff = js->d_uoff + P.uoff.size();
+    for (size_t o : up_off) js->d_up.push_back(I + o);
+    for (size_t o : down_off) js->d_down.push_back(I + o);
     v.pgeo = js->d_dbls + o_geo;
     v.prim = js->d_dbls + o_prim;
     v.boys = js->d_dbls + o_boys;
-    v.bgrid = P.bgrid;
-    v.bcol = P.bcol;
-    v.bstep = P.bstep;
-    v.btmax = P.btmax;
-    v.inv_bstep = 1.0 / P.bstep;
+    v.cgeo = js->d_dbls + o_cen;
     js->d_U = js->d_dbls + o_U;
+    v.H = js->HV;
+    v.V = js->HV + nh;
+    v.tasks = js->d_tasks;
+    v.chunks = js->d_chunks;
+    v.part = js->part;
     v.Y0 = js->Y0;
     v.Y1 = js->Y1;
     v.YJ = js->YJ;
     js->ready = true;
     return true;
+}
+
+template <int G>
+static void jit_launch_potential(const JitPlan &P, const JitView &v, hipStream_t s) {
+    const int t0 = P.gtask[G], nwg = (P.gtask[G + 1] - t0) / JIT_WPG;
+    if (nwg > 0)
+        hipLaunchKernelGGL(jit_potential_kernel<G>, dim3(nwg), dim3(64 * JIT_WPG), 0, s, v, v.tasks + t0, v.cgeo, v.H, v.segs, v.boys);
 }
 
 bool jit_matvec(H2ERI_p h, JitState *js, int nvec, const double *X, double *Y, void *stream, double *ms5) {
@@ -1265,40 +1360,36 @@ bool jit_matvec(H2ERI_p h, JitState *js, int nvec, const double *X, double *Y, v
         const double *x = X + (size_t)k * N;
         double *y = Y + (size_t)k * N;
         if (!mark(k, 0)) return false;
-        hipLaunchKernelGGL(jit_zero_kernel, dim3(1024), dim3(256), 0, s, js->Y1, (long long)std::max(P.nY, 1));
-        hipLaunchKernelGGL(jit_zero_kernel, dim3(1024), dim3(256), 0, s, js->YJ, (long long)std::max(N, 1));
-        hipLaunchKernelGGL(jit_zero_kernel, dim3(1024), dim3(256), 0, s, js->YD, (long long)std::max(N, 1));
+        const long long nz = (long long)std::max(P.nY, 1) + 2LL * std::max(N, 1);   // Y1, YJ, YD
+        hipLaunchKernelGGL(jit_zero_kernel, dim3((unsigned)std::min<long long>(1024, (nz + 255) / 256)), dim3(256), 0, s, js->Y1, nz);
         JIT_HIP(hipGetLastError());
         if (!mark(k, 1)) return false;
         for (int L = P.max_level; L >= 0; L--) {
-            const int nn = (int)P.level_nodes[L].size();
-            if (nn == 0) continue;
-            hipLaunchKernelGGL(jit_up_kernel, dim3(nn), dim3(256), 0, s, js->d_level[L], js->d_uoff, js->d_unr,
+            if (js->n_up[L] == 0) continue;
+            hipLaunchKernelGGL(jit_up_kernel, dim3(js->n_up[L]), dim3(1024), 0, s, js->d_up[L], js->d_uoff, js->d_unr,
                                js->d_unc, js->d_uin0, js->d_y0off, js->d_uin, js->d_U, x, js->Y0, N);
             JIT_HIP(hipGetLastError());
         }
         if (!mark(k, 2)) return false;
         JitView v = js->view;
         v.X = x;
-        const int ntask = (int)P.t_pair.size();
-        if (P.n_big > 0) {
-            hipLaunchKernelGGL(jit_task_kernel<JIT_LDS>, dim3(P.n_big), dim3(64), 0, s, v, 0, P.n_big);
-            JIT_HIP(hipGetLastError());
-        }
-        if (ntask > P.n_big) {
-            hipLaunchKernelGGL(jit_task_kernel<JIT_LDS_S>, dim3(ntask - P.n_big), dim3(64), 0, s, v, P.n_big, ntask);
-            JIT_HIP(hipGetLastError());
-        }
-        const int ngroup = (int)P.r_pair.size();
-        if (ngroup > 0) {
-            hipLaunchKernelGGL(jit_reduce_kernel, dim3((ngroup + 255) / 256), dim3(256), 0, s, v, ngroup);
-            JIT_HIP(hipGetLastError());
-        }
+        unsigned ndens = 0;
+        for (int l = 0; l < JIT_NORD; l++) ndens += (unsigned)(P.coff[l + 1] - P.coff[l] + 255) / 256;
+        if (ndens > 0) hipLaunchKernelGGL(jit_density_kernel, dim3(ndens), dim3(256), 0, s, v);
+        JIT_HIP(hipGetLastError());
+        jit_launch_potential<2>(P, v, s);
+        jit_launch_potential<1>(P, v, s);
+        jit_launch_potential<0>(P, v, s);
+        JIT_HIP(hipGetLastError());
+        if (!P.chunks.empty()) hipLaunchKernelGGL(jit_reduce_kernel, dim3((unsigned)P.chunks.size()), dim3(256), 0, s, v);
+        const int nout = (int)P.oent.size();
+        if (nout > 0)
+            hipLaunchKernelGGL(jit_rows_kernel, dim3((unsigned)(((long long)nout * JIT_RLANES + 255) / 256)), dim3(256), 0, s, v, nout);
+        JIT_HIP(hipGetLastError());
         if (!mark(k, 3)) return false;
         for (int L = 0; L <= P.max_level; L++) {
-            const int nn = (int)P.level_nodes[L].size();
-            if (nn == 0) continue;
-            hipLaunchKernelGGL(jit_down_kernel, dim3(nn), dim3(256), 0, s, js->d_level[L], js->d_uoff, js->d_unr,
+            if (js->n_down[L] == 0) continue;
+            hipLaunchKernelGGL(jit_down_kernel, dim3(js->n_down[L]), dim3(256), 0, s, js->d_down[L], js->d_uoff, js->d_unr,
                                js->d_unc, js->d_uin0, js->d_y0off, js->d_uin, js->d_U, js->YD, js->Y1, N);
             JIT_HIP(hipGetLastError());
         }
@@ -1324,15 +1415,48 @@ bool jit_matvec(H2ERI_p h, JitState *js, int nvec, const double *X, double *Y, v
     return true;
 }
 
+// ---------------------------------------------------------------------------
+// Host emulation (tests)
+// ---------------------------------------------------------------------------
+template <int LA, int LB>
+static void jit_potential_host(const JitView &v, const JitTask &t, const double *bt) {
+    constexpr int NA = jit_nherm(LA), NB = jit_nherm(LB);
+    const int bw = 1 << t.lbw, ns = 64 >> t.lbw;
+    const double *Hb = v.H + v.hoff[LB] - (long long)v.coff[LB] * NB;
+    for (int b = 0; b < t.n; b++) {
+        const double *bg = v.cgeo + 4 * (size_t)(t.c0 + b);
+        std::vector<double> V((size_t)NA * ns, 0.0);
+        for (int sg = t.s0; sg < t.s1; sg++)
+            for (int sl = 0; sl < ns; sl++)
+                for (int j = v.segs[2 * sg] + sl; j < v.segs[2 * sg + 1]; j += ns) {
+                    const double *g = v.cgeo + 4 * (size_t)j;
+                    jit_pair<LA, LB>(bg[0], bg[1], bg[2], bg[3], g[0], g[1], g[2], g[3], Hb + (long long)j * NB, bt, &V[(size_t)NA * sl]);
+                }
+        for (int k = 0; k < NA; k++) {
+            double s = 0.0;
+            for (int sl = 0; sl < ns; sl++) s += V[(size_t)NA * sl + k];
+            v.part[t.poff + (long long)k * bw + b] = s;
+        }
+    }
+}
+template <int... C>
+static void jit_potential_host_any(const JitView &v, const JitTask &t, const double *bt, std::integer_sequence<int, C...>) {
+    ([&] { if (t.cls == C) jit_potential_host<C / JIT_NORD, C % JIT_NORD>(v, t, bt); }(), ...);
+}
+template <int L>
+static void jit_density_host(const JitView &v) {
+    for (int c = v.coff[L]; c < v.coff[L + 1]; c++) jit_density<L>(v, c);
+}
+
 }  // namespace h2e
 
 using namespace h2e;
 
 extern "C" {
 
-// Host execution of the on-the-fly matvec (tests only): the same row-task
-// code on one lane, the sweeps as plain loops.  Returns 0, or -1 with the
-// error set.
+// Host execution of the on-the-fly matvec (tests only): the device's
+// densities, pair terms and rows on the host, the sweeps as plain loops.
+// Returns 0, or -1 with the error set.
 int H2ERI_jit_emulate(H2ERI_p h, const double *x, double *y) {
     if (!h || !x || !y) { set_error(ERR_ARG, "jit_emulate: null argument"); return -1; }
     JitPlan P;
@@ -1353,25 +1477,31 @@ int H2ERI_jit_emulate(H2ERI_p h, const double *x, double *y) {
             }
         }
     JitView v{};
-    v.N = N;
-    v.pinfo = P.pinfo.data(); v.pgeo = P.pgeo.data(); v.prim = P.prim.data();
-    v.boys = P.boys; v.bgrid = P.bgrid; v.bcol = P.bcol; v.bstep = P.bstep; v.btmax = P.btmax; v.inv_bstep = 1.0 / P.bstep;
+    jit_view_counts(P, v);
+    v.pinfo = P.pinfo.data(); v.pgeo = P.pgeo.data(); v.prim = P.prim.data(); v.boys = P.boys.data();
     v.kl_pair = P.kl_pair.data(); v.kl_moff = P.kl_moff.data(); v.kmap = P.kmap.data();
-    v.t_pair = P.t_pair.data(); v.t_e0 = P.t_e0.data(); v.t_e1 = P.t_e1.data(); v.gent = P.gent.data();
-    v.r_pair = P.r_pair.data(); v.r_omap = P.r_omap.data(); v.r_t0 = P.r_t0.data(); v.r_t1 = P.r_t1.data();
-    v.r_tasks = P.r_tasks.data(); v.omap = P.omap.data();
-    std::vector<double> part(std::max<size_t>(P.t_pair.size(), 1) * JIT_NAB, 0.0);
+    v.e_c0 = P.e_c0.data(); v.ecen = P.ecen.data(); v.cptr = P.cptr.data(); v.cent = P.cent.data(); v.cprim = P.cprim.data();
+    v.cgeo = P.cgeo.data(); v.tasks = P.tasks.data(); v.segs = P.segs.data(); v.chunks = P.chunks.data();
+    v.cpoff = P.cpoff.data(); v.oent = P.oent.data();
+    std::vector<double> part((size_t)P.npart + 1, 0.0), HV(2 * (size_t)P.nherm + 2, 0.0);
     v.part = part.data();
+    v.H = HV.data();
+    v.V = HV.data() + P.nherm + 1;
     v.X = x; v.Y0 = Y0.data(); v.YJ = YJ.data(); v.Y1 = Y1.data();
-    const int ntask = (int)P.t_pair.size();
+    jit_density_host<0>(v);
+    jit_density_host<1>(v);
+    jit_density_host<2>(v);
+    jit_density_host<3>(v);
+    jit_density_host<4>(v);
+    const int ntask = (int)P.tasks.size();
     std::atomic<int> next(0);
     auto worker = [&]() {
-        std::vector<double> lds(JIT_LDS);
-        std::vector<long long> pk(6 * (JIT_KMAX + 1));
         for (int t = next++; t < ntask; t = next++) {
-            const short *hm = &jit_tabs_host.herm[0][0][0], *eo = &jit_tabs_host.eoff[0][0];
-            if (t < P.n_big) jit_task<1, JIT_LDS, 3>(v, t, 0, lds.data(), hm, eo, pk.data());
-            else jit_task<1, JIT_LDS_S, 2>(v, t, 0, lds.data(), hm, eo, pk.data());
+            const JitTask &tk = P.tasks[t];
+            if (tk.n == 0) continue;
+            const int LT = tk.cls / JIT_NORD + tk.cls % JIT_NORD;
+            jit_potential_host_any(v, tk, v.boys + (size_t)LT * JIT_BGRID * JIT_BROW,
+                                   std::make_integer_sequence<int, JIT_NORD * JIT_NORD>{});
         }
     };
     const int nth = std::max(1, std::min(16, (int)std::thread::hardware_concurrency()));
@@ -1379,7 +1509,8 @@ int H2ERI_jit_emulate(H2ERI_p h, const double *x, double *y) {
     for (int i = 1; i < nth; i++) pool.emplace_back(worker);
     worker();
     for (auto &th : pool) th.join();
-    for (int g = 0; g < (int)P.r_pair.size(); g++) jit_reduce(v, g);
+    for (const JitChunk &c : P.chunks) jit_reduce(v, c, 0, 1);
+    for (int e : P.oent) jit_rows_any<1>(v, e, 0);
     for (int L = 0; L <= P.max_level; L++)
         for (int n : P.level_nodes[L]) {
             const double *Un = P.U.data() + P.uoff[n];
@@ -1396,13 +1527,14 @@ int H2ERI_jit_emulate(H2ERI_p h, const double *x, double *y) {
     return 0;
 }
 
-// Work of one on-the-fly matvec: out4 = {row tasks, shell quartets,
-// primitive quartets, integral values}.  Host only.  Returns 0 or -1.
+// Work of one on-the-fly matvec: out4 = {tasks, shell quartets, primitive
+// quartets, integral values}, each block counted from both sides.  Host only.
+// Returns 0 or -1.
 int H2ERI_jit_stats(H2ERI_p h, double *out4) {
     if (!h || !out4) { set_error(ERR_ARG, "jit_stats: null argument"); return -1; }
     JitPlan P;
     if (!jit_plan(h, P)) return -1;
-    out4[0] = (double)P.t_pair.size();
+    out4[0] = (double)P.ntask;
     out4[1] = P.quartets;
     out4[2] = P.prim_quartets;
     out4[3] = P.eri_values;

@@ -500,11 +500,11 @@ int H2ERI_plan_stats(H2ERI_p h2eri, const int ub_bits, const int nv, double *out
 int H2ERI_plan_emulate(H2ERI_p h2eri, const int ub_bits, const int nv, const double *X, double *Y);
 
 /* Host execution of a BD_JIT matvec (no HIP call, tests only): the device's
- * row-task code on one lane, the sweeps as plain loops; y = A x.  Returns 0,
- * -1 on failure. */
+ * densities, pair terms and rows on the host, the sweeps as plain loops;
+ * y = A x.  Returns 0, -1 on failure. */
 int H2ERI_jit_emulate(H2ERI_p h2eri, const double *x, double *y);
 
-/* Work of one BD_JIT matvec, counted on the host: out4 = {row tasks, shell
+/* Work of one BD_JIT matvec, counted on the host: out4 = {tasks, shell
  * quartets, primitive quartets, integral values}.  Returns 0, -1 on failure. */
 int H2ERI_jit_stats(H2ERI_p h2eri, double *out4);
 
