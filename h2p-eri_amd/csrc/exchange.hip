@@ -41,6 +41,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <map>
 #include <numeric>
 
 #include "h2eri_internal.h"
@@ -62,8 +63,6 @@ struct KTerm {
     long long Loff;
     int Rsrc, Rrs, Rcs;   // R[c][t] = src[Roff + c*Rrs + t*Rcs]
     long long Roff;
-    long long Goff;       // G in its chunk's scratch: [q / 8][n][t][q % 8], gld(|B(j)|) / 8 blocks
-    int pad_[2];
 };
 
 struct KGemm {           // out (m x n, ld ldo) = A (m x k, PB, ld lda) * X (k x n, CB, ld ldx)
@@ -73,9 +72,9 @@ struct KGemm {           // out (m x n, ld ldo) = A (m x k, PB, ld lda) * X (k x
 
 struct KTask {           // one workgroup: term and tile origin
     int term;
-    int e0;               // ket: first local n; bra: first local q; direct: first (m,q) index
-    int t0;               // ket: first t; bra: split of local m
-    int pad_;             // ket: first local q
+    int e0;               // block: first local q; direct: first (m,q) index
+    int t0;               // block: split of local m
+    int pad_;
 };
 
 struct KGemmTask {
@@ -86,25 +85,18 @@ struct KNode {           // per row/column range: basis-function set and the ori
     int bf_off, nbf;      // B(node) = bfidx[bf_off .. bf_off + nbf)
     int q_ptr;            // byQ CSR rows: qptr[q_ptr .. q_ptr + nbf]   entries (column c, p)
     int m_ptr;            // byM CSR rows: mptr[m_ptr .. m_ptr + nbf]   entries (row r, local n)
-    int s_ptr;            // byN split table: nspl[s_ptr + n * (nsplit + 1) + s] = first entry (row r, local m)
-    int nsplit;           //   of local n with local m >= s * ssz (entries of each n sorted by m)
-    int ssz;              // functions m per split: the nbf functions in nsplit = ceil(nbf / KSPLIT) even parts
+    int g_ptr;            // merged lists of pairs of q: gptr[g_ptr + g]   entries (p, columns c of the two q)
+    int b_ptr;            // bra block lists: bptr[b_ptr + ((split * steps of 16 n) + step) * 8 + wave], and the next one
+    int nsplit;           // splits of the functions m
+    int ssz;              // functions m per split: the nbf functions in nsplit = ceil(nbf / KM) even parts
 };
 
 static const int KWG = 256;
-// G is stored in blocks of 8 functions q, [q / 8][n][t][q % 8]: a ket task
-// (8 q) then writes whole 64-byte (n, t) records, two per 128-byte line, and
-// four consecutive q form one aligned 32-byte store.  gld(|B(j)|) is the
-// padded q count.
-__host__ __device__ inline int gld(int nbf_j) { return (nbf_j + 7) & ~7; }
-__device__ inline size_t gidx(int q, int n, int t, int nbf_i, int kk) {
-    return (((size_t)(q >> 3) * nbf_i + n) * kk + t) * 8 + (q & 7);
-}
 // Workgroups are dispatched to the 8 XCDs round-robin by id, and each XCD has
 // its own L2.  This bijection of [0, n) hands out runs of C consecutive tasks
 // of the list, run j to XCD j mod 8 (the tail of fewer than 8 runs is split
 // into 8 contiguous ranges), so tasks next to each other in the list, which
-// share G columns, L rows or R rows, read them through one L2.
+// share L rows and D, read them through one L2.
 __device__ inline int xcd_task(int bid, int n, int C) {
     const int full = n / (8 * C);
     const int x = bid & 7, k = bid >> 3;
@@ -112,250 +104,231 @@ __device__ inline int xcd_task(int bid, int n, int C) {
     const int n2 = n - full * 8 * C, k2 = (bid - full * 8 * C) >> 3, q = n2 >> 3, r = n2 & 7;
     return full * 8 * C + x * q + min(x, r) + k2;
 }
-// runs of consecutive tasks per XCD (measured on C30H62: K 16.3 ms with the
-// plain round-robin order, 15.5 ms with these; one contiguous range per XCD
-// cut the bra's HBM reads from 39 to 22 GB but unbalanced the XCDs)
-static const int KRUN_KET = 64, KRUN_BRA = 8;
-static const int KQC = 8;       // column functions q per ket task (one group of four per wave)
-// most local m rows per bra task (LDS block KSPLIT x 32); on C30H62, with
-// tasks of 16 q, K took 13.0 ms with 256, 12.5 ms with 192 and even splits,
-// 12.9 ms with 160
-static const int KSPLIT = 192;
-static const int KEB = 4;       // entry blocks of 16 sharing one walk over t in the bra
+static const int KRUN = 8;      // consecutive tasks per XCD
+static const int KQ = 16;       // column functions q per task (eight pairs)
+static const int KGN = 258;     // doubles per function n of the G tile (16 t x 16 q, and two that shift the LDS banks)
+static const int KGT = 16 * KGN;
+static const int KBWG = 512;    // threads of a block task (8 waves)
+static const int KPAD = 32;     // readable doubles past every operand array
+// Most local functions m of a task (its K block in LDS): 352, the G tile and
+// the node's function offsets take 79,488 bytes, two workgroups per CU; the
+// functions of a larger node are cut into even splits, each of which forms
+// its G again.
+static const int KM = 352;
+static const int KMNONE = 0xffffff;   // local m of a block's row without an entry (24 bits)
 
-// Ket on MFMA: G[n][t][q] = sum over the entries (c, p) of q of R[c][t] D[n][p].
-// Per q this is a GEMM (rows t, columns n, inner dimension the entries of q).
-// Task = (term, t tile of 16, 64 functions n, KQC functions q); the four
-// waves split it 2 x 2 into 32 functions n (two MFMA tiles that share every
-// gathered R operand and entry index) by KQC / 2 functions q.  A wave computes
-// four consecutive q together, walking their entry lists in step, and stores
-// the four q of each (n, t) record as one aligned 32-byte write (single
-// 8-byte writes scattered over 16 rows cost four times their bytes in HBM
-// write traffic).  Registers are capped for four waves per SIMD: uncapped, the
-// eight accumulators take 200 and halve the waves that hide the gathers.
-__global__ __launch_bounds__(KWG) __attribute__((amdgpu_waves_per_eu(4))) void kx_ket(const KTask *__restrict__ tasks, const KTerm *__restrict__ terms,
-                                               const KNode *__restrict__ nodes, const int *__restrict__ bfidx,
-                                               const int *__restrict__ qptr, const int2 *__restrict__ qent,
-                                               const double *__restrict__ PB, const double *__restrict__ CB,
-                                               const double *__restrict__ SC, double *__restrict__ GS,
-                                               const double *__restrict__ D, int nbf) {
-    const KTask tk = tasks[xcd_task(blockIdx.x, gridDim.x, KRUN_KET)];   // term, nl0, t0, ql0
-    const KTerm t = terms[tk.term];
-    const KNode ni = nodes[t.ni], nj = nodes[t.nj];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    // wave w: functions n [nl0, nl0 + 32) as two MFMA tiles that share every
-    // R operand, and half of the task's functions q
-    const int nl0 = tk.e0 + 32 * (w & 1);
-    static_assert(KQC % 8 == 0, "each wave stores whole groups of four q");
-    const int qbeg = tk.pad_ + (KQC / 2) * (w >> 1);
-    const int qend = min(qbeg + KQC / 2, nj.nbf);
-    if (nl0 >= ni.nbf || qbeg >= qend) return;   // whole wave
-    const double *R = (t.Rsrc == KS_PB ? PB : (t.Rsrc == KS_CB ? CB : SC)) + t.Roff;
-    int nl[2], bfn[2];
-    bool nv[2];
-    #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        nl[h] = nl0 + 16 * h + (lane & 15);
-        nv[h] = nl[h] < ni.nbf;
-        // D is symmetric (the entry point's contract), so D[n][p] is read as
-        // D[p][n]: the 16 lanes of an entry (consecutive functions n of the
-        // node) read along one row of D instead of down a column
-        bfn[h] = nv[h] ? bfidx[ni.bf_off + nl[h]] : 0;
-    }
-    const int ta = tk.t0 + (lane & 15);   // A operand row (t)
-    const bool tv = ta < t.kk;
-    const int kl = lane >> 4;
-    double *G = GS + t.Goff;
-    for (int qg = qbeg; qg < qend; qg += 4) {
-        // The entry lists of the four q are walked together (entries past a
-        // list are zeros), so each iteration has the gathers of eight
-        // independent accumulations in flight.
-        int qa[4], qb[4], len = 0;
-        #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int ql = qg + j;
-            qa[j] = ql < qend ? qptr[nj.q_ptr + ql] : 0;
-            qb[j] = ql < qend ? qptr[nj.q_ptr + ql + 1] : 0;
-            len = max(len, qb[j] - qa[j]);
-        }
-        d4 acc[2][4];
-        #pragma unroll
-        for (int h = 0; h < 2; h++)
-            #pragma unroll
-            for (int j = 0; j < 4; j++) acc[h][j] = d4{0.0, 0.0, 0.0, 0.0};
-        // entry indices come in windows of 16 per q: lane l loads entry
-        // (l & 15) of q (l >> 4) and the lanes of each step take theirs by
-        // a cross-lane shuffle, which keeps them off the vector memory path
-        const int jq = lane >> 4;
-        const int wa = jq == 0 ? qa[0] : jq == 1 ? qa[1] : jq == 2 ? qa[2] : qa[3];
-        const int wb = jq == 0 ? qb[0] : jq == 1 ? qb[1] : jq == 2 ? qb[2] : qb[3];
-        for (int w0 = 0; w0 < len; w0 += 16) {
-            const int ew = wa + w0 + (lane & 15);
-            const int2 mine = ew < wb ? qent[ew] : make_int2(-1, 0);
-            for (int s4 = 0; s4 < 16 && w0 + s4 < len; s4 += 4) {
-                int2 cp[4];
-                #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int src = 16 * j + s4 + kl;
-                    cp[j] = make_int2(__shfl(mine.x, src), __shfl(mine.y, src));
-                }
-                double a[4], b[2][4];
-                #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const bool ev = cp[j].x >= 0;
-                    a[j] = (ev && tv) ? R[(long long)cp[j].x * t.Rrs + (long long)ta * t.Rcs] : 0.0;
-                    #pragma unroll
-                    for (int h = 0; h < 2; h++) b[h][j] = (ev && nv[h]) ? D[(size_t)cp[j].y * nbf + bfn[h]] : 0.0;
-                }
-                #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    #pragma unroll
-                    for (int h = 0; h < 2; h++) acc[h][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j], b[h][j], acc[h][j], 0, 0, 0);
-            }
-        }
-        #pragma unroll
-        for (int h = 0; h < 2; h++)
-            #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int tt = tk.t0 + kl + 4 * r;
-                if (tt < t.kk && nv[h])
-                    *reinterpret_cast<d4 *>(G + gidx(qg, nl[h], tt, ni.nbf, t.kk)) =
-                        d4{acc[h][0][r], acc[h][1][r], acc[h][2][r], acc[h][3][r]};
-            }
-    }
+// Operand addresses are a uniform base and a byte offset O per lane: 32 bits,
+// or 64 where an operand array of a term or D is larger than 4 GB (or a node
+// has more functions than the LDS should list).
+struct __attribute__((packed, aligned(8))) KU2 { double x, y; };   // 16 bytes at 8-byte alignment
+template <typename O>
+__device__ __forceinline__ void kload4(const double *p, O byte, double (&o)[4]) {
+    const KU2 *q = reinterpret_cast<const KU2 *>(reinterpret_cast<const char *>(p) + byte);
+    const KU2 a = q[0], b = q[1];
+    o[0] = a.x; o[1] = a.y; o[2] = b.x; o[3] = b.y;
+}
+template <typename O>
+__device__ __forceinline__ double kload(const double *p, O byte) {
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + byte);
 }
 
-// Bra on MFMA: K[m][q] += sum_n sum_{(r,m) of n} sum_t L[r][t] G[n][t][q].
-// For each n the rows r that pair with n form a GEMM (rows: those entries,
-// columns q, inner dimension t).  Task = (term, 32 functions q as two MFMA
-// column tiles that share every L operand, split of ssz <= KSPLIT functions
-// m); wave w takes the functions n = w, w + 4, ... and adds its 16 x 16
-// output tiles into an LDS block of the split with FP64 LDS atomics (tiles
-// of different n may share an m); the block is added into K at the end.
-// Tasks of 16 q read every L row twice as often: K 12.5 ms against 12.1.  The t loop issues the operands of four MFMA steps at once,
-// and one walk over t serves up to KEB blocks of 16 entries of n, which share
-// its G operands.
-__global__ __launch_bounds__(KWG) void kx_bra(const KTask *__restrict__ tasks, const KTerm *__restrict__ terms,
-                                               const KNode *__restrict__ nodes, const int *__restrict__ bfidx,
-                                               const int *__restrict__ nspl, const int2 *__restrict__ nent,
-                                               const double *__restrict__ PB, const double *__restrict__ CB,
-                                               const double *__restrict__ SC, const double *__restrict__ GS,
-                                               double *__restrict__ K1, double *__restrict__ Kd, int nbf) {
-    __shared__ double Kb[KSPLIT * 32];
-    const KTask tk = tasks[xcd_task(blockIdx.x, gridDim.x, KRUN_BRA)];   // term, ql0, split
+// One block term's share of K: a workgroup takes 16 functions q of the column
+// node and a split of the row node's functions m, and walks the functions n
+// of the row node in steps of 16 and the inner index t in steps of 16:
+//   ket  G[n][t][q] = sum over the entries (c, p) of q of R[c][t] D[p][n]
+//        into LDS: wave w the functions q = 2w, 2w+1, one MFMA tile
+//        (16 t x 16 n) each.  The two entry lists are merged on p, so that
+//        one D operand serves both; an entry a function does not have meets
+//        a zero D operand.  D is symmetric (the entry point's contract):
+//        D[p][n] lets the 16 lanes of an entry read along a row.
+//   bra  K[m][q] += sum over the entries (r, m) of n of L[r][t] G[n][t][q]:
+//        the entries of every n in blocks of 16 rows, dealt to the waves in
+//        turn; a block's tile is added into the K block in LDS with FP64 LDS
+//        atomics (tiles of different n may share an m).
+// At the end the K block is added into K with FP64 global atomics.
+//
+// Both loops take their operands as one stream over all steps: while eight
+// ket entries (or one bra block) are consumed the next ones are in flight,
+// across the barriers too, and their indices one further ahead.  16 waves
+// per CU (128 VGPRs, two workgroups by LDS) cover the rest.
+//
+// What bounds it: the operand loads' address path (busy for over half of the
+// time) and FP64 MFMA issue (64 cycles each, 37%); half of the MFMA work is
+// padding, since entries per function come in eights (ket) and sixteens
+// (bra).  G stays in LDS: as two kernels with G in HBM (14.7 GB for C30H62,
+// 73 GB for (H2O)64, written and read back) a build was bound by that round
+// trip and by twice the ket's D loads.  K per build, two kernels / this one:
+// C10H22 2.77 / 1.51 ms, C30H62 13.1 / 7.4 ms, (H2O)64 76.6 / 41.5 ms.  Tried:
+// four waves of four q each with everything prefetched into registers (2
+// waves per SIMD, waits that the compiler cannot order: C30H62 20.5 ms); a
+// third workgroup per CU for nodes of at most 152 functions (no gain).
+template <typename O>
+__global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ tasks, const KTerm *__restrict__ terms,
+                                                    const KNode *__restrict__ nodes, const int *__restrict__ bfidx,
+                                                    const int *__restrict__ gptr, const int4 *__restrict__ ge,
+                                                    const int *__restrict__ bptr, const int2 *__restrict__ brow,
+                                                    const double *__restrict__ PB, const double *__restrict__ CB,
+                                                    const double *__restrict__ SC, const double *__restrict__ D,
+                                                    double *__restrict__ KA, int nacc, int nbf) {
+    extern __shared__ double lds[];
+    const KTask tk = tasks[xcd_task(blockIdx.x, gridDim.x, KRUN)];   // term, first q, split
     const KTerm t = terms[tk.term];
     const KNode ni = nodes[t.ni], nj = nodes[t.nj];
-    const int split = tk.t0, ql0 = tk.e0;
-    const int ml0 = split * ni.ssz;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, kl = lane >> 4;
-    for (int i = threadIdx.x; i < KSPLIT * 32; i += KWG) Kb[i] = 0.0;
+    double *Gt = lds, *Kb = lds + KGT;
+    int *nof = reinterpret_cast<int *>(Kb + ni.ssz * KQ);   // function of every local n (32-bit form)
+    const int q0 = tk.e0, split = tk.t0, ml0 = split * ni.ssz;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int l16 = lane & 15, kl = lane >> 4;
+    const int mlN = min(ni.ssz, ni.nbf - ml0);
+    for (int i = threadIdx.x; i < mlN * KQ; i += KBWG) Kb[i] = 0.0;
+    if (sizeof(O) == 4)
+        for (int i = threadIdx.x; i < ni.nbf; i += KBWG) nof[i] = bfidx[ni.bf_off + i];
+    auto func = [&](int n) { return sizeof(O) == 4 ? nof[n] : bfidx[ni.bf_off + n]; };
     __syncthreads();
     const double *L = (t.Lsrc == KS_PB ? PB : (t.Lsrc == KS_CB ? CB : SC)) + t.Loff;
-    const double *G = GS + t.Goff;
-    bool qv[2];
-    #pragma unroll
-    for (int h = 0; h < 2; h++) qv[h] = ql0 + 16 * h + (lane & 15) < nj.nbf;
-    const int ns1 = ni.nsplit + 1;
-    for (int nl = w; nl < ni.nbf; nl += KWG / 64) {
-        const int eb = nspl[ni.s_ptr + nl * ns1 + split], ee = nspl[ni.s_ptr + nl * ns1 + split + 1];
-        const double *Gn[2];
+    const double *R = (t.Rsrc == KS_PB ? PB : (t.Rsrc == KS_CB ? CB : SC)) + t.Roff;
+    const int kk = t.kk, nstep = (ni.nbf + 15) >> 4;
+    const O Rrs = (O)t.Rrs * 8, Rcs = (O)t.Rcs * 8, Lld = (O)t.Lld * 8, Dld = (O)nbf * 8;
+
+    // ---- ket stream: entries in eights, s within the list, t0 and n0 of the tile
+    const int grp = (q0 >> 1) + w;
+    const bool gok = 2 * grp < nj.nbf;
+    const int ga = gok ? gptr[nj.g_ptr + grp] : 0, gs = gok ? (gptr[nj.g_ptr + grp + 1] - ga) >> 3 : 0;
+    int ks = 0, kt = 0, kn = 0;    // position of the operands loaded next
+    int4 xc[2];                    // the entries loaded next (columns of the two q, p)
+    int2 oc[2];                    // columns of the operands in flight
+    double oa[2][2], od[2];
+    auto ket_index = [&](int s) {
         #pragma unroll
-        for (int h = 0; h < 2; h++) Gn[h] = G + gidx(min(ql0 + 16 * h + (lane & 15), gld(nj.nbf) - 1), nl, 0, ni.nbf, t.kk);
-        // up to KEB blocks of 16 entries per walk over t, so that each G
-        // operand load feeds KEB accumulations
-        for (int e0 = eb; e0 < ee; e0 += 16 * KEB) {
-            const double *Lr[KEB];
-            bool evj[KEB];
-            #pragma unroll
-            for (int j = 0; j < KEB; j++) {
-                const int e = e0 + 16 * j + (lane & 15);
-                evj[j] = e < ee;
-                Lr[j] = L + (long long)(evj[j] ? nent[e].x : 0) * t.Lld;
+        for (int u = 0; u < 2; u++) xc[u] = ge[ga + 8 * s + 4 * u + kl];
+    };
+    auto ket_load = [&]() {   // rows of t past the last repeat it (their G is stored as zero), as do n (not used)
+        const O to = (O)min(kt + l16, kk - 1) * Rcs, no = (O)func(min(kn + l16, ni.nbf - 1)) * 8;
+        #pragma unroll
+        for (int u = 0; u < 2; u++) {
+            oc[u] = make_int2(xc[u].x, xc[u].y);
+            oa[u][0] = kload(R, (O)max(xc[u].x, 0) * Rrs + to);
+            oa[u][1] = kload(R, (O)max(xc[u].y, 0) * Rrs + to);
+            od[u] = kload(D, (O)xc[u].z * Dld + no);
+        }
+        ks = ks + 1 < gs ? ks + 1 : 0;
+        if (ks == 0) {
+            kt = kt + 16 < kk ? kt + 16 : 0;
+            if (kt == 0) kn += 16;
+        }
+        ket_index(ks);
+    };
+    if (gs > 0) { ket_index(0); ket_load(); }
+    // ---- bra stream: blocks of the wave's list of the step, t0, step
+    const int *bp = bptr + ni.b_ptr + split * nstep * 8 + w;
+    int bb = bp[0], be = bp[1], bi = bb, bt = 0, bs = 0;   // position of the rows loaded next
+    int2 xr;                       // rows loaded next (row, local m | local n << 24),
+    int xt, om;                    // their t; local m and n of the operands in flight
+    double ol[4];
+    auto bra_index = [&]() { xr = brow[(long long)bi * 16 + l16]; xt = bt; };
+    auto bra_load = [&]() {
+        kload4(L, (O)xr.x * Lld + (O)(xt + 4 * kl) * 8, ol);
+        om = xr.y;
+        bi++;
+        if (bi == be) {
+            bt += 16;
+            if (bt >= kk) {
+                bt = 0;
+                bs = min(bs + 1, nstep - 1);
+                bb = bp[8 * bs];
+                be = bp[8 * bs + 1];
             }
-            const int nblk = min(KEB, (ee - e0 + 15) / 16);   // blocks with entries (wave-uniform)
-            d4 acc[KEB][2];
-            #pragma unroll
-            for (int j = 0; j < KEB; j++) acc[j][0] = acc[j][1] = d4{0.0, 0.0, 0.0, 0.0};
-            for (int t0 = 0; t0 < t.kk; t0 += 16) {
-                double b[2][4];
+            bi = bb;
+        }
+        bra_index();
+    };
+    bra_index();
+    bra_load();
+
+    for (int st = 0; st < nstep; st++) {
+        const int b0 = bp[8 * st], b1 = bp[8 * st + 1];
+        for (int t0 = 0; t0 < kk; t0 += 16) {
+            d4 acc[2];
+            acc[0] = acc[1] = d4{0.0, 0.0, 0.0, 0.0};
+            for (int s = 0; s < gs; s++) {
+                double a[2][2], b[2][2];
                 #pragma unroll
-                for (int h = 0; h < 2; h++)
-                    #pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int tt = t0 + 4 * u + kl;
-                        b[h][u] = (qv[h] && tt < t.kk) ? Gn[h][(size_t)tt * 8] : 0.0;
-                    }
-                #pragma unroll
-                for (int j = 0; j < KEB; j++) {
-                    if (j >= nblk) break;
-                    double a[4];
-                    #pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int tt = t0 + 4 * u + kl;
-                        a[u] = (evj[j] && tt < t.kk) ? Lr[j][tt] : 0.0;
-                    }
-                    #pragma unroll
-                    for (int u = 0; u < 4; u++)
-                        #pragma unroll
-                        for (int h = 0; h < 2; h++) acc[j][h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[h][u], acc[j][h], 0, 0, 0);
+                for (int u = 0; u < 2; u++) {
+                    a[u][0] = oa[u][0];
+                    a[u][1] = oa[u][1];
+                    b[u][0] = oc[u].x >= 0 ? od[u] : 0.0;
+                    b[u][1] = oc[u].y >= 0 ? od[u] : 0.0;
                 }
+                ket_load();
+                #pragma unroll
+                for (int u = 0; u < 2; u++)
+                    #pragma unroll
+                    for (int j = 0; j < 2; j++) acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][j], b[u][j], acc[j], 0, 0, 0);
             }
             #pragma unroll
-            for (int j = 0; j < KEB; j++) {
-                if (j >= nblk) break;
+            for (int r = 0; r < 4; r++) {
+                const int tl = kl + 4 * r;
+                const bool tv = t0 + tl < kk;   // zero past the last t: what the bra's loads find there does not count
+                *reinterpret_cast<double2 *>(Gt + l16 * KGN + tl * 16 + 2 * w) = make_double2(tv ? acc[0][r] : 0.0, tv ? acc[1][r] : 0.0);
+            }
+            __syncthreads();
+            // MFMA u takes the inner indices t = 4 k + u
+            for (int b = b0; b < b1; b++) {
+                double a[4];
+                #pragma unroll
+                for (int u = 0; u < 4; u++) a[u] = ol[u];
+                const int mn = om;
+                bra_load();
+                const double *g = Gt + (__builtin_amdgcn_readfirstlane(mn) >> 24) * KGN + kl * 64 + l16;
+                d4 x = d4{0.0, 0.0, 0.0, 0.0};
+                #pragma unroll
+                for (int u = 0; u < 4; u++) x = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], g[16 * u], x, 0, 0, 0);
                 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const int er = e0 + 16 * j + kl + 4 * r;
-                    if (er < ee) {
-                        const int mrow = nent[er].y - ml0;
-                        #pragma unroll
-                        for (int h = 0; h < 2; h++)
-                            if (qv[h]) atomicAdd(&Kb[mrow * 32 + 16 * h + (lane & 15)], acc[j][h][r]);
-                    }
+                    const int m = __shfl(mn, kl + 4 * r) & KMNONE;   // lane e of the wave holds entry e's
+                    if (m != KMNONE) atomicAdd(&Kb[(m - ml0) * KQ + l16], x[r]);
                 }
             }
+            __syncthreads();
         }
     }
-    __syncthreads();
-    double *Kout = t.diag ? Kd : K1;
-    const int mlN = min(ni.ssz, ni.nbf - ml0);
-    for (int i = threadIdx.x; i < mlN * 32; i += KWG) {
-        const int qq = ql0 + (i & 31);
+    double *Kout = KA + (size_t)nbf * nbf * (2 * (blockIdx.x % nacc) + (t.diag ? 1 : 0));
+    for (int i = threadIdx.x; i < mlN * KQ; i += KBWG) {
+        const int qq = q0 + (i & (KQ - 1));
         const double v = Kb[i];
         if (qq < nj.nbf && v != 0.0)
-            unsafeAtomicAdd(Kout + (size_t)bfidx[ni.bf_off + ml0 + (i >> 5)] * nbf + bfidx[nj.bf_off + qq], v);
+            unsafeAtomicAdd(Kout + (size_t)func(ml0 + i / KQ) * nbf + bfidx[nj.bf_off + qq], v);
     }
 }
 
 // Dense core with identity bases: K[m][q] += sum_{(r,n)} sum_{(c,p)} C[r][c] D[n][p].
+// One wave per (m, q), its lanes over the (row, column) entry pairs: a
+// thread per (m, q) walked up to a thousand dependent gathers (C30H62: 890 us
+// for 1 MFLOP).
 __global__ __launch_bounds__(KWG) void kx_direct(const KTask *__restrict__ tasks, const KTerm *__restrict__ terms,
                                                   const KNode *__restrict__ nodes, const int *__restrict__ bfidx,
                                                   const int *__restrict__ qptr, const int2 *__restrict__ qent,
                                                   const int *__restrict__ mptr, const int2 *__restrict__ ment,
                                                   const double *__restrict__ CB, const double *__restrict__ D,
-                                                  double *__restrict__ K1, double *__restrict__ Kd, int nbf) {
+                                                  double *__restrict__ KA, int nbf) {
     const KTask tk = tasks[blockIdx.x];
     const KTerm t = terms[tk.term];
     const KNode ni = nodes[t.ni], nj = nodes[t.nj];
-    const int e = tk.e0 + threadIdx.x;
-    if (e >= ni.nbf * nj.nbf) return;
+    const int e = tk.e0 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (e >= ni.nbf * nj.nbf) return;   // whole wave
     const int ml = e / nj.nbf, ql = e - ml * nj.nbf;
     const double *C = CB + t.Loff;
+    const int q0 = qptr[nj.q_ptr + ql], nq = qptr[nj.q_ptr + ql + 1] - q0;
+    const int r0 = mptr[ni.m_ptr + ml], nr = mptr[ni.m_ptr + ml + 1] - r0;
     double acc = 0.0;
-    const int q0 = qptr[nj.q_ptr + ql], q1 = qptr[nj.q_ptr + ql + 1];
-    for (int j = mptr[ni.m_ptr + ml]; j < mptr[ni.m_ptr + ml + 1]; j++) {
-        const int2 rn = ment[j];
-        const double *Cr = C + (long long)rn.x * t.Lld;
-        const double *Dn = D + (size_t)bfidx[ni.bf_off + rn.y] * nbf;
-        double s = 0.0;
-        for (int i = q0; i < q1; i++) {
-            const int2 cp = qent[i];
-            s = fma(Cr[cp.x], Dn[cp.y], s);
-        }
-        acc += s;
+    for (long long k = lane; k < (long long)nr * nq; k += 64) {
+        const int j = (int)(k / nq), i = (int)(k - (long long)j * nq);
+        const int2 rn = ment[r0 + j], cp = qent[q0 + i];
+        acc = fma(C[(long long)rn.x * t.Lld + cp.x], D[(size_t)bfidx[ni.bf_off + rn.y] * nbf + cp.y], acc);
     }
+    for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d, 64);
     const int m = bfidx[ni.bf_off + ml], q = bfidx[nj.bf_off + ql];
-    unsafeAtomicAdd((t.diag ? Kd : K1) + (size_t)m * nbf + q, acc);
+    if (lane == 0) unsafeAtomicAdd(KA + (t.diag ? (size_t)nbf * nbf : 0) + (size_t)m * nbf + q, acc);
 }
 
 // Grouped FP64 GEMM on MFMA: a 64 x 64 output tile per workgroup, wave w owns
@@ -422,14 +395,28 @@ __global__ void kx_zero(double *__restrict__ p, size_t n) {
     for (; i < n; i += s) p[i] = 0.0;
 }
 
-// K = K1 + K1^T + K_diag
-__global__ void kx_final(const double *__restrict__ K1, const double *__restrict__ Kd, double *__restrict__ K, int nbf) {
+// K = K1 + K1^T + K_diag, each summed over its nacc copies in order; 32 x 32
+// tiles, K1^T through LDS.
+__global__ __launch_bounds__(256) void kx_final(const double *__restrict__ KA, int nacc, double *__restrict__ K, int nbf) {
+    __shared__ double tr[32][33];
     const size_t n2 = (size_t)nbf * nbf;
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t s = (size_t)gridDim.x * blockDim.x;
-    for (; i < n2; i += s) {
-        const size_t r = i / nbf, c = i - r * nbf;
-        K[i] = K1[i] + K1[c * nbf + r] + Kd[i];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32;
+    for (int k = ty; k < 32; k += 8) {   // the transposed tile: rows c0.., columns r0..
+        const int r = c0 + k, c = r0 + tx;
+        double s = 0.0;
+        if (r < nbf && c < nbf)
+            for (int a = 0; a < nacc; a++) s += KA[2 * n2 * a + (size_t)r * nbf + c];
+        tr[k][tx] = s;
+    }
+    __syncthreads();
+    for (int k = ty; k < 32; k += 8) {
+        const int r = r0 + k, c = c0 + tx;
+        if (r >= nbf || c >= nbf) continue;
+        const size_t i = (size_t)r * nbf + c;
+        double s1 = 0.0, sd = 0.0;
+        for (int a = 0; a < nacc; a++) { s1 += KA[2 * n2 * a + i]; sd += KA[2 * n2 * a + n2 + i]; }
+        K[i] = (s1 + tr[tx][k]) + sd;
     }
 }
 
@@ -441,43 +428,41 @@ struct KPlan {
     std::vector<KTerm> terms;
     std::vector<KGemm> gemms;
     std::vector<KNode> nodes;
-    std::vector<int> bfidx, qptr, mptr, nspl;
-    std::vector<int2> qent, ment, nent;
-    std::vector<KTask> ket, bra, direct;
+    std::vector<int> bfidx, qptr, mptr, bptr, gptr;
+    // bra blocks: 16 (row r, local m | local n within the step << 24) each, the
+    // last row repeated with m = KMNONE past a block's entries
+    std::vector<int2> qent, ment, brow;
+    std::vector<int4> ge;   // ket entries: columns c of the two q (-1: none), p
+    std::vector<KTask> block, direct;
     std::vector<KGemmTask> gtasks;
     long long nSC = 0;      // L / R products (computed once)
-    long long nG = 0;       // G scratch of the largest chunk of terms
-    std::vector<int> ket_chunk, bra_chunk;   // first ket / bra task of every chunk, and the end
+    int nacc = 1;           // copies of the K accumulators
+    int mmax = 1, nmax = 1; // most functions m of a split, and of a node
+    bool wide = false;      // 64-bit offsets (kx_block)
     double flops = 0;
 };
 
-// Default bound of the G scratch of one chunk (bytes): the terms run in
-// chunks whose G fits it, each chunk's ket then its bra; with two or more
-// chunks, chunk c + 1's ket runs beside chunk c's bra on a second stream, in
-// a second region (the scratch is twice the bound).  Measured K per build
-// against the bound (unbounded / 4 / 2 / 1 GiB / 256 MiB): C30H62 12.2 /
-// 12.7 / 13.1 / 13.9 / 22.2 ms with 16.0 / 10.3 / 6.0 / 3.9 / 2.3 GB
-// resident; (H2O)64 75.7 ms unbounded (76 GB), 80.1 ms at 4 and at 1 GiB
-// (16.0 and 9.6 GB).  On one stream the chunks cost more (C30H62 16.7 ms at
-// 1 GiB): a launch of a small chunk has too few tasks to fill the GPU.
-static const double KG_BUDGET_DEFAULT = 2.0 * 1024.0 * 1024.0 * 1024.0;
+// Default bound of the K accumulators (bytes): workgroups add into one of
+// several copies of (K1, K_diag), up to KACC_MAX as the bound allows, so that
+// the atomics of the eight XCDs meet less on one address; kx_final adds the
+// copies.  C30H62 4.6 MB, (H2O)64 20 MB per matrix.
+static const double KACC_BUDGET_DEFAULT = 2.0 * 1024.0 * 1024.0 * 1024.0;
+static const int KACC_MAX = 4;
 
 struct KState {
     KPlan P;
     bool ready = false;
-    double g_budget = KG_BUDGET_DEFAULT;   // bytes of the G scratch (H2ERI_set_exchange_scratch)
-    double *PB = nullptr, *CB = nullptr, *SC = nullptr, *K1 = nullptr, *Kd = nullptr, *D = nullptr, *K = nullptr;
-    double *GS = nullptr;   // G of two chunks of terms (chunk c in region c % 2)
-    hipStream_t side = nullptr;                        // odd chunks, beside the caller's stream
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    double budget = KACC_BUDGET_DEFAULT;   // bytes of the accumulators (H2ERI_set_exchange_scratch)
+    double *PB = nullptr, *CB = nullptr, *SC = nullptr, *KA = nullptr, *D = nullptr, *K = nullptr;
     double *Ds = nullptr;   // the density after screening (the kernels' D)
     int *sbf = nullptr;     // shell_bf_sidx
     KTerm *terms = nullptr;
     KGemm *gemms = nullptr;
     KNode *nodes = nullptr;
-    int *bfidx = nullptr, *qptr = nullptr, *mptr = nullptr, *nspl = nullptr;
-    int2 *qent = nullptr, *ment = nullptr, *nent = nullptr;
-    KTask *ket = nullptr, *bra = nullptr, *direct = nullptr;
+    int *bfidx = nullptr, *qptr = nullptr, *mptr = nullptr, *bptr = nullptr, *gptr = nullptr;
+    int2 *qent = nullptr, *ment = nullptr, *brow = nullptr;
+    int4 *ge = nullptr;
+    KTask *block = nullptr, *direct = nullptr;
     KGemmTask *gtasks = nullptr;
     size_t resident = 0;
 };
@@ -487,15 +472,12 @@ static void kfree(void *&p) {
 }
 
 static void kstate_release(KState *k) {
-    void **ps[] = {(void **)&k->PB, (void **)&k->CB, (void **)&k->SC, (void **)&k->GS, (void **)&k->K1, (void **)&k->Kd, (void **)&k->D,
+    void **ps[] = {(void **)&k->PB, (void **)&k->CB, (void **)&k->SC, (void **)&k->KA, (void **)&k->D,
                    (void **)&k->K, (void **)&k->terms, (void **)&k->gemms, (void **)&k->nodes, (void **)&k->bfidx,
-                   (void **)&k->qptr, (void **)&k->mptr, (void **)&k->qent, (void **)&k->ment, (void **)&k->nspl,
-                   (void **)&k->nent, (void **)&k->ket,
-                   (void **)&k->bra, (void **)&k->direct, (void **)&k->gtasks, (void **)&k->Ds, (void **)&k->sbf};
+                   (void **)&k->qptr, (void **)&k->mptr, (void **)&k->qent, (void **)&k->ment, (void **)&k->bptr,
+                   (void **)&k->brow, (void **)&k->gptr, (void **)&k->ge,
+                   (void **)&k->block, (void **)&k->direct, (void **)&k->gtasks, (void **)&k->Ds, (void **)&k->sbf};
     for (void **p : ps) kfree(*p);
-    if (k->side) { (void)hipStreamDestroy(k->side); k->side = nullptr; }
-    if (k->ev_fork) { (void)hipEventDestroy(k->ev_fork); k->ev_fork = nullptr; }
-    if (k->ev_join) { (void)hipEventDestroy(k->ev_join); k->ev_join = nullptr; }
     k->ready = false;
     k->P = KPlan();
 }
@@ -503,14 +485,13 @@ static void kstate_release(KState *k) {
 struct KBuilder {
     H2ERI_p h;
     KPlan &P;
-    double g_budget;                 // bytes of G per chunk of terms
-    std::vector<long long> gsize;    // G doubles of every term (0: direct)
+    double budget;                   // bytes of the K accumulators
     std::vector<int> ra, rb;
     std::vector<char> sw;
     std::vector<long long> pb_off;   // expanded basis of each tree node in PB (-1: none)
     std::vector<int> node_list;      // tree node -> KNode id (-1: not built)
 
-    KBuilder(H2ERI_p h_, KPlan &p_, double g_budget_) : h(h_), P(p_), g_budget(g_budget_) {}
+    KBuilder(H2ERI_p h_, KPlan &p_, double budget_) : h(h_), P(p_), budget(budget_) {}
 
     int rank_of(int n) const { return h->U[n] ? h->U[n]->ncol : 0; }
     int rows_of(int n) const { return h->mat_cluster[2 * n + 1] - h->mat_cluster[2 * n] + 1; }
@@ -607,24 +588,56 @@ struct KBuilder {
         kn.m_ptr = (int)P.mptr.size();
         for (int i = 0; i < nb; i++) { P.mptr.push_back((int)P.ment.size()); P.ment.insert(P.ment.end(), bym[i].begin(), bym[i].end()); }
         P.mptr.push_back((int)P.ment.size());
-        // byN: for each local n the (row, local m) entries, sorted by m, with the
-        // first entry of every split of ssz functions m (at most KSPLIT, the
-        // node's functions in even parts so that no split task is a sliver)
+        // pairs of q: their entries merged on p, padded with empty entries to
+        // whole eights
+        kn.g_ptr = (int)P.gptr.size();
+        for (int g = 0; g < nb; g += 2) {
+            P.gptr.push_back((int)P.ge.size());
+            std::map<int, int2> at;
+            for (int j = 0; j < 2 && g + j < nb; j++)
+                for (const int2 &e : byq[g + j]) {
+                    int2 &c = at.emplace(e.y, make_int2(-1, -1)).first->second;
+                    (j == 0 ? c.x : c.y) = e.x;
+                }
+            for (const auto &e : at) P.ge.push_back(make_int4(e.second.x, e.second.y, e.first, 0));
+            for (size_t k = at.size(); k & 7; k++) P.ge.push_back(make_int4(-1, -1, 0, 0));
+        }
+        P.gptr.push_back((int)P.ge.size());
+        // bra: for each local n the (row, local m) entries, sorted by m; per
+        // split of ssz functions m (at most KM, even parts so that no split is
+        // a sliver) and step of 16 n, blocks of up to 16 entries dealt to the
+        // eight waves in turn (a wave without one gets an empty block)
         std::vector<std::vector<int2>> byn(nb);
         for (int ml = 0; ml < nb; ml++)
             for (const int2 &e : bym[ml]) byn[e.y].push_back(make_int2(e.x, ml));
-        kn.nsplit = (nb + KSPLIT - 1) / KSPLIT;
-        kn.ssz = kn.nsplit > 0 ? (nb + kn.nsplit - 1) / kn.nsplit : KSPLIT;
-        kn.s_ptr = (int)P.nspl.size();
-        for (int nl = 0; nl < nb; nl++) {
-            const int base = (int)P.nent.size();
-            int k = 0;
-            for (int sp = 0; sp <= kn.nsplit; sp++) {
-                while (k < (int)byn[nl].size() && byn[nl][k].y < sp * kn.ssz) k++;
-                P.nspl.push_back(base + k);
+        kn.nsplit = (nb + KM - 1) / KM;
+        kn.ssz = kn.nsplit > 0 ? (nb + kn.nsplit - 1) / kn.nsplit : KM;
+        kn.b_ptr = (int)P.bptr.size();
+        for (int sp = 0; sp < kn.nsplit; sp++)
+            for (int n0 = 0; n0 < nb; n0 += 16) {
+                struct Blk { int nl, e0, cnt; };
+                std::vector<Blk> wv[8];
+                int turn = 0;
+                for (int nl = n0; nl < std::min(n0 + 16, nb); nl++) {
+                    int a = 0, b = 0;
+                    while (a < (int)byn[nl].size() && byn[nl][a].y < sp * kn.ssz) a++;
+                    for (b = a; b < (int)byn[nl].size() && byn[nl][b].y < (sp + 1) * kn.ssz;) b++;
+                    for (int e = a; e < b; e += 16)
+                        wv[turn++ & 7].push_back(Blk{nl, e, std::min(16, b - e)});
+                }
+                for (int w = 0; w < 8; w++) {
+                    P.bptr.push_back((int)P.brow.size() / 16);
+                    if (wv[w].empty()) wv[w].push_back(Blk{n0, 0, 0});
+                    for (const Blk &k : wv[w])
+                        for (int e = 0; e < 16; e++) {
+                            const int2 a = k.cnt ? byn[k.nl][k.e0 + std::min(e, k.cnt - 1)] : make_int2(0, 0);
+                            P.brow.push_back(make_int2(a.x, (e < k.cnt ? a.y : KMNONE) | (k.nl - n0) << 24));
+                        }
+                }
             }
-            P.nent.insert(P.nent.end(), byn[nl].begin(), byn[nl].end());
-        }
+        P.bptr.push_back((int)P.brow.size() / 16);
+        P.mmax = std::max(P.mmax, kn.ssz);
+        P.nmax = std::max(P.nmax, nb);
         P.nodes.push_back(kn);
         node_list[node] = (int)P.nodes.size() - 1;
         return node_list[node];
@@ -704,7 +717,6 @@ struct KBuilder {
             if (bas1) { t.Rsrc = KS_SC; t.Roff = gemm(pb_off[n1], k1, m1, k1, c.VT, k, k); t.Rrs = k; t.Rcs = 1; }
             else { t.Rsrc = KS_CB; t.Roff = c.VT; t.Rrs = k; t.Rcs = 1; }
         }
-        t.Goff = -1;   // placed when the terms are cut into chunks
         P.terms.push_back(t);
     }
 
@@ -727,37 +739,32 @@ struct KBuilder {
         for (int g = 0; g < (int)P.gemms.size(); g++)
             for (int r0 = 0; r0 < P.gemms[g].m; r0 += 64)
                 for (int c0 = 0; c0 < P.gemms[g].n; c0 += 64) P.gtasks.push_back(KGemmTask{g, r0, c0, 0});
-        // chunks of consecutive terms whose G fits the budget (a larger term
-        // alone); G offsets restart in every chunk
-        const long long budget = std::max(1LL, (long long)(g_budget / 8.0));
-        long long used = 0;
-        bool open = false;
+        // block tasks: 16 functions q by a split of the functions m, the terms
+        // with the most work first (a workgroup's time goes with the steps of
+        // n, t and entries)
+        std::vector<std::pair<double, int>> order;
         for (int ti = 0; ti < (int)P.terms.size(); ti++) {
-            KTerm &t = P.terms[ti];
+            const KTerm &t = P.terms[ti];
             const KNode &ni = P.nodes[t.ni], &nj = P.nodes[t.nj];
             if (t.direct) {
                 const long long ne = (long long)ni.nbf * nj.nbf;
-                for (long long e0 = 0; e0 < ne; e0 += KWG) P.direct.push_back(KTask{ti, (int)e0, 0, 0});
+                for (long long e0 = 0; e0 < ne; e0 += KWG / 64) P.direct.push_back(KTask{ti, (int)e0, 0, 0});
                 continue;
             }
-            const long long gs = ((long long)t.kk * ni.nbf * gld(nj.nbf) + 31) & ~31LL;
-            if (!open || (used > 0 && used + gs > budget)) {
-                P.ket_chunk.push_back((int)P.ket.size());
-                P.bra_chunk.push_back((int)P.bra.size());
-                used = 0;
-                open = true;
-            }
-            t.Goff = used;
-            used += gs;
-            P.nG = std::max(P.nG, used);
-            for (int t0 = 0; t0 < t.kk; t0 += 16)
-                for (int nl0 = 0; nl0 < ni.nbf; nl0 += 64)
-                    for (int ql0 = 0; ql0 < nj.nbf; ql0 += KQC) P.ket.push_back(KTask{ti, nl0, t0, ql0});
-            for (int ql0 = 0; ql0 < nj.nbf; ql0 += 32)
-                for (int sp = 0; sp < ni.nsplit; sp++) P.bra.push_back(KTask{ti, ql0, sp, 0});
+            const double reach = std::max({(double)t.m1 * t.Rrs + (double)t.kk * t.Rcs, (double)t.m0 * t.Lld + t.kk + KPAD,
+                                           (double)h->num_bf * h->num_bf});
+            if (reach * 8.0 >= 4294967296.0 || ni.nbf > 4096) P.wide = true;
+            const double steps = (double)((ni.nbf + 15) / 16) * ((t.kk + 15) / 16);
+            order.push_back({steps * (4.0 + (double)t.m1 / nj.nbf + (double)t.m0 / ni.nbf), ti});
         }
-        P.ket_chunk.push_back((int)P.ket.size());
-        P.bra_chunk.push_back((int)P.bra.size());
+        std::stable_sort(order.begin(), order.end(), [](const std::pair<double, int> &a, const std::pair<double, int> &b) { return a.first > b.first; });
+        for (const auto &o : order) {
+            const KNode &ni = P.nodes[P.terms[o.second].ni], &nj = P.nodes[P.terms[o.second].nj];
+            for (int ql0 = 0; ql0 < nj.nbf; ql0 += KQ)
+                for (int sp = 0; sp < ni.nsplit; sp++) P.block.push_back(KTask{o.second, ql0, sp, 0});
+        }
+        const double acc = 16.0 * (double)h->num_bf * h->num_bf;   // bytes of one (K1, K_diag)
+        P.nacc = std::max(1, (int)std::min((double)KACC_MAX, budget / acc));
         return validate();
     }
 
@@ -774,7 +781,7 @@ struct KBuilder {
         }
         for (const KNode &n : P.nodes) {
             bool ok = n.bf_off >= 0 && n.bf_off + n.nbf <= (long long)P.bfidx.size() && n.q_ptr + n.nbf < (long long)P.qptr.size() &&
-                      n.m_ptr + n.nbf < (long long)P.mptr.size();
+                      n.m_ptr + n.nbf < (long long)P.mptr.size() && n.g_ptr + (n.nbf + 1) / 2 < (long long)P.gptr.size();
             for (int i = 0; ok && i < n.nbf; i++) ok = P.bfidx[n.bf_off + i] >= 0 && P.bfidx[n.bf_off + i] < nbf;
             if (!ok) { set_error(ERR_ARG, "exchange plan check failed: node lists"); return false; }
         }
@@ -784,49 +791,48 @@ struct KBuilder {
             // entries: columns < m1, p < nbf; rows < m0, local n < |B(i)|
             for (int j = P.qptr[nj.q_ptr]; ok && j < P.qptr[nj.q_ptr + nj.nbf]; j++)
                 ok = P.qent[j].x >= 0 && P.qent[j].x < t.m1 && P.qent[j].y >= 0 && P.qent[j].y < nbf;
+            const int ng = (nj.nbf + 1) / 2;
+            for (int g = 0; ok && g < ng; g++) {
+                const int ga = P.gptr[nj.g_ptr + g], gb = P.gptr[nj.g_ptr + g + 1];
+                ok = ga >= 0 && ga <= gb && gb <= (int)P.ge.size() && (gb - ga) % 8 == 0;
+                for (int j = ga; ok && j < gb; j++) {
+                    ok = P.ge[j].z >= 0 && P.ge[j].z < nbf && P.ge[j].x < t.m1 && P.ge[j].y < t.m1;
+                }
+            }
             for (int j = P.mptr[ni.m_ptr]; ok && j < P.mptr[ni.m_ptr + ni.nbf]; j++)
                 ok = P.ment[j].x >= 0 && P.ment[j].x < t.m0 && P.ment[j].y >= 0 && P.ment[j].y < ni.nbf;
-            // byN splits: increasing, inside nent, entries of a split within its m range
-            const int ns1 = ni.nsplit + 1;
-            // (the splits cover every local m: nsplit * ssz >= nbf)
-            ok = ok && ni.nsplit >= 1 && ni.ssz >= 1 && ni.ssz <= KSPLIT && (long long)ni.nsplit * ni.ssz >= ni.nbf &&
-                 ni.s_ptr >= 0 && ni.s_ptr + (long long)ni.nbf * ns1 <= (long long)P.nspl.size();
-            for (int nl = 0; ok && nl < ni.nbf; nl++)
-                for (int sp = 0; ok && sp < ni.nsplit; sp++) {
-                    const int eb = P.nspl[ni.s_ptr + nl * ns1 + sp], ee = P.nspl[ni.s_ptr + nl * ns1 + sp + 1];
-                    ok = eb >= 0 && eb <= ee && ee <= (int)P.nent.size();
-                    for (int e = eb; ok && e < ee; e++)
-                        ok = P.nent[e].x >= 0 && P.nent[e].x < t.m0 && P.nent[e].y >= sp * ni.ssz &&
-                             P.nent[e].y < std::min((sp + 1) * ni.ssz, ni.nbf);
+            // bra blocks: at least one per step and wave, rows below m0, m within
+            // the split (the splits cover every local m)
+            const int nst = (ni.nbf + 15) / 16;
+            ok = ok && ni.nsplit >= 1 && ni.ssz >= 1 && ni.ssz <= KM && (long long)ni.nsplit * ni.ssz >= ni.nbf && ni.b_ptr >= 0 &&
+                 ni.b_ptr + (long long)ni.nsplit * nst * 8 < (long long)P.bptr.size() && ni.nbf < KMNONE;
+            for (int k = 0; ok && k < ni.nsplit * nst * 8; k++) {
+                const int sp = k / (nst * 8);
+                const int b0 = P.bptr[ni.b_ptr + k], b1 = P.bptr[ni.b_ptr + k + 1];
+                ok = b0 >= 0 && b0 < b1 && b1 <= (int)(P.brow.size() / 16);
+                for (int e = 16 * b0; ok && e < 16 * b1; e++) {
+                    const int m = P.brow[e].y & KMNONE, nl = P.brow[e].y >> 24;
+                    ok = P.brow[e].x >= 0 && P.brow[e].x < t.m0 && nl >= 0 && nl < 16 && nl == P.brow[e & ~15].y >> 24 &&
+                         (m == KMNONE || (m >= sp * ni.ssz && m < std::min((sp + 1) * ni.ssz, ni.nbf)));
                 }
+            }
             ok = ok && t.Loff >= 0 && t.Loff + (long long)(t.m0 - 1) * t.Lld + t.kk <= size_of(t.Lsrc);
             if (!t.direct) {
                 const long long last = t.Roff + (long long)(t.m1 - 1) * t.Rrs + (long long)(t.kk - 1) * t.Rcs;
-                ok = ok && t.Roff >= 0 && last < size_of(t.Rsrc) && t.Goff >= 0 &&
-                     t.Goff % 4 == 0 && t.Goff + (long long)t.kk * ni.nbf * gld(nj.nbf) <= P.nG;
+                ok = ok && t.Roff >= 0 && last < size_of(t.Rsrc);
             }
             if (!ok) { set_error(ERR_ARG, "exchange plan check failed: term"); return false; }
         }
-        // chunks: the task ranges cover both lists in order, and all tasks of
-        // a term fall in one chunk (the chunks share one G region)
-        const size_t nc = P.ket_chunk.size();
-        bool ok = nc >= 1 && P.bra_chunk.size() == nc && P.ket_chunk.front() == 0 && P.bra_chunk.front() == 0 &&
-                  P.ket_chunk.back() == (int)P.ket.size() && P.bra_chunk.back() == (int)P.bra.size();
-        std::vector<int> tchunk(P.terms.size(), -1);
-        for (size_t c = 0; ok && c + 1 < nc; c++) {
-            ok = P.ket_chunk[c] <= P.ket_chunk[c + 1] && P.bra_chunk[c] <= P.bra_chunk[c + 1];
-            for (int side = 0; ok && side < 2; side++) {
-                const std::vector<KTask> &L = side == 0 ? P.ket : P.bra;
-                const std::vector<int> &B = side == 0 ? P.ket_chunk : P.bra_chunk;
-                for (int i = B[c]; ok && i < B[c + 1]; i++) {
-                    const int ti = L[i].term;
-                    ok = ti >= 0 && ti < (int)P.terms.size() && !P.terms[ti].direct &&
-                         (tchunk[ti] < 0 || tchunk[ti] == (int)c);
-                    if (ok) tchunk[ti] = (int)c;
-                }
-            }
+        // block tasks: each within its term
+        bool ok = true;
+        for (size_t i = 0; ok && i < P.block.size(); i++) {
+            const KTask &k = P.block[i];
+            ok = k.term >= 0 && k.term < (int)P.terms.size() && !P.terms[k.term].direct;
+            if (!ok) break;
+            const KNode &ni = P.nodes[P.terms[k.term].ni], &nj = P.nodes[P.terms[k.term].nj];
+            ok = k.e0 >= 0 && k.e0 < nj.nbf && k.e0 % KQ == 0 && k.t0 >= 0 && k.t0 < ni.nsplit;
         }
-        if (!ok) { set_error(ERR_ARG, "exchange plan check failed: chunks"); return false; }
+        if (!ok) { set_error(ERR_ARG, "exchange plan check failed: tasks"); return false; }
         return true;
     }
 };
@@ -859,7 +865,7 @@ static bool k_upload(H2ERI_p h) {
     if (!h->thread_Kmat_workbuf) h->thread_Kmat_workbuf = (void **)new KState();
     KState *k = kstate(h);
     if (k->ready) return true;
-    const double budget = k->g_budget;
+    const double budget = k->budget;
     kstate_release(k);
     KBuilder b(h, k->P, budget);
     if (!b.build()) return false;
@@ -873,12 +879,12 @@ static bool k_upload(H2ERI_p h) {
         return true;
     };
     const size_t nn2 = (size_t)nbf * nbf;
-    if (!up((void **)&k->PB, P.PB.empty() ? nullptr : P.PB.data(), P.PB.size() * 8) ||
-        !up((void **)&k->CB, P.CB.empty() ? nullptr : P.CB.data(), P.CB.size() * 8) ||
-        !up((void **)&k->SC, nullptr, (size_t)P.nSC * 8) ||
-        !up((void **)&k->GS, nullptr, (size_t)P.nG * 8 * (P.ket_chunk.size() > 2 ? 2 : 1)) ||
-        !up((void **)&k->K1, nullptr, nn2 * 8) ||
-        !up((void **)&k->Kd, nullptr, nn2 * 8) || !up((void **)&k->D, nullptr, nn2 * 8) ||
+    // operand arrays end in KPAD zeros: the bra's loads of four t run past a row's end
+    k->P.PB.resize(P.PB.size() + KPAD, 0.0);
+    k->P.CB.resize(P.CB.size() + KPAD, 0.0);
+    if (!up((void **)&k->PB, P.PB.data(), P.PB.size() * 8) || !up((void **)&k->CB, P.CB.data(), P.CB.size() * 8) ||
+        !up((void **)&k->SC, nullptr, ((size_t)P.nSC + KPAD) * 8) ||
+        !up((void **)&k->KA, nullptr, nn2 * 16 * P.nacc) || !up((void **)&k->D, nullptr, nn2 * 8) ||
         !up((void **)&k->K, nullptr, nn2 * 8) || !up((void **)&k->Ds, nullptr, nn2 * 8) ||
         !up((void **)&k->sbf, h->shell_bf_sidx, (size_t)(h->nshell + 1) * 4) ||
         !up((void **)&k->terms, P.terms.empty() ? nullptr : P.terms.data(), P.terms.size() * sizeof(KTerm)) ||
@@ -886,20 +892,21 @@ static bool k_upload(H2ERI_p h) {
         !up((void **)&k->nodes, P.nodes.empty() ? nullptr : P.nodes.data(), P.nodes.size() * sizeof(KNode)) ||
         !up((void **)&k->bfidx, P.bfidx.data(), P.bfidx.size() * 4) || !up((void **)&k->qptr, P.qptr.data(), P.qptr.size() * 4) ||
         !up((void **)&k->mptr, P.mptr.data(), P.mptr.size() * 4) ||
-        !up((void **)&k->nspl, P.nspl.data(), P.nspl.size() * 4) ||
-        !up((void **)&k->nent, P.nent.empty() ? nullptr : P.nent.data(), P.nent.size() * sizeof(int2)) ||
+        !up((void **)&k->bptr, P.bptr.data(), P.bptr.size() * 4) ||
+        !up((void **)&k->brow, P.brow.empty() ? nullptr : P.brow.data(), P.brow.size() * sizeof(int2)) ||
         !up((void **)&k->qent, P.qent.empty() ? nullptr : P.qent.data(), P.qent.size() * sizeof(int2)) ||
         !up((void **)&k->ment, P.ment.empty() ? nullptr : P.ment.data(), P.ment.size() * sizeof(int2)) ||
-        !up((void **)&k->ket, P.ket.empty() ? nullptr : P.ket.data(), P.ket.size() * sizeof(KTask)) ||
-        !up((void **)&k->bra, P.bra.empty() ? nullptr : P.bra.data(), P.bra.size() * sizeof(KTask)) ||
+        !up((void **)&k->gptr, P.gptr.data(), P.gptr.size() * 4) ||
+        !up((void **)&k->ge, P.ge.empty() ? nullptr : P.ge.data(), P.ge.size() * sizeof(int4)) ||
+        !up((void **)&k->block, P.block.empty() ? nullptr : P.block.data(), P.block.size() * sizeof(KTask)) ||
         !up((void **)&k->direct, P.direct.empty() ? nullptr : P.direct.data(), P.direct.size() * sizeof(KTask)) ||
         !up((void **)&k->gtasks, P.gtasks.empty() ? nullptr : P.gtasks.data(), P.gtasks.size() * sizeof(KGemmTask)))
         return false;
-    if (P.ket_chunk.size() > 2) {   // two or more chunks: odd ones run on a second stream
-        KHIP(hipStreamCreateWithFlags(&k->side, hipStreamNonBlocking));
-        KHIP(hipEventCreateWithFlags(&k->ev_fork, hipEventDisableTiming));
-        KHIP(hipEventCreateWithFlags(&k->ev_join, hipEventDisableTiming));
-    }
+    const int lds = (KGT + P.mmax * KQ) * 8 + (P.wide ? 0 : P.nmax * 4);   // G tile, K block, functions
+    for (const void *f : {reinterpret_cast<const void *>(&kx_block<unsigned>), reinterpret_cast<const void *>(&kx_block<unsigned long long>)})
+        KHIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    // (zeros also between the products, whose rows end where the next begins)
+    KHIP(hipMemset(k->SC, 0, ((size_t)P.nSC + KPAD) * 8));
     // L / R products do not depend on D: computed once at upload
     if (!P.gtasks.empty()) {
         hipLaunchKernelGGL(kx_gemm, dim3((unsigned)P.gtasks.size()), dim3(KWG), 0, 0, k->gtasks, k->gemms, k->PB, k->CB, k->SC);
@@ -920,40 +927,21 @@ static bool k_run(H2ERI_p h, const double *D_dev, double *K_dev, hipStream_t s) 
     const long long nblk = (long long)h->nshell * h->nshell;
     hipLaunchKernelGGL(kx_dlist, dim3((unsigned)((nblk + 255) / 256)), dim3(256), 0, s, k->sbf, h->nshell, D_dev, k->Ds, nbf);
     D_dev = k->Ds;
-    hipLaunchKernelGGL(kx_zero, dim3(zb), dim3(256), 0, s, k->K1, nn2);
-    hipLaunchKernelGGL(kx_zero, dim3(zb), dim3(256), 0, s, k->Kd, nn2);
+    hipLaunchKernelGGL(kx_zero, dim3(zb), dim3(256), 0, s, k->KA, nn2 * 2 * P.nacc);
     KHIP(hipGetLastError());
-    // every chunk of terms: its ket writes G, its bra reads it back.  Chunk c
-    // uses G region c % 2 on stream c % 2 (the caller's, or the second stream
-    // forked from it after the zeroing), so chunk c + 1's ket runs beside
-    // chunk c's bra and a region is reused only after its previous bra; both
-    // streams add into K1 / Kd with atomics and join before kx_final.
-    const int nchunk = (int)P.ket_chunk.size() - 1;
-    const bool two = nchunk > 1;
-    if (two) {
-        KHIP(hipEventRecord(k->ev_fork, s));
-        KHIP(hipStreamWaitEvent(k->side, k->ev_fork, 0));
-    }
+    // the blocks add into the accumulators with atomics; the K block's LDS is
+    // that of the largest split
+    if (!P.block.empty())
+        hipLaunchKernelGGL(P.wide ? kx_block<unsigned long long> : kx_block<unsigned>, dim3((unsigned)P.block.size()), dim3(KBWG),
+                           (size_t)(KGT + P.mmax * KQ) * 8 + (size_t)(P.wide ? 0 : P.nmax * 4), s, k->block, k->terms,
+                           k->nodes, k->bfidx, k->gptr, k->ge, k->bptr, k->brow, k->PB, k->CB, k->SC, D_dev, k->KA,
+                           P.nacc, nbf);
     if (!P.direct.empty())
         hipLaunchKernelGGL(kx_direct, dim3((unsigned)P.direct.size()), dim3(KWG), 0, s, k->direct, k->terms, k->nodes,
-                           k->bfidx, k->qptr, k->qent, k->mptr, k->ment, k->CB, D_dev, k->K1, k->Kd, nbf);
-    for (int c = 0; c < nchunk; c++) {
-        hipStream_t q = (two && (c & 1)) ? k->side : s;
-        double *G = k->GS + (two && (c & 1) ? P.nG : 0);
-        const int kb = P.ket_chunk[c], ke = P.ket_chunk[c + 1], bb = P.bra_chunk[c], be = P.bra_chunk[c + 1];
-        if (ke > kb)
-            hipLaunchKernelGGL(kx_ket, dim3((unsigned)(ke - kb)), dim3(KWG), 0, q, k->ket + kb, k->terms, k->nodes,
-                               k->bfidx, k->qptr, k->qent, k->PB, k->CB, k->SC, G, D_dev, nbf);
-        if (be > bb)
-            hipLaunchKernelGGL(kx_bra, dim3((unsigned)(be - bb)), dim3(KWG), 0, q, k->bra + bb, k->terms, k->nodes,
-                               k->bfidx, k->nspl, k->nent, k->PB, k->CB, k->SC, G, k->K1, k->Kd, nbf);
-    }
+                           k->bfidx, k->qptr, k->qent, k->mptr, k->ment, k->CB, D_dev, k->KA, nbf);
     KHIP(hipGetLastError());
-    if (two) {
-        KHIP(hipEventRecord(k->ev_join, k->side));
-        KHIP(hipStreamWaitEvent(s, k->ev_join, 0));
-    }
-    hipLaunchKernelGGL(kx_final, dim3(zb), dim3(256), 0, s, k->K1, k->Kd, K_dev, nbf);
+    const unsigned nt = (unsigned)(nbf + 31) / 32;
+    hipLaunchKernelGGL(kx_final, dim3(nt, nt), dim3(256), 0, s, k->KA, P.nacc, K_dev, nbf);
     KHIP(hipGetLastError());
     return true;
 }
@@ -1037,16 +1025,17 @@ void H2ERI_exchange_workbuf_free(H2ERI_p h) {
 int H2ERI_exchange_plan_check(H2ERI_p h, double *out4) {
     if (!h || !h->U || !h->c_B_blks || !h->c_D_blks) { set_error(ERR_ARG, "exchange_plan_check: nothing built"); return -1; }
     KPlan P;
-    KBuilder b(h, P, kstate(h) ? kstate(h)->g_budget : KG_BUDGET_DEFAULT);
+    KBuilder b(h, P, kstate(h) ? kstate(h)->budget : KACC_BUDGET_DEFAULT);
     if (!b.build()) return -1;
     if (out4) {
         const double nn2 = (double)h->num_bf * h->num_bf;
         out4[0] = P.flops;
         out4[1] = (double)P.terms.size();
-        const double nG = (double)P.nG * (P.ket_chunk.size() > 2 ? 2 : 1);   // two regions with two or more chunks
-        out4[2] = 8.0 * ((double)P.PB.size() + (double)P.CB.size() + (double)P.nSC + nG + 5.0 * nn2) +
-                  4.0 * ((double)P.bfidx.size() + P.qptr.size() + P.mptr.size()) + 8.0 * ((double)P.qent.size() + P.ment.size());
-        out4[3] = (double)P.nSC + nG;
+        const double nacc = 2.0 * P.nacc * nn2;
+        out4[2] = 8.0 * ((double)P.PB.size() + (double)P.CB.size() + (double)P.nSC + nacc + 3.0 * nn2) +
+                  4.0 * ((double)P.bfidx.size() + P.qptr.size() + P.mptr.size() + P.gptr.size() + P.bptr.size()) +
+                  8.0 * ((double)P.qent.size() + P.ment.size() + P.brow.size()) + 16.0 * (double)P.ge.size();
+        out4[3] = (double)P.nSC + nacc;
     }
     return (int)P.terms.size();
 }
@@ -1059,21 +1048,20 @@ void H2ERI_exchange_stats(H2ERI_p h, double *out4) {
     out4[0] = k->P.flops;
     out4[1] = (double)k->P.terms.size();
     out4[2] = (double)k->resident;
-    out4[3] = (double)(k->P.nSC + k->P.nG * (k->P.ket_chunk.size() > 2 ? 2 : 1));
+    out4[3] = (double)k->P.nSC + 2.0 * k->P.nacc * (double)h->num_bf * h->num_bf;
 }
 
-// Bound of the exchange build's G scratch in bytes (additive, tuning): the
-// block terms run in chunks whose intermediate G fits it, each chunk's ket
-// then its bra, in one scratch region reused by every chunk.  Releases the
+// Bound of the exchange build's K accumulators in bytes (additive, tuning):
+// at least one copy of (K1, K_diag) whatever the bound.  Releases the
 // exchange plan (rebuilt by the next K build).
 void H2ERI_set_exchange_scratch(H2ERI_p h, const double bytes) {
     if (!h || !(bytes >= 1024.0)) { set_error(ERR_ARG, "H2ERI_set_exchange_scratch: at least 1024 bytes"); return; }
     if (!h->thread_Kmat_workbuf) h->thread_Kmat_workbuf = (void **)new KState();
     KState *k = kstate(h);
-    if (k->g_budget == bytes) return;
+    if (k->budget == bytes) return;
     device_release_graph_kind(h, 2);
     kstate_release(k);
-    k->g_budget = bytes;
+    k->budget = bytes;
 }
 
 }  // extern "C"
