@@ -1153,42 +1153,47 @@ __global__ void queue_reset_kernel(int *ctr, int nlist) {
     if (i < nlist) ctr[QC_LISTS + i] = 0;
 }
 
-// x[i] = c_i * D[g_i >> 1], c_i = 2 when the low bit is set
-// (src/H2ERI_build_Coulomb.c:26-62).
+// x_k[i] = c_i * D_k[g_i >> 1], c_i = 2 when the low bit is set
+// (src/H2ERI_build_Coulomb.c:26-62), for the nd densities of the call: the
+// map is read once per four densities.
 __global__ void uncontract_kernel(const int *__restrict__ gidx, const double *__restrict__ D, double *__restrict__ x,
-                                  int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        int g = gidx[i];
-        double v = D[g >> 1];
-        x[i] = (g & 1) ? 2.0 * v : v;
+                                  int n, long long nn, int nd) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int g = gidx[i];
+    const double c = (g & 1) ? 2.0 : 1.0;
+    #pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int k = 4 * blockIdx.y + u;
+        if (k < nd) x[(long long)k * n + i] = c * D[k * nn + (g >> 1)];
     }
 }
 
-// Jh[g_i >> 1] = s_i * y[i], s_i = 1/2 when the low bit is clear (M == N)
-// (src/H2ERI_build_Coulomb.c:90-116).  The map i -> g_i >> 1 is injective.
-__global__ void contract_scatter_kernel(const int *__restrict__ gidx, const double *__restrict__ y,
-                                        double *__restrict__ Jh, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        int g = gidx[i];
-        Jh[g >> 1] = (g & 1) ? y[i] : 0.5 * y[i];
-    }
-}
-
-// J = Jh + Jh^T through 32x32 LDS tiles (src/H2ERI_build_Coulomb.c:119-132).
-__global__ void symmetrize_kernel(const double *__restrict__ Jh, double *__restrict__ J, int n) {
-    __shared__ double tile[32][33];
-    const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 32 x 8 threads
-    for (int k = ty; k < 32; k += 8) {
-        int r = bx + k, c = by + tx;   // read the transposed tile
-        tile[k][tx] = (r < n && c < n) ? Jh[(size_t)r * n + c] : 0.0;
-    }
-    __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-        int r = by + k, c = bx + tx;
-        if (r < n && c < n) J[(size_t)r * n + c] = Jh[(size_t)r * n + c] + tile[tx][k];
+// J_k[e] from the pair rows of element e = (i, j) (src/H2ERI_build_Coulomb.c:
+// 90-132): with M != N the element's one row, stored for (i, j) and (j, i)
+// alike; with M == N half of the row of (i, j) plus half of that of (j, i);
+// zero where the pair was screened.  jmap[e] = row << 2 | flags (1: add the
+// transposed element's row, 2: halve both), or ~0; a shell pair stored in
+// both orders, which this library does not write, has flag 1 on both.
+// One pass that writes J once (its bound): clearing a half matrix, scattering
+// into it and adding its transpose were three launches and five times the
+// traffic (C100H202: 50 us per density, 0.8 ms per 16; now 12 and 170 us).
+__global__ void contract_kernel(const unsigned *__restrict__ jmap, const double *__restrict__ y, double *__restrict__ J,
+                                int nbf, long long n, int nd) {
+    const long long nn = (long long)nbf * nbf, e = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (e >= nn) return;
+    const unsigned m = jmap[e];
+    const bool none = m == ~0u, both = !none && (m & 1);
+    const unsigned m2 = both ? jmap[(e % nbf) * nbf + e / nbf] : 0;   // the transposed element's row
+    const double c = (m & 2) ? 0.5 : 1.0;
+    #pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int k = 4 * blockIdx.y + u;
+        if (k >= nd) break;
+        const double *yk = y + k * n;
+        double v = none ? 0.0 : c * yk[m >> 2];
+        if (both) v += c * yk[m2 >> 2];
+        J[k * nn + e] = v;
     }
 }
 
@@ -1209,9 +1214,7 @@ __global__ void transpose16_kernel(const double *__restrict__ X, long long ld, d
 }
 
 __global__ void zero_kernel(double *__restrict__ p, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) p[i] = 0.0;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1360,8 +1363,9 @@ struct DevState {
     DevPlan plans[NWIDTH];
     // Coulomb and host-pointer staging
     int *d_gidx = nullptr;
-    double *d_D = nullptr, *d_J = nullptr, *d_Jh = nullptr, *d_y = nullptr, *d_x = nullptr;
-    size_t d_io_len = 0;
+    unsigned *d_jmap = nullptr;
+    double *d_D = nullptr, *d_J = nullptr, *d_y = nullptr, *d_x = nullptr;
+    size_t d_io_len = 0, d_dj_len = 0;   // doubles of d_x / d_y, and of d_D / d_J
     hipStream_t side = nullptr;         // near-field stream (schedule 2)
     hipGraphExec_t graph = nullptr;     // captured hot-path sequence (H2ERI_graph_capture)
     int graph_kind = -1;                // its kind (0 matvec, 1 Coulomb, 2 exchange)
@@ -1380,7 +1384,7 @@ struct DevState {
     // buffers of the captured Coulomb graph: only H2ERI_graph_capture
     // allocates them and only release_graph frees them, so no eager call
     // that grows its own buffers can leave the graph pointing at freed memory
-    double *g_x = nullptr, *g_y = nullptr, *g_Jh = nullptr;
+    double *g_x = nullptr, *g_y = nullptr;
     // workspace of the pass being enqueued when it is not the plan's own
     // (the allocation-free entry point puts it in the file-scope scratch
     // array); null: the plan's Wv and counters
@@ -1428,17 +1432,16 @@ static void release_graph(DevState *d) {
     d->graph_kind = -1;
     free_dev((void *&)d->g_x);
     free_dev((void *&)d->g_y);
-    free_dev((void *&)d->g_Jh);
 }
 
 static void release_buffers(DevState *d) {
     release_graph(d);   // a graph refers to the buffers below
     release_plans(d);
-    void **ps[] = {(void **)&d->S64, (void **)&d->S32, (void **)&d->d_gidx, (void **)&d->d_D, (void **)&d->d_J,
-                   (void **)&d->d_Jh, (void **)&d->d_y, (void **)&d->d_x};
+    void **ps[] = {(void **)&d->S64, (void **)&d->S32, (void **)&d->d_gidx, (void **)&d->d_jmap, (void **)&d->d_D,
+                   (void **)&d->d_J, (void **)&d->d_y, (void **)&d->d_x};
     for (void **p : ps) free_dev(*p);
     jit_release(d->jit);
-    d->d_io_len = 0;
+    d->d_io_len = d->d_dj_len = 0;
     d->st = Storage();
     d->st_ready = false;
     d->resident_bytes = 0;
@@ -2321,6 +2324,16 @@ static bool upload_storage(H2ERI_p h) {
                 for (int k = 0; k < nrow; k++) g[xo + j * nrow + k] = (((scol + j) * nbf + srow + k) << 1) | two;
         }
         if (!alloc_copy((void **)&d->d_gidx, g.data(), (size_t)N * sizeof(int))) return false;
+        // the inverse, per element of J (N <= nbf^2 < 2^30)
+        std::vector<unsigned> jm((size_t)nbf * nbf, ~0u);
+        for (int i = 0; i < N; i++) jm[g[i] >> 1] = (unsigned)i << 2 | ((g[i] & 1) ? 0 : 3);
+        for (int i = 0; i < N; i++) {
+            if (!(g[i] & 1)) continue;
+            unsigned &t = jm[(size_t)((g[i] >> 1) % nbf) * nbf + (g[i] >> 1) / nbf];
+            if (t == ~0u) t = (unsigned)i << 2;
+            else if (t >> 2 != (unsigned)i) { t |= 1; jm[g[i] >> 1] |= 1; }
+        }
+        if (!alloc_copy((void **)&d->d_jmap, jm.data(), jm.size() * sizeof(unsigned))) return false;
     }
     d->st_ready = true;
     return true;
@@ -2638,28 +2651,26 @@ static bool matvec_host_impl(H2ERI_p h, int nvec, const double *x, double *y) {
 }
 
 // J_k = contract(A uncontract(D_k)) for ndens densities on the device, with
-// x and y in xb / yb (N * ndens doubles each) and the half matrix in Jh
-// (num_bf^2 doubles).
+// x and y in xb / yb (N * ndens doubles each).
 static bool coulomb_run(H2ERI_p h, int ndens, const double *D_dev, double *J_dev, hipStream_t s, double *xb,
-                        double *yb, double *Jh) {
+                        double *yb) {
     DevState *d = dstate(h);
     const int N = h->krnl_mat_size, nbf = h->num_bf;
-    const size_t nn = (size_t)nbf * nbf;
-    for (int k = 0; k < ndens; k++) {
-        hipLaunchKernelGGL(uncontract_kernel, dim3((N + 255) / 256), dim3(256), 0, s, d->d_gidx, D_dev + k * nn,
-                           xb + (size_t)k * N, N);
+    const long long nn = (long long)nbf * nbf;
+    const unsigned quads = (unsigned)(ndens + 3) / 4;
+    for (unsigned q = 0; q < quads; q += 65535) {   // grid.y holds 65,535
+        const unsigned ny = std::min(quads - q, 65535u);
+        const long long k = 4LL * q;
+        hipLaunchKernelGGL(uncontract_kernel, dim3((N + 255) / 256, ny), dim3(256), 0, s, d->d_gidx, D_dev + k * nn, xb + k * N, N,
+                           nn, ndens - (int)k);
         HIP_OK(hipGetLastError());
     }
     if (!matvec_multi_dev_impl(h, ndens, xb, yb, s)) return false;
-    for (int k = 0; k < ndens; k++) {
-        hipLaunchKernelGGL(zero_kernel, dim3((unsigned)std::min<size_t>((nn + 255) / 256, 4096)), dim3(256), 0, s,
-                           Jh, nn);
-        HIP_OK(hipGetLastError());
-        hipLaunchKernelGGL(contract_scatter_kernel, dim3((N + 255) / 256), dim3(256), 0, s, d->d_gidx,
-                           yb + (size_t)k * N, Jh, N);
-        HIP_OK(hipGetLastError());
-        dim3 grid((nbf + 31) / 32, (nbf + 31) / 32);
-        hipLaunchKernelGGL(symmetrize_kernel, grid, dim3(256), 0, s, Jh, J_dev + k * nn, nbf);
+    for (unsigned q = 0; q < quads; q += 65535) {
+        const unsigned ny = std::min(quads - q, 65535u);
+        const long long k = 4LL * q;
+        hipLaunchKernelGGL(contract_kernel, dim3((unsigned)((nn + 255) / 256), ny), dim3(256), 0, s, d->d_jmap, yb + k * N,
+                           J_dev + k * nn, nbf, (long long)N, ndens - (int)k);
         HIP_OK(hipGetLastError());
     }
     return true;
@@ -2670,10 +2681,8 @@ static bool coulomb_dev_impl(H2ERI_p h, int ndens, const double *D_dev, double *
     if (!upload_storage(h)) return false;
     DevState *d = dstate(h);
     if (!d->d_gidx) { set_error(ERR_ARG, "Coulomb build needs shell-pair metadata"); return false; }
-    const size_t nn = (size_t)h->num_bf * h->num_bf;
     if (!ensure_io(d, (size_t)h->krnl_mat_size * ndens)) return false;
-    if (!d->d_Jh) HIP_OK(hipMalloc(&d->d_Jh, sizeof(double) * nn));
-    return coulomb_run(h, ndens, D_dev, J_dev, s, d->d_x, d->d_y, d->d_Jh);
+    return coulomb_run(h, ndens, D_dev, J_dev, s, d->d_x, d->d_y);
 }
 
 // Reads and clears the error flag of every persistent plan's counters, after
@@ -2828,11 +2837,15 @@ void H2ERI_build_Coulomb_multi(H2ERI_p h, const int ndens, const double *den_mat
     DevState *d = dstate(h);
     HostTiming tm(d);
     const size_t nn = (size_t)h->num_bf * h->num_bf;
-    free_dev((void *&)d->d_D);
-    free_dev((void *&)d->d_J);
-    if (hipMalloc(&d->d_D, nn * 8 * ndens) != hipSuccess || hipMalloc(&d->d_J, nn * 8 * ndens) != hipSuccess) {
-        set_error(ERR_DEVICE, "H2ERI_build_Coulomb: device allocation of D/J failed");
-        return;
+    if (d->d_dj_len < nn * ndens) {   // kept for the next call: freeing waits for the device
+        free_dev((void *&)d->d_D);
+        free_dev((void *&)d->d_J);
+        d->d_dj_len = 0;
+        if (hipMalloc(&d->d_D, nn * 8 * ndens) != hipSuccess || hipMalloc(&d->d_J, nn * 8 * ndens) != hipSuccess) {
+            set_error(ERR_DEVICE, "H2ERI_build_Coulomb: device allocation of D/J failed");
+            return;
+        }
+        d->d_dj_len = nn * ndens;
     }
     if (hipMemcpy(d->d_D, den_mats, nn * 8 * ndens, hipMemcpyHostToDevice) != hipSuccess) { set_error(ERR_DEVICE, "copy D"); return; }
     if (!coulomb_dev_impl(h, ndens, d->d_D, d->d_J, nullptr)) return;
@@ -2888,11 +2901,10 @@ int H2ERI_graph_capture(H2ERI_p h, const int kind, const int n, const double *in
     if (!d->ev_join && hipEventCreateWithFlags(&d->ev_join, hipEventDisableTiming) != hipSuccess) { set_error(ERR_DEVICE, "event"); return -1; }
     release_graph(d);   // also frees the previous graph's buffers
     if (kind == 1) {
-        // the graph's own x, y and half-matrix buffers (nothing else resizes them)
+        // the graph's own x and y buffers (nothing else resizes them)
         if (!d->d_gidx) { set_error(ERR_ARG, "Coulomb build needs shell-pair metadata"); return -1; }
-        const size_t nx = (size_t)h->krnl_mat_size * n, nn = (size_t)h->num_bf * h->num_bf;
-        if (hipMalloc(&d->g_x, sizeof(double) * nx) != hipSuccess || hipMalloc(&d->g_y, sizeof(double) * nx) != hipSuccess ||
-            hipMalloc(&d->g_Jh, sizeof(double) * nn) != hipSuccess) {
+        const size_t nx = (size_t)h->krnl_mat_size * n;
+        if (hipMalloc(&d->g_x, sizeof(double) * nx) != hipSuccess || hipMalloc(&d->g_y, sizeof(double) * nx) != hipSuccess) {
             release_graph(d);
             set_error(ERR_DEVICE, "H2ERI_graph_capture: allocation failed");
             return -1;
@@ -2905,7 +2917,7 @@ int H2ERI_graph_capture(H2ERI_p h, const int kind, const int n, const double *in
     if (ok) {
         d->capturing = true;
         ok = kind == 0   ? matvec_multi_dev_impl(h, n, in_dev, out_dev, cs)
-             : kind == 1 ? coulomb_run(h, n, in_dev, out_dev, cs, d->g_x, d->g_y, d->g_Jh)
+             : kind == 1 ? coulomb_run(h, n, in_dev, out_dev, cs, d->g_x, d->g_y)
                          : exchange_enqueue(h, in_dev, out_dev, cs);
         d->capturing = false;
         const bool end_ok = hipStreamEndCapture(cs, &g) == hipSuccess;
