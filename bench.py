@@ -59,11 +59,11 @@ def log(*a):
 # timing helpers
 # ---------------------------------------------------------------------------
 def pass_widths(n):
-    """Vectors per pass of a batched call of n vectors (16, 8, 4, 2, 1 as the
-    library splits it)."""
+    """Widths of the passes of a batched call of n vectors (16 per pass, the
+    last vectors in the narrowest of 1, 2, 4, 8, 16 that holds them)."""
     out = []
     while n > 0:
-        w = 16 if n >= 16 else 8 if n >= 8 else 4 if n >= 4 else 2 if n >= 2 else 1
+        w = 16 if n > 8 else 8 if n > 4 else 4 if n > 2 else n
         out.append(w)
         n -= w
     return out

@@ -105,6 +105,14 @@ __device__ __forceinline__ RTask uniform(const RTask &a) {
     return t;
 }
 
+// The pass's external vectors: vector v at v * ld, n of them (the pass is NV
+// wide; the others read as zero and are not written).  ld < 0: an
+// element-major copy.
+struct ExtLd {
+    long long ld;
+    int n;
+};
+
 static const int WG = 256;       // threads per workgroup (4 waves)
 // Output elements per reduce task: 1024 / NV values fill the task's 256
 // threads four deep.  Both executors use the same chunks, so their plans and
@@ -159,13 +167,14 @@ __device__ __forceinline__ void wst(double *p, double v) {
 // threads take values q = tid, tid + WG, ... (contiguous in its
 // NV-interleaved layout), so every thread works for any NV, and each sums
 // the slots in list order with eight loads in flight.  From the external
-// input the threads take elements and read the NV vectors.
+// input the threads take elements and read the first ldx.n vectors (a pass
+// wider than the vectors left has zeros in the others).
 template <int NV, bool COH, int NT, int XS = NV>
 __device__ __forceinline__ void stage_vec(const int *__restrict__ vsrc, int b, int e, int off, int n,
-                                          const double *__restrict__ Wv, const double *__restrict__ X, long long ldx,
+                                          const double *__restrict__ Wv, const double *__restrict__ X, ExtLd ldx,
                                           double *dst, int tid) {
     const int s0 = vsrc[b];
-    if (s0 < 0 && ldx < 0) {   // the external input as an element-major copy (NV values per element)
+    if (s0 < 0 && ldx.ld < 0) {   // the external input as an element-major copy (NV values per element)
         const double *p = X + (long long)(-s0 - 1 + off) * NV;
         for (int q = tid; q < n * NV; q += NT) dst[XS == NV ? q : (q / NV) * XS + q % NV] = p[q];
         return;
@@ -174,7 +183,7 @@ __device__ __forceinline__ void stage_vec(const int *__restrict__ vsrc, int b, i
         const double *p = X + (long long)(-s0 - 1 + off);
         for (int i = tid; i < n; i += NT) {
             #pragma unroll
-            for (int v = 0; v < NV; v++) dst[i * XS + v] = p[(long long)v * ldx + i];
+            for (int v = 0; v < NV; v++) dst[i * XS + v] = NV == 1 || v < ldx.n ? p[v * ldx.ld + i] : 0.0;
         }
         return;
     }
@@ -397,7 +406,7 @@ template <typename T> struct Dot8 { static const int RC = 4, XS = 10, RW = 4; };
 
 template <typename T, int NV, bool COH, int NT = WG>
 __device__ void bgemv_tile_valu(const BTask &task, const T *__restrict__ S, const int *__restrict__ vsrc,
-                                double *__restrict__ Wv, const double *__restrict__ X, long long ldx, double *lds) {
+                                double *__restrict__ Wv, const double *__restrict__ X, ExtLd ldx, double *lds) {
     // At NV = 8 the descriptor stays as loaded: the register allocation of
     // the two tile paths together fits 128 VGPRs only that way (measured on
     // the compiler's output), and the path choice is made uniform below.
@@ -710,7 +719,7 @@ __device__ void mfma_tile16_2s(const BTask &t, const T *__restrict__ base, const
     const int Cp = (C + 15) & ~15, ng = Cp >> 4;   // groups of 16 columns, at most 4
     double *xin = lds;                                // Cp x 16, zero past C
     double *tr = lds + T16_MAXC * NV + 256 * w;       // this wave's 16 x 16 transposition tile
-    stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, -1, xin, tid);
+    stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, ExtLd{-1, 16}, xin, tid);
     for (int q = C * NV + tid; q < Cp * NV; q += WG) xin[q] = 0.0;
     __syncthreads();
     const In16 y = in16_make(vsrc, t.v1b, t.v1e, t.v1off);
@@ -785,11 +794,11 @@ __device__ void mfma_tile16(const BTask &task, const T *__restrict__ S, const in
     double *xin = lds;
     double *yin = lds + (st0 ? Cp * NV : 0);
     if (st0) {
-        stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, -1, xin, tid);
+        stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, ExtLd{-1, 16}, xin, tid);
         for (int q = C * NV + tid; q < Cp * NV; q += WG) xin[q] = 0.0;
     }
     if (do1) {
-        stage_vec<NV, COH, WG>(vsrc, t.v1b, t.v1e, t.v1off, R, Wv, Xt, -1, yin, tid);
+        stage_vec<NV, COH, WG>(vsrc, t.v1b, t.v1e, t.v1off, R, Wv, Xt, ExtLd{-1, 16}, yin, tid);
         for (int q = R * NV + tid; q < Rp * NV; q += WG) yin[q] = 0.0;
     }
     __syncthreads();
@@ -873,7 +882,7 @@ __device__ void mfma_tile16(const BTask &task, const T *__restrict__ S, const in
 // A tile task: the MFMA products at 16 vectors per pass, the VALU tile below.
 template <typename T, int NV, bool COH, int NT = WG>
 __device__ __forceinline__ void bgemv_tile(const BTask &task, const T *__restrict__ S, const int *__restrict__ vsrc,
-                                           double *__restrict__ Wv, const double *__restrict__ X, long long ldx,
+                                           double *__restrict__ Wv, const double *__restrict__ X, ExtLd ldx,
                                            double *lds) {
     if constexpr (NV == 16) {
         // X is the element-major copy of the input (the pass's first launch
@@ -891,7 +900,7 @@ __device__ __forceinline__ void bgemv_tile(const BTask &task, const T *__restric
 // as (g0 + g1) + (g2 + g3), or g0 + g1.
 template <int NV, bool COH>
 __device__ void reduce_task(const RTask &task, const int *__restrict__ src, double *__restrict__ Wv,
-                            double *__restrict__ Y, long long ldy, double *lds) {
+                            double *__restrict__ Y, ExtLd ldy, double *lds) {
     const RTask t = uniform(task);
     const int n = t.len * NV;
     const int K = n <= 64 ? 4 : (n <= 128 ? 2 : 1);
@@ -924,7 +933,7 @@ __device__ void reduce_task(const RTask &task, const int *__restrict__ src, doub
     auto put = [&](int q, double v) {
         if (t.flags & 1) {
             const int i = q / NV, w = q - i * NV;
-            Y[(long long)w * ldy + t.dst + i] = v;
+            if (NV == 1 || w < ldy.n) Y[w * ldy.ld + t.dst + i] = v;
         } else {
             wst<COH>(Wv + t.dst * NV + q, v);
         }
@@ -962,7 +971,7 @@ __device__ __forceinline__ void stage_task(int b, const BTask *__restrict__ t64,
                                            const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                            const double *__restrict__ S64, const float *__restrict__ S32,
                                            double *__restrict__ Wv, const double *__restrict__ X,
-                                           double *__restrict__ Y, long long ldx, double *lds) {
+                                           double *__restrict__ Y, ExtLd ldx, double *lds) {
     if (b < n64) {
         const BTask t = t64[b];
         bgemv_tile<double, NV, false>(t, S64, vsrc, Wv, X, ldx, lds);
@@ -995,7 +1004,7 @@ __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void stage_kernel(const B
                                                    int nw32, const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                                    const double *__restrict__ S64, const float *__restrict__ S32,
                                                    double *__restrict__ Wv, const double *__restrict__ X,
-                                                   double *__restrict__ Y, long long ldx) {
+                                                   double *__restrict__ Y, ExtLd ldx) {
     __shared__ double lds[LDS_DOUBLES];
     stage_task<NV>(blockIdx.x, t64, n64, t32, n32, rt, nr, w64, nw64, w32, nw32, vsrc, rsrc, S64, S32, Wv, X, Y, ldx,
                    lds);
@@ -1011,7 +1020,7 @@ __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void stage_loop_kernel(co
                                                         int nw32, const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                                         const double *__restrict__ S64, const float *__restrict__ S32,
                                                         double *__restrict__ Wv, const double *__restrict__ X,
-                                                        double *__restrict__ Y, long long ldx) {
+                                                        double *__restrict__ Y, ExtLd ldx) {
     __shared__ double lds[LDS_DOUBLES];
     const int total = n64 + n32 + nr + (nw64 + 3) / 4 + (nw32 + 3) / 4;
     for (int b = blockIdx.x; b < total; b += gridDim.x) {
@@ -1094,7 +1103,7 @@ __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void queue_kernel(const Q
                                                       const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                                       const double *__restrict__ S64, const float *__restrict__ S32,
                                                       double *__restrict__ Wv, const double *__restrict__ X,
-                                                      double *__restrict__ Y, long long ldx) {
+                                                      double *__restrict__ Y, ExtLd ldx) {
     __shared__ double lds[LDS_DOUBLES];
     __shared__ int s_next[2];
     if (threadIdx.x == 0) s_next[0] = __hip_atomic_fetch_add(ctr + QC_TICKET, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1118,9 +1127,9 @@ __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void queue_kernel(const Q
             __syncthreads();
             if constexpr (GROUP) {
                 const MolPtrs m = mols[q.pad_[0]];
-                if (q.kind == 0) bgemv_tile<double, NV, true>(m.t64[q.idx], m.S64, m.vsrc, m.Wv, m.X, m.ldx, lds);
-                else if (q.kind == 1) bgemv_tile<float, NV, true>(m.t32[q.idx], m.S32, m.vsrc, m.Wv, m.X, m.ldx, lds);
-                else reduce_task<NV, true>(m.rt[q.idx], m.rsrc, m.Wv, m.Y, m.ldx, lds);
+                if (q.kind == 0) bgemv_tile<double, NV, true>(m.t64[q.idx], m.S64, m.vsrc, m.Wv, m.X, ExtLd{m.ldx, 1}, lds);
+                else if (q.kind == 1) bgemv_tile<float, NV, true>(m.t32[q.idx], m.S32, m.vsrc, m.Wv, m.X, ExtLd{m.ldx, 1}, lds);
+                else reduce_task<NV, true>(m.rt[q.idx], m.rsrc, m.Wv, m.Y, ExtLd{m.ldx, 1}, lds);
             } else {
                 if (q.kind == 0) bgemv_tile<double, NV, true>(t64[q.idx], S64, vsrc, Wv, X, ldx, lds);
                 else if (q.kind == 1) bgemv_tile<float, NV, true>(t32[q.idx], S32, vsrc, Wv, X, ldx, lds);
@@ -1197,14 +1206,15 @@ __global__ void contract_kernel(const unsigned *__restrict__ jmap, const double 
     }
 }
 
-// Element-major copy of 16 vectors (Xt[i * 16 + v] = X[v * ld + i]), the
+// Element-major copy of 16 vectors (Xt[i * 16 + v] = X[v * ld + i], zero from
+// vector nv on), the
 // first launch of a 16-vector pass: both sides coalesced through a 16 x 256
 // LDS tile.
-__global__ void transpose16_kernel(const double *__restrict__ X, long long ld, double *__restrict__ Xt, int n) {
+__global__ void transpose16_kernel(const double *__restrict__ X, long long ld, int nv, double *__restrict__ Xt, int n) {
     __shared__ double tile[16][257];
     const int i0 = blockIdx.x * 256, tid = threadIdx.x;
     #pragma unroll
-    for (int v = 0; v < 16; v++) tile[v][tid] = i0 + tid < n ? X[(long long)v * ld + i0 + tid] : 0.0;
+    for (int v = 0; v < 16; v++) tile[v][tid] = v < nv && i0 + tid < n ? X[(long long)v * ld + i0 + tid] : 0.0;
     __syncthreads();
     #pragma unroll
     for (int k = 0; k < 16; k++) {
@@ -1340,8 +1350,15 @@ static const int NWIDTH = 5;   // batch widths: vectors per pass over the matrix
 static const int NV_VARIANTS[NWIDTH] = {1, 2, 4, 8, 16};
 static inline int nv_index(int nv) { return nv == 1 ? 0 : (nv == 2 ? 1 : (nv == 4 ? 2 : (nv == 8 ? 3 : 4))); }
 static inline bool nv_valid(int nv) { return nv == 1 || nv == 2 || nv == 4 || nv == 8 || nv == 16; }
-// widest pass for the vectors left: 16, 8, 4, 2 or 1
-static inline int nv_pass(int rem) { return rem >= 16 ? 16 : (rem >= 8 ? 8 : (rem >= 4 ? 4 : (rem >= 2 ? 2 : 1))); }
+// Pass for the vectors left: 16, and the narrowest that holds the last ones
+// (its spare vectors are zero).  One wider pass is faster than the narrower
+// ones that add up to it: a pass costs little more than its stream of the
+// matrix data.  Tuned passes of 1 / 2 / 4 / 8 / 16, ms: C30H62 FP32-stored 0.30
+// / 0.34 / 0.40 / 0.50 / 0.68, C100H202 1.51 / - / 2.02 / 2.73 / 3.39, (H2O)64
+// 0.73 / - / 1.08 / 1.80 / 2.38: 3 vectors as 4 take 0.40 in place of 0.63,
+// 5 as 8 0.50 (2.73, 1.80) in place of 0.70 (3.53, 1.81), 9 as 16 0.68
+// (3.39, 2.38) in place of 0.79 (4.24, 2.53).
+static inline int nv_pass(int rem) { return rem > 8 ? 16 : (rem > 4 ? 8 : (rem > 2 ? 4 : rem)); }
 
 // Tuning configuration of one batch width.
 struct Tune {
@@ -1361,6 +1378,7 @@ struct DevState {
     double *S64 = nullptr;
     float *S32 = nullptr;
     DevPlan plans[NWIDTH];
+    bool no_pad[NWIDTH] = {false, false, false, false, false};   // widths that did not fit a padded pass (pass_plan)
     // Coulomb and host-pointer staging
     int *d_gidx = nullptr;
     unsigned *d_jmap = nullptr;
@@ -2418,6 +2436,23 @@ static DevPlan *get_plan(H2ERI_p h, int nv) {
     return &dp;
 }
 
+// Plan of the next pass for `rem` vectors left (nv_pass); when a pass wider
+// than that cannot be planned or held (its workspace), the widest of at most
+// `rem` vectors, from then on.
+static DevPlan *pass_plan(H2ERI_p h, int rem) {
+    const int nv = nv_pass(rem), i = nv_index(nv);
+    const bool padded = nv > rem;
+    if (!padded || !dstate_get(h)->no_pad[i]) {
+        DevPlan *dp = get_plan(h, nv);
+        if (dp || !padded || h->BD_JIT || !dstate(h)->st_ready) return dp;
+        dstate(h)->no_pad[i] = true;
+        release_plan(dstate(h), i);
+        (void)hipGetLastError();
+        h2eri_clear_error();
+    }
+    return get_plan(h, nv / 2);
+}
+
 // Workgroups of one stage launch: a tile or reduce task each, four wave tiles each.
 static inline int stage_blocks(const Stage &st) {
     return st.t64_cnt + st.t32_cnt + st.r_cnt + (st.w64_cnt + 3) / 4 + (st.w32_cnt + 3) / 4;
@@ -2437,7 +2472,7 @@ static inline int launch_blocks(const Stage &st, const DevState *d, int nv) {
 }
 
 template <int NV>
-static void launch_stage(const Stage &st, const DevPlan &dp, DevState *d, const double *X, double *Y, long long ld,
+static void launch_stage(const Stage &st, const DevPlan &dp, DevState *d, const double *X, double *Y, ExtLd ld,
                          hipStream_t s) {
     const int nb = stage_blocks(st), grid = launch_blocks(st, d, NV);
     hipLaunchKernelGGL(grid < nb ? stage_loop_kernel<NV> : stage_kernel<NV>, dim3(grid), dim3(WG), 0, s,
@@ -2453,19 +2488,19 @@ static void collect_phase_ms(H2ERI_p h, DevState *d);
 static const int QUEUE_SPIN_LIMIT = 1 << 22;
 
 template <int NV>
-static void launch_queue(const DevPlan &dp, DevState *d, const double *X, double *Y, long long ld, hipStream_t s) {
+static void launch_queue(const DevPlan &dp, DevState *d, const double *X, double *Y, ExtLd ld, hipStream_t s) {
     hipLaunchKernelGGL((queue_kernel<NV, false>), dim3(dp.q_grid), dim3(WG), 0, s, dp.d_q, dp.q_n,
                        dp.d_need, pass_ctr(d, dp), d->spin_limit, (const MolPtrs *)nullptr, dp.d_t64, dp.d_t32, dp.d_rt,
                        dp.d_vsrc, dp.d_rsrc, d->S64, d->S32, pass_Wv(d, dp), NV == 16 ? dp.Xt : X, Y, ld);
 }
 
 // One pass of the persistent executor on stream s (reset + queue launch).
-static bool run_queue(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, double *Y, hipStream_t s) {
+static bool run_queue(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, double *Y, int n, hipStream_t s) {
     if (!dp.q_ready) { set_error(ERR_DEVICE, "persistent executor: queue not built"); return false; }
-    const long long ld = h->krnl_mat_size;
+    const ExtLd ld{h->krnl_mat_size, n};
     const bool tim = d->phase_timing && !d->capturing;
     if (dp.P.nv == 16) {
-        hipLaunchKernelGGL(transpose16_kernel, dim3((unsigned)((ld + 255) / 256)), dim3(256), 0, s, X, ld, dp.Xt, (int)ld);
+        hipLaunchKernelGGL(transpose16_kernel, dim3((unsigned)((ld.ld + 255) / 256)), dim3(256), 0, s, X, ld.ld, ld.n, dp.Xt, (int)ld.ld);
         HIP_OK(hipGetLastError());
     }
     hipLaunchKernelGGL(queue_reset_kernel, dim3((std::max(dp.q_nlist, QC_LISTS) + 255) / 256), dim3(256), 0, s,
@@ -2497,17 +2532,18 @@ static bool run_queue(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, doub
     return true;
 }
 
-// Enqueue one batched matvec of nv vectors: X (nv x N, vector-major) -> Y.
+// Enqueue one pass of the plan's width for n vectors (at most that many): X
+// (n x N, vector-major) -> Y.
 // In phase-timing mode an event pair brackets every launch.
-static bool run_matvec(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, double *Y, hipStream_t s) {
-    if (d->cfg[nv_index(dp.P.nv)].executor == 1) return run_queue(h, d, dp, X, Y, s);
+static bool run_matvec(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, double *Y, int n, hipStream_t s) {
+    if (d->cfg[nv_index(dp.P.nv)].executor == 1) return run_queue(h, d, dp, X, Y, n, s);
     const Plan &P = dp.P;
-    const long long ld = h->krnl_mat_size;
+    const ExtLd ld{h->krnl_mat_size, n};
     const bool tim = d->phase_timing && !d->capturing;
     bool has_side = false;
     for (const Stage &st : P.stages) has_side |= st.stream == 1;
     if (P.nv == 16) {   // element-major copy of the input, before the fork
-        hipLaunchKernelGGL(transpose16_kernel, dim3((unsigned)((ld + 255) / 256)), dim3(256), 0, s, X, ld, dp.Xt, (int)ld);
+        hipLaunchKernelGGL(transpose16_kernel, dim3((unsigned)((ld.ld + 255) / 256)), dim3(256), 0, s, X, ld.ld, ld.n, dp.Xt, (int)ld.ld);
         HIP_OK(hipGetLastError());
     }
     if (tim) {
@@ -2604,11 +2640,11 @@ static bool matvec_multi_dev_impl(H2ERI_p h, int nvec, const double *X, double *
     int done = 0;
     while (done < nvec) {
         const int rem = nvec - done;
-        const int nv = nv_pass(rem);
-        DevPlan *dp = get_plan(h, nv);
+        DevPlan *dp = pass_plan(h, rem);
         if (!dp) return false;
-        if (!run_matvec(h, dstate(h), *dp, X + done * N, Y + done * N, s)) return false;
-        done += nv;
+        const int n = std::min(dp->P.nv, rem);
+        if (!run_matvec(h, dstate(h), *dp, X + done * N, Y + done * N, n, s)) return false;
+        done += n;
     }
     return true;
 }
@@ -2790,7 +2826,7 @@ static bool matvec_noalloc_impl(H2ERI_p h, const double *X, double *Y, hipStream
     d->phase_timing = false;
     d->ws_Wv = (double *)((char *)base + ctr_bytes);
     d->ws_ctr = queue ? ctr : nullptr;
-    const bool ok = run_matvec(h, d, *dp, X, Y, s);
+    const bool ok = run_matvec(h, d, *dp, X, Y, 1, s);
     d->ws_Wv = nullptr;
     d->ws_ctr = nullptr;
     d->phase_timing = was_timing;
@@ -2891,9 +2927,9 @@ int H2ERI_graph_capture(H2ERI_p h, const int kind, const int n, const double *in
         if (!upload_storage(h)) return -1;
         for (int done = 0; done < n;) {
             const int rem = n - done;
-            const int nv = nv_pass(rem);
-            if (!get_plan(h, nv)) return -1;
-            done += nv;
+            const DevPlan *dp = pass_plan(h, rem);
+            if (!dp) return -1;
+            done += std::min(dp->P.nv, rem);
         }
     }
     if (!d->side && hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking) != hipSuccess) { set_error(ERR_DEVICE, "stream"); return -1; }
@@ -3316,7 +3352,7 @@ int H2ERI_group_matvec(void *group, void *stream) {
     hipLaunchKernelGGL((queue_kernel<1, true>), dim3(g->q_grid), dim3(WG), 0, s, g->d_q, g->q_n, g->d_need,
                        g->d_ctr, QUEUE_SPIN_LIMIT, g->d_mols, (const BTask *)nullptr, (const BTask *)nullptr,
                        (const RTask *)nullptr, (const int *)nullptr, (const int *)nullptr, (const double *)nullptr,
-                       (const float *)nullptr, (double *)nullptr, (const double *)nullptr, (double *)nullptr, 0LL);
+                       (const float *)nullptr, (double *)nullptr, (const double *)nullptr, (double *)nullptr, ExtLd{0, 1});
     if (hipGetLastError() != hipSuccess) { set_error(ERR_DEVICE, "H2ERI_group_matvec: launch failed"); return -1; }
     return 0;
 }
