@@ -43,6 +43,7 @@
 #include <cmath>
 #include <map>
 #include <numeric>
+#include <type_traits>
 
 #include "h2eri_internal.h"
 
@@ -72,7 +73,7 @@ struct KGemm {           // out (m x n, ld ldo) = A (m x k, PB, ld lda) * X (k x
 
 struct KTask {           // one workgroup: term and tile origin
     int term;
-    int e0;               // block: first local q; direct: first (m,q) index
+    int e0;               // block: first column slot; direct: first (m,q) index
     int t0;               // block: split of local m
     int pad_;
 };
@@ -85,7 +86,8 @@ struct KNode {           // per row/column range: basis-function set and the ori
     int bf_off, nbf;      // B(node) = bfidx[bf_off .. bf_off + nbf)
     int q_ptr;            // byQ CSR rows: qptr[q_ptr .. q_ptr + nbf]   entries (column c, p)
     int m_ptr;            // byM CSR rows: mptr[m_ptr .. m_ptr + nbf]   entries (row r, local n)
-    int g_ptr;            // merged lists of pairs of q: gptr[g_ptr + g]   entries (p, columns c of the two q)
+    int g_ptr;            // merged lists of pairs of column slots: gptr[g_ptr + g]   entries (p, columns c of the two)
+    int c_off, ngrp;      // functions q of the 2 ngrp column slots: bfidx[c_off + slot] (-1: none)
     int b_ptr;            // bra block lists: bptr[b_ptr + ((split * steps of 16 n) + step) * 8 + wave], and the next one
     int nsplit;           // splits of the functions m
     int ssz;              // functions m per split: the nbf functions in nsplit = ceil(nbf / KM) even parts
@@ -105,7 +107,8 @@ __device__ inline int xcd_task(int bid, int n, int C) {
     return full * 8 * C + x * q + min(x, r) + k2;
 }
 static const int KRUN = 8;      // consecutive tasks per XCD
-static const int KQ = 16;       // column functions q per task (eight pairs)
+static const int KQ = 16;       // column slots q per task (eight pairs)
+static const int KNQ = 8;      // fours of a pair's entries whose R operands stay in registers
 static const int KGN = 258;     // doubles per function n of the G tile (16 t x 16 q, and two that shift the LDS banks)
 static const int KGT = 16 * KGN;
 static const int KBWG = 512;    // threads of a block task (8 waves)
@@ -132,36 +135,52 @@ __device__ __forceinline__ double kload(const double *p, O byte) {
     return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + byte);
 }
 
-// One block term's share of K: a workgroup takes 16 functions q of the column
-// node and a split of the row node's functions m, and walks the functions n
-// of the row node in steps of 16 and the inner index t in steps of 16:
+// f(integral constant of min(n, KNQ)): straight-line code for every length
+template <typename F>
+__device__ __forceinline__ void kfours(int n, F f) {
+    switch (min(n, KNQ)) {
+    case 0: break;
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 3: f(std::integral_constant<int, 3>()); break;
+    case 4: f(std::integral_constant<int, 4>()); break;
+    case 5: f(std::integral_constant<int, 5>()); break;
+    case 6: f(std::integral_constant<int, 6>()); break;
+    case 7: f(std::integral_constant<int, 7>()); break;
+    default: f(std::integral_constant<int, KNQ>()); break;
+    }
+}
+
+// One block term's share of K: a workgroup takes 16 column slots q of the
+// column node and a split of the row node's functions m, and walks the inner
+// index t in steps of 16 and, for each, the functions n of the row node in
+// steps of 16:
 //   ket  G[n][t][q] = sum over the entries (c, p) of q of R[c][t] D[p][n]
-//        into LDS: wave w the functions q = 2w, 2w+1, one MFMA tile
-//        (16 t x 16 n) each.  The two entry lists are merged on p, so that
-//        one D operand serves both; an entry a function does not have meets
-//        a zero D operand.  D is symmetric (the entry point's contract):
-//        D[p][n] lets the 16 lanes of an entry read along a row.
+//        into LDS: a wave takes two q, one MFMA tile (16 t x 16 n) each.  The
+//        two entry lists are merged on p, so that one D operand serves both;
+//        an entry a function does not have meets a zero D operand.  D is
+//        symmetric (the entry point's contract): D[p][n] lets the 16 lanes of
+//        an entry read along a row.  The R operands of the first 32 entries
+//        stay in registers over all steps of n: a step loads one D operand
+//        per two MFMAs.  Entries past them are read again in every step.
 //   bra  K[m][q] += sum over the entries (r, m) of n of L[r][t] G[n][t][q]:
 //        the entries of every n in blocks of 16 rows, dealt to the waves in
 //        turn; a block's tile is added into the K block in LDS with FP64 LDS
-//        atomics (tiles of different n may share an m).
+//        atomics (tiles of different n may share an m).  Its operands are one
+//        stream over all steps: the next block's rows are in flight across
+//        the barriers, and their indices one further ahead.
 // At the end the K block is added into K with FP64 global atomics.
 //
-// Both loops take their operands as one stream over all steps: while eight
-// ket entries (or one bra block) are consumed the next ones are in flight,
-// across the barriers too, and their indices one further ahead.  16 waves
-// per CU (128 VGPRs, two workgroups by LDS) cover the rest.
-//
-// What bounds it: the operand loads' address path (busy for over half of the
-// time) and FP64 MFMA issue (64 cycles each, 37%); half of the MFMA work is
-// padding, since entries per function come in eights (ket) and sixteens
-// (bra).  G stays in LDS: as two kernels with G in HBM (14.7 GB for C30H62,
-// 73 GB for (H2O)64, written and read back) a build was bound by that round
-// trip and by twice the ket's D loads.  K per build, two kernels / this one:
-// C10H22 2.77 / 1.51 ms, C30H62 13.1 / 7.4 ms, (H2O)64 76.6 / 41.5 ms.  Tried:
-// four waves of four q each with everything prefetched into registers (2
-// waves per SIMD, waits that the compiler cannot order: C30H62 20.5 ms); a
-// third workgroup per CU for nodes of at most 152 functions (no gain).
+// What bounds it: the bra (C30H62: ket steps alone 2.3 ms, bra alone 3.7 ms of
+// the build's 5.6; the LDS atomics and the shuffles of their rows are 0.7 ms
+// of the bra, and a wave waits at the two barriers of a step for the one with
+// most blocks) and FP64 MFMA issue (64 cycles each); about half of the MFMA
+// work is padding, since the entries of an n come in sixteens.  A second block
+// in flight per wave: no gain (5.64 / 5.72 ms).  16 waves per CU (128 VGPRs,
+// two workgroups by LDS): 40 entries in registers spill (5.86 ms).
+// K per build with G in HBM between two kernels / G in LDS, R read in every
+// step of n and neighbouring functions paired in order / this one:
+// C10H22 2.77 / 1.52 / 1.17 ms, C30H62 13.1 / 7.37 / 5.64 ms.
 template <typename O>
 __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ tasks, const KTerm *__restrict__ terms,
                                                     const KNode *__restrict__ nodes, const int *__restrict__ bfidx,
@@ -190,38 +209,34 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
     const int kk = t.kk, nstep = (ni.nbf + 15) >> 4;
     const O Rrs = (O)t.Rrs * 8, Rcs = (O)t.Rcs * 8, Lld = (O)t.Lld * 8, Dld = (O)nbf * 8;
 
-    // ---- ket stream: entries in eights, s within the list, t0 and n0 of the tile
-    const int grp = (q0 >> 1) + w;
-    const bool gok = 2 * grp < nj.nbf;
-    const int ga = gok ? gptr[nj.g_ptr + grp] : 0, gs = gok ? (gptr[nj.g_ptr + grp + 1] - ga) >> 3 : 0;
-    int ks = 0, kt = 0, kn = 0;    // position of the operands loaded next
-    int4 xc[2];                    // the entries loaded next (columns of the two q, p)
-    int2 oc[2];                    // columns of the operands in flight
-    double oa[2][2], od[2];
-    auto ket_index = [&](int s) {
-        #pragma unroll
-        for (int u = 0; u < 2; u++) xc[u] = ge[ga + 8 * s + 4 * u + kl];
+    // ---- ket: entries in fours; pairs come longest first, and the waves of
+    // one SIMD (w, w + 4) take a long and a short one
+    const int grp = (q0 >> 1) + (w < 4 ? w : 11 - w), qw = 2 * (grp - (q0 >> 1));
+    const bool gok = grp < nj.ngrp;
+    const int ga = gok ? gptr[nj.g_ptr + grp] : 0, gs = gok ? (gptr[nj.g_ptr + grp + 1] - ga) >> 2 : 0;
+    double ra[KNQ][2];      // R operands of the entries of the two q
+    O pd[KNQ];              // rows of D
+    unsigned has0 = 0, has1 = 0;   // entry i of the lane's exists for the first / second q
+    auto ket_rows = [&](int t0) {   // rows of t past the last repeat it (their G is stored as zero)
+        const O to = (O)min(t0 + l16, kk - 1) * Rcs;
+        kfours(gs, [&](auto N) {
+            int4 x[N];
+            #pragma unroll
+            for (int i = 0; i < N; i++) x[i] = ge[ga + 4 * i + kl];
+            has0 = has1 = 0;
+            #pragma unroll
+            for (int i = 0; i < N; i++) {
+                ra[i][0] = kload(R, (O)max(x[i].x, 0) * Rrs + to);
+                ra[i][1] = kload(R, (O)max(x[i].y, 0) * Rrs + to);
+                pd[i] = (O)x[i].z * Dld;
+                has0 |= x[i].x >= 0 ? 1u << i : 0u;
+                has1 |= x[i].y >= 0 ? 1u << i : 0u;
+            }
+        });
     };
-    auto ket_load = [&]() {   // rows of t past the last repeat it (their G is stored as zero), as do n (not used)
-        const O to = (O)min(kt + l16, kk - 1) * Rcs, no = (O)func(min(kn + l16, ni.nbf - 1)) * 8;
-        #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            oc[u] = make_int2(xc[u].x, xc[u].y);
-            oa[u][0] = kload(R, (O)max(xc[u].x, 0) * Rrs + to);
-            oa[u][1] = kload(R, (O)max(xc[u].y, 0) * Rrs + to);
-            od[u] = kload(D, (O)xc[u].z * Dld + no);
-        }
-        ks = ks + 1 < gs ? ks + 1 : 0;
-        if (ks == 0) {
-            kt = kt + 16 < kk ? kt + 16 : 0;
-            if (kt == 0) kn += 16;
-        }
-        ket_index(ks);
-    };
-    if (gs > 0) { ket_index(0); ket_load(); }
     // ---- bra stream: blocks of the wave's list of the step, t0, step
     const int *bp = bptr + ni.b_ptr + split * nstep * 8 + w;
-    int bb = bp[0], be = bp[1], bi = bb, bt = 0, bs = 0;   // position of the rows loaded next
+    int bi = bp[0], be = bp[1], bt = 0, bs = 0;   // position of the rows loaded next
     int2 xr;                       // rows loaded next (row, local m | local n << 24),
     int xt, om;                    // their t; local m and n of the operands in flight
     double ol[4];
@@ -231,45 +246,61 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
         om = xr.y;
         bi++;
         if (bi == be) {
-            bt += 16;
-            if (bt >= kk) {
-                bt = 0;
-                bs = min(bs + 1, nstep - 1);
-                bb = bp[8 * bs];
-                be = bp[8 * bs + 1];
+            if (++bs == nstep) {
+                bs = 0;
+                bt = bt + 16 < kk ? bt + 16 : 0;
             }
-            bi = bb;
+            bi = bp[8 * bs];
+            be = bp[8 * bs + 1];
         }
         bra_index();
     };
     bra_index();
     bra_load();
 
-    for (int st = 0; st < nstep; st++) {
-        const int b0 = bp[8 * st], b1 = bp[8 * st + 1];
-        for (int t0 = 0; t0 < kk; t0 += 16) {
+    for (int t0 = 0; t0 < kk; t0 += 16) {
+        ket_rows(t0);
+        for (int st = 0; st < nstep; st++) {
+            const int b0 = bp[8 * st], b1 = bp[8 * st + 1];
+            const O no = (O)func(min(16 * st + l16, ni.nbf - 1)) * 8;   // n past the last repeat it (not used)
             d4 acc[2];
             acc[0] = acc[1] = d4{0.0, 0.0, 0.0, 0.0};
-            for (int s = 0; s < gs; s++) {
-                double a[2][2], b[2][2];
+            kfours(gs, [&](auto N) {
+                double d[N];
                 #pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    a[u][0] = oa[u][0];
-                    a[u][1] = oa[u][1];
-                    b[u][0] = oc[u].x >= 0 ? od[u] : 0.0;
-                    b[u][1] = oc[u].y >= 0 ? od[u] : 0.0;
+                for (int i = 0; i < N; i++) d[i] = kload(D, pd[i] + no);
+                #pragma unroll
+                for (int i = 0; i < N; i++) {
+                    acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[i][0], has0 >> i & 1 ? d[i] : 0.0, acc[0], 0, 0, 0);
+                    acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[i][1], has1 >> i & 1 ? d[i] : 0.0, acc[1], 0, 0, 0);
                 }
-                ket_load();
+            });
+            for (int s = KNQ; s < gs; s += 4) {   // entries past the registers
+                const O to = (O)min(t0 + l16, kk - 1) * Rcs;
+                int4 x[4];
+                double a[4][2], d[4];
                 #pragma unroll
-                for (int u = 0; u < 2; u++)
-                    #pragma unroll
-                    for (int j = 0; j < 2; j++) acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][j], b[u][j], acc[j], 0, 0, 0);
+                for (int u = 0; u < 4; u++) {
+                    x[u] = ge[ga + 4 * min(s + u, gs - 1) + kl];
+                    if (s + u >= gs) x[u].x = x[u].y = -1;
+                }
+                #pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    a[u][0] = kload(R, (O)max(x[u].x, 0) * Rrs + to);
+                    a[u][1] = kload(R, (O)max(x[u].y, 0) * Rrs + to);
+                    d[u] = kload(D, (O)x[u].z * Dld + no);
+                }
+                #pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][0], x[u].x >= 0 ? d[u] : 0.0, acc[0], 0, 0, 0);
+                    acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][1], x[u].y >= 0 ? d[u] : 0.0, acc[1], 0, 0, 0);
+                }
             }
             #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int tl = kl + 4 * r;
                 const bool tv = t0 + tl < kk;   // zero past the last t: what the bra's loads find there does not count
-                *reinterpret_cast<double2 *>(Gt + l16 * KGN + tl * 16 + 2 * w) = make_double2(tv ? acc[0][r] : 0.0, tv ? acc[1][r] : 0.0);
+                *reinterpret_cast<double2 *>(Gt + l16 * KGN + tl * 16 + qw) = make_double2(tv ? acc[0][r] : 0.0, tv ? acc[1][r] : 0.0);
             }
             __syncthreads();
             // MFMA u takes the inner indices t = 4 k + u
@@ -294,10 +325,10 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
     }
     double *Kout = KA + (size_t)nbf * nbf * (2 * (blockIdx.x % nacc) + (t.diag ? 1 : 0));
     for (int i = threadIdx.x; i < mlN * KQ; i += KBWG) {
-        const int qq = q0 + (i & (KQ - 1));
+        const int slot = q0 + (i & (KQ - 1));
+        const int q = slot < 2 * nj.ngrp ? bfidx[nj.c_off + slot] : -1;
         const double v = Kb[i];
-        if (qq < nj.nbf && v != 0.0)
-            unsafeAtomicAdd(Kout + (size_t)func(ml0 + i / KQ) * nbf + bfidx[nj.bf_off + qq], v);
+        if (q >= 0 && v != 0.0) unsafeAtomicAdd(Kout + (size_t)func(ml0 + i / KQ) * nbf + q, v);
     }
 }
 
@@ -488,6 +519,7 @@ struct KBuilder {
     double budget;                   // bytes of the K accumulators
     std::vector<int> ra, rb;
     std::vector<char> sw;
+    std::vector<int> bf_shell;       // shell of every basis function
     std::vector<long long> pb_off;   // expanded basis of each tree node in PB (-1: none)
     std::vector<int> node_list;      // tree node -> KNode id (-1: not built)
 
@@ -499,6 +531,9 @@ struct KBuilder {
     bool pair_rows() {
         const int N = h->krnl_mat_size, np = h->num_sp;
         ra.assign(N, -1); rb.assign(N, -1); sw.assign(N, 0);
+        bf_shell.assign(h->num_bf, -1);
+        for (int s = 0; s < h->nshell; s++)
+            for (int k = h->shell_bf_sidx[s]; k < h->shell_bf_sidx[s + 1] && k < h->num_bf; k++) bf_shell[k] = s;
         for (int i = 0; i < np; i++) {
             const int s0 = h->sp_shell_idx[i], s1 = h->sp_shell_idx[i + np];
             const int f0 = h->shell_bf_sidx[s0], n0 = h->shell_bf_sidx[s0 + 1] - f0;
@@ -555,6 +590,100 @@ struct KBuilder {
             }
     }
 
+    // Column slots of a node: pairs of functions q and their entries merged on
+    // p, in fours.  Functions of one shell share their partners, so pairs are
+    // taken within a shell first; the functions left over meet the one whose
+    // list leaves the fewest entries single.  Long lists are cut (the parts
+    // are slots of their own and add into the same q) and pairs come longest
+    // first, so that the eight waves of a task have lists of about one length:
+    // with pairs of neighbours in order the longest list of a task was twice
+    // the mean (C30H62: 175 GFLOP of ket steps for 90 GFLOP of entries, 97 for
+    // 71 with the pairs sorted and uncut).  The cut is the one with the
+    // fewest MFMAs per step of n: `bra` per task and two per four of the
+    // longest list, four past those in registers.
+    void column_pairs(KNode &kn, const std::vector<int> &bfs, const std::vector<std::vector<int2>> &byq, double bra) {
+        const int nb = (int)bfs.size();
+        struct Pair { int a, b; std::vector<int4> e; };
+        std::vector<Pair> pairs;
+        std::vector<int> single;
+        for (int i = 0; i < nb;) {
+            int j = i + 1;
+            while (j < nb && bf_shell[bfs[j]] == bf_shell[bfs[i]]) j++;
+            for (; i + 1 < j; i += 2) pairs.push_back(Pair{i, i + 1, {}});
+            if (i < j) single.push_back(i++);
+        }
+        std::vector<std::vector<int>> ps(nb);   // partners p, sorted
+        for (int i = 0; i < nb; i++) {
+            for (const int2 &e : byq[i]) ps[i].push_back(e.y);
+            std::sort(ps[i].begin(), ps[i].end());
+        }
+        std::stable_sort(single.begin(), single.end(), [&](int x, int y) { return ps[x].size() > ps[y].size(); });
+        std::vector<char> used(single.size(), 0);
+        for (size_t i = 0; i < single.size(); i++) {
+            if (used[i]) continue;
+            const std::vector<int> &x = ps[single[i]];
+            size_t best = 0, cost = 0, seen = 0;
+            for (size_t j = i + 1; j < single.size() && seen < 64; j++) {
+                if (used[j]) continue;
+                seen++;
+                const std::vector<int> &y = ps[single[j]];
+                size_t k = 0, l = 0, common = 0;
+                while (k < x.size() && l < y.size()) {
+                    if (x[k] == y[l]) { common++; k++; l++; }
+                    else if (x[k] < y[l]) k++;
+                    else l++;
+                }
+                const size_t c = x.size() + y.size() - 2 * common;
+                if (best == 0 || c < cost) { best = j; cost = c; }
+            }
+            if (best) used[best] = 1;
+            pairs.push_back(Pair{single[i], best ? single[best] : -1, {}});
+        }
+        for (Pair &p : pairs) {
+            std::map<int, int2> at;
+            for (int j = 0; j < 2; j++)
+                if ((j == 0 ? p.a : p.b) >= 0)
+                    for (const int2 &e : byq[j == 0 ? p.a : p.b]) {
+                        int2 &c = at.emplace(e.y, make_int2(-1, -1)).first->second;
+                        (j == 0 ? c.x : c.y) = e.x;
+                    }
+            for (const auto &e : at) p.e.push_back(make_int4(e.second.x, e.second.y, e.first, 0));
+        }
+        // lengths in fours of the parts for a cut of `cap` fours, longest first
+        auto parts = [&](int cap) {
+            std::vector<std::pair<int, int>> v;   // length, pair
+            for (int i = 0; i < (int)pairs.size(); i++) {
+                const int n4 = ((int)pairs[i].e.size() + 3) / 4, np = (n4 + cap - 1) / cap;
+                for (int k = 0; k < np; k++) v.push_back({n4 * (k + 1) / np - n4 * k / np, i});
+            }
+            std::stable_sort(v.begin(), v.end(), [](const std::pair<int, int> &x, const std::pair<int, int> &y) { return x.first > y.first; });
+            return v;
+        };
+        std::vector<std::pair<int, int>> v;
+        double cost = 0.0;
+        for (int cap : {4, 5, 6, 7, 8, 9, 10, 11, 12, 14, 16, 20, 24, 32, 48, 64, 1 << 28}) {
+            std::vector<std::pair<int, int>> w = parts(cap);
+            double c = 0.0;
+            for (size_t g = 0; g < w.size(); g += KQ / 2) c += bra + 2.0 * w[g].first + 2.0 * std::max(0, w[g].first - KNQ);
+            if (v.empty() || c < cost) { v = w; cost = c; }
+        }
+        kn.g_ptr = (int)P.gptr.size();
+        kn.c_off = (int)P.bfidx.size();
+        kn.ngrp = (int)v.size();
+        std::vector<size_t> at(pairs.size(), 0);
+        for (const auto &g : v) {
+            const Pair &p = pairs[g.second];
+            P.gptr.push_back((int)P.ge.size());
+            for (int k = 0; k < 4 * g.first; k++) {
+                const size_t i = at[g.second]++;
+                P.ge.push_back(i < p.e.size() ? p.e[i] : make_int4(-1, -1, 0, 0));
+            }
+            P.bfidx.push_back(bfs[p.a]);
+            P.bfidx.push_back(p.b >= 0 ? bfs[p.b] : -1);
+        }
+        P.gptr.push_back((int)P.ge.size());
+    }
+
     // basis-function set and orientation lists of a tree node's row range
     int list_of(int node) {
         if (node_list[node] >= 0) return node_list[node];
@@ -588,21 +717,6 @@ struct KBuilder {
         kn.m_ptr = (int)P.mptr.size();
         for (int i = 0; i < nb; i++) { P.mptr.push_back((int)P.ment.size()); P.ment.insert(P.ment.end(), bym[i].begin(), bym[i].end()); }
         P.mptr.push_back((int)P.ment.size());
-        // pairs of q: their entries merged on p, padded with empty entries to
-        // whole eights
-        kn.g_ptr = (int)P.gptr.size();
-        for (int g = 0; g < nb; g += 2) {
-            P.gptr.push_back((int)P.ge.size());
-            std::map<int, int2> at;
-            for (int j = 0; j < 2 && g + j < nb; j++)
-                for (const int2 &e : byq[g + j]) {
-                    int2 &c = at.emplace(e.y, make_int2(-1, -1)).first->second;
-                    (j == 0 ? c.x : c.y) = e.x;
-                }
-            for (const auto &e : at) P.ge.push_back(make_int4(e.second.x, e.second.y, e.first, 0));
-            for (size_t k = at.size(); k & 7; k++) P.ge.push_back(make_int4(-1, -1, 0, 0));
-        }
-        P.gptr.push_back((int)P.ge.size());
         // bra: for each local n the (row, local m) entries, sorted by m; per
         // split of ssz functions m (at most KM, even parts so that no split is
         // a sliver) and step of 16 n, blocks of up to 16 entries dealt to the
@@ -636,6 +750,8 @@ struct KBuilder {
                 }
             }
         P.bptr.push_back((int)P.brow.size() / 16);
+        // a step of n costs a wave about four MFMAs per bra block
+        column_pairs(kn, bfs, byq, 4.0 * (P.bptr.back() - P.bptr[kn.b_ptr]) / (8.0 * kn.nsplit * ((nb + 15) / 16)));
         P.mmax = std::max(P.mmax, kn.ssz);
         P.nmax = std::max(P.nmax, nb);
         P.nodes.push_back(kn);
@@ -760,7 +876,7 @@ struct KBuilder {
         std::stable_sort(order.begin(), order.end(), [](const std::pair<double, int> &a, const std::pair<double, int> &b) { return a.first > b.first; });
         for (const auto &o : order) {
             const KNode &ni = P.nodes[P.terms[o.second].ni], &nj = P.nodes[P.terms[o.second].nj];
-            for (int ql0 = 0; ql0 < nj.nbf; ql0 += KQ)
+            for (int ql0 = 0; ql0 < 2 * nj.ngrp; ql0 += KQ)
                 for (int sp = 0; sp < ni.nsplit; sp++) P.block.push_back(KTask{o.second, ql0, sp, 0});
         }
         const double acc = 16.0 * (double)h->num_bf * h->num_bf;   // bytes of one (K1, K_diag)
@@ -781,8 +897,10 @@ struct KBuilder {
         }
         for (const KNode &n : P.nodes) {
             bool ok = n.bf_off >= 0 && n.bf_off + n.nbf <= (long long)P.bfidx.size() && n.q_ptr + n.nbf < (long long)P.qptr.size() &&
-                      n.m_ptr + n.nbf < (long long)P.mptr.size() && n.g_ptr + (n.nbf + 1) / 2 < (long long)P.gptr.size();
+                      n.m_ptr + n.nbf < (long long)P.mptr.size() && n.g_ptr + n.ngrp < (long long)P.gptr.size() &&
+                      n.c_off >= 0 && n.c_off + 2LL * n.ngrp <= (long long)P.bfidx.size();
             for (int i = 0; ok && i < n.nbf; i++) ok = P.bfidx[n.bf_off + i] >= 0 && P.bfidx[n.bf_off + i] < nbf;
+            for (int i = 0; ok && i < 2 * n.ngrp; i++) ok = P.bfidx[n.c_off + i] >= -1 && P.bfidx[n.c_off + i] < nbf;
             if (!ok) { set_error(ERR_ARG, "exchange plan check failed: node lists"); return false; }
         }
         for (const KTerm &t : P.terms) {
@@ -791,10 +909,9 @@ struct KBuilder {
             // entries: columns < m1, p < nbf; rows < m0, local n < |B(i)|
             for (int j = P.qptr[nj.q_ptr]; ok && j < P.qptr[nj.q_ptr + nj.nbf]; j++)
                 ok = P.qent[j].x >= 0 && P.qent[j].x < t.m1 && P.qent[j].y >= 0 && P.qent[j].y < nbf;
-            const int ng = (nj.nbf + 1) / 2;
-            for (int g = 0; ok && g < ng; g++) {
+            for (int g = 0; ok && g < nj.ngrp; g++) {
                 const int ga = P.gptr[nj.g_ptr + g], gb = P.gptr[nj.g_ptr + g + 1];
-                ok = ga >= 0 && ga <= gb && gb <= (int)P.ge.size() && (gb - ga) % 8 == 0;
+                ok = ga >= 0 && ga <= gb && gb <= (int)P.ge.size() && (gb - ga) % 4 == 0;
                 for (int j = ga; ok && j < gb; j++) {
                     ok = P.ge[j].z >= 0 && P.ge[j].z < nbf && P.ge[j].x < t.m1 && P.ge[j].y < t.m1;
                 }
@@ -830,7 +947,7 @@ struct KBuilder {
             ok = k.term >= 0 && k.term < (int)P.terms.size() && !P.terms[k.term].direct;
             if (!ok) break;
             const KNode &ni = P.nodes[P.terms[k.term].ni], &nj = P.nodes[P.terms[k.term].nj];
-            ok = k.e0 >= 0 && k.e0 < nj.nbf && k.e0 % KQ == 0 && k.t0 >= 0 && k.t0 < ni.nsplit;
+            ok = k.e0 >= 0 && k.e0 < 2 * nj.ngrp && k.e0 % KQ == 0 && k.t0 >= 0 && k.t0 < ni.nsplit;
         }
         if (!ok) { set_error(ERR_ARG, "exchange plan check failed: tasks"); return false; }
         return true;
