@@ -86,7 +86,8 @@ struct KNode {           // per row/column range: basis-function set and the ori
     int bf_off, nbf;      // B(node) = bfidx[bf_off .. bf_off + nbf)
     int q_ptr;            // byQ CSR rows: qptr[q_ptr .. q_ptr + nbf]   entries (column c, p)
     int m_ptr;            // byM CSR rows: mptr[m_ptr .. m_ptr + nbf]   entries (row r, local n)
-    int g_ptr;            // merged lists of pairs of column slots: gptr[g_ptr + g]   entries (p, columns c of the two)
+    int g_ptr;            // merged lists of pairs of column slots: gptr[g_ptr + 2 g]   entries (p, columns c of the two),
+                          // gptr[g_ptr + 2 g + 1] of their fours (the first ones) have every entry in both
     int c_off, ngrp;      // functions q of the 2 ngrp column slots: bfidx[c_off + slot] (-1: none)
     int b_ptr;            // bra block lists: bptr[b_ptr + ((split * steps of 16 n) + step) * 8 + wave], and the next one
     int nsplit;           // splits of the functions m
@@ -118,7 +119,13 @@ static const int KPAD = 32;     // readable doubles past every operand array
 // functions of a larger node are cut into even splits, each of which forms
 // its G again.
 static const int KM = 352;
-static const int KMNONE = 0xffffff;   // local m of a block's row without an entry (24 bits)
+// A bra entry: row r, and the byte of m's row in the K block (16 bits; the row
+// past the last is a sink for rows of a block without an entry) under local n
+// (4 bits) and flags of the block.
+static const int KMORE = 16;          // the wave's next block is of the same functions m
+static const int KFIRST = 32;         // the block before is not
+static const int KEMPTY = 64;         // no entry at all
+static const int KCHAIN = 3;          // most blocks in a row of the same m
 
 // Operand addresses are a uniform base and a byte offset O per lane: 32 bits,
 // or 64 where an operand array of a term or D is larger than 4 GB (or a node
@@ -134,6 +141,12 @@ template <typename O>
 __device__ __forceinline__ double kload(const double *p, O byte) {
     return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + byte);
 }
+
+static const int KNS = 2;       // fours read at a time past them
+
+// byte offset of a row: 24-bit factors (checked on the host) in the 32-bit form
+__device__ __forceinline__ unsigned krow(int r, unsigned ld) { return __umul24(r, ld); }
+__device__ __forceinline__ unsigned long long krow(int r, unsigned long long ld) { return (unsigned long long)r * ld; }
 
 // f(integral constant of min(n, KNQ)): straight-line code for every length
 template <typename F>
@@ -164,23 +177,33 @@ __device__ __forceinline__ void kfours(int n, F f) {
 //        stay in registers over all steps of n: a step loads one D operand
 //        per two MFMAs.  Entries past them are read again in every step.
 //   bra  K[m][q] += sum over the entries (r, m) of n of L[r][t] G[n][t][q]:
-//        the entries of every n in blocks of 16 rows, dealt to the waves in
-//        turn; a block's tile is added into the K block in LDS with FP64 LDS
-//        atomics (tiles of different n may share an m).  Its operands are one
-//        stream over all steps: the next block's rows are in flight across
-//        the barriers, and their indices one further ahead.
+//        the entries of every n in blocks of 16 rows, dealt to the waves; the
+//        functions n of a shell have the same m, so up to three of them add
+//        up in one tile, which is added into the K block in LDS with FP64 LDS
+//        atomics (tiles of different shells may share an m).  Its operands are one
+//        stream over all steps: the next two blocks' rows are in flight, across
+//        the barriers too, and their indices two further ahead.
 // At the end the K block is added into K with FP64 global atomics.
 //
-// What bounds it: the bra (C30H62: ket steps alone 2.3 ms, bra alone 3.7 ms of
-// the build's 5.6; the LDS atomics and the shuffles of their rows are 0.7 ms
-// of the bra, and a wave waits at the two barriers of a step for the one with
-// most blocks) and FP64 MFMA issue (64 cycles each); about half of the MFMA
-// work is padding, since the entries of an n come in sixteens.  A second block
-// in flight per wave: no gain (5.64 / 5.72 ms).  16 waves per CU (128 VGPRs,
-// two workgroups by LDS): 40 entries in registers spill (5.86 ms).
+// What bounds it: FP64 MFMA issue together with VALU issue, which it does not
+// overlap: an MFMA takes 64 cycles of its SIMD, at most 62 TFLOP/s on this
+// card, and every VALU instruction beside it adds about two (twelve per MFMA:
+// 44 TFLOP/s).  C30H62 issues 193 GFLOP of MFMAs, half of them padding (the
+// entries of an n come in sixteens, those of a q in fours): 3.1 ms of the 5.15.
+// So the loops are kept short of VALU work: fours that both functions have
+// meet their D operands unmasked, rows without an entry add into a sink
+// instead of being masked, K block bytes and flags are in the lists.  Masks,
+// index arithmetic and register copies in the loops: 5.50 ms.
+// What is left beside it: a wave waits at a step's two barriers for the one
+// with most work (0.6 ms), the loads of a new t (0.2) and the LDS atomics
+// (0.15).  Operand latency is covered: rows padded to whole 128-byte lines
+// (5.55 ms), a second block in flight (5.52) and the next step's D in
+// registers (5.63) changed nothing or cost.  16 waves per CU (128 VGPRs, two
+// workgroups by LDS): 40 entries in registers spill (5.86 ms against 5.64).
 // K per build with G in HBM between two kernels / G in LDS, R read in every
-// step of n and neighbouring functions paired in order / this one:
-// C10H22 2.77 / 1.52 / 1.17 ms, C30H62 13.1 / 7.37 / 5.64 ms.
+// step of n and neighbouring functions paired in order / R in registers and
+// balanced slots / this one: C10H22 2.77 / 1.52 / 1.16 / 1.08 ms, C30H62
+// 13.1 / 7.37 / 5.64 / 5.15 ms.
 template <typename O>
 __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ tasks, const KTerm *__restrict__ terms,
                                                     const KNode *__restrict__ nodes, const int *__restrict__ bfidx,
@@ -194,7 +217,7 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
     const KTerm t = terms[tk.term];
     const KNode ni = nodes[t.ni], nj = nodes[t.nj];
     double *Gt = lds, *Kb = lds + KGT;
-    int *nof = reinterpret_cast<int *>(Kb + ni.ssz * KQ);   // function of every local n (32-bit form)
+    int *nof = reinterpret_cast<int *>(Kb + (ni.ssz + 1) * KQ);   // function of every local n (32-bit form)
     const int q0 = tk.e0, split = tk.t0, ml0 = split * ni.ssz;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int l16 = lane & 15, kl = lane >> 4;
@@ -213,7 +236,8 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
     // one SIMD (w, w + 4) take a long and a short one
     const int grp = (q0 >> 1) + (w < 4 ? w : 11 - w), qw = 2 * (grp - (q0 >> 1));
     const bool gok = grp < nj.ngrp;
-    const int ga = gok ? gptr[nj.g_ptr + grp] : 0, gs = gok ? (gptr[nj.g_ptr + grp + 1] - ga) >> 2 : 0;
+    const int *gp = gptr + nj.g_ptr + 2 * grp;
+    const int ga = gok ? gp[0] : 0, gs = gok ? (gp[2] - ga) >> 2 : 0, gfull = gok ? gp[1] : 0;
     double ra[KNQ][2];      // R operands of the entries of the two q
     O pd[KNQ];              // rows of D
     unsigned has0 = 0, has1 = 0;   // entry i of the lane's exists for the first / second q
@@ -234,17 +258,28 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
             }
         });
     };
-    // ---- bra stream: blocks of the wave's list of the step, t0, step
+    // ---- bra stream: pairs of blocks of the wave's list of the step, steps, t0.
+    // A set of operands is loaded where its last use lies, so that no copy of
+    // registers waits for the load.
     const int *bp = bptr + ni.b_ptr + split * nstep * 8 + w;
-    int bi = bp[0], be = bp[1], bt = 0, bs = 0;   // position of the rows loaded next
-    int2 xr;                       // rows loaded next (row, local m | local n << 24),
-    int xt, om;                    // their t; local m and n of the operands in flight
-    double ol[4];
-    auto bra_index = [&]() { xr = brow[(long long)bi * 16 + l16]; xt = bt; };
-    auto bra_load = [&]() {
-        kload4(L, (O)xr.x * Lld + (O)(xt + 4 * kl) * 8, ol);
-        om = xr.y;
-        bi++;
+    int bi = bp[0], be = bp[1], bs = 0, bt = 0, xt = 0;   // position of the rows xr; t of the operands loaded next
+    int2 xr[2];                    // rows loaded next (row, local m | (local n | KMORE) << 24)
+    int om[2];                     // local m and n of the operands in flight
+    double ol[2][4];
+    const unsigned xo = l16 * 8;
+    auto bra_index = [&](int j) {
+        xr[j] = *reinterpret_cast<const int2 *>(reinterpret_cast<const char *>(brow + (long long)(bi + j) * 16) + xo);
+    };
+    auto bra_load = [&](int j) {
+        kload4(L, krow(xr[j].x, Lld) + (O)(xt + 4 * kl) * 8, ol[j]);
+        // a copy that keeps xr free for the load below (sharing its register would
+        // put a copy that waits for that load at the end of the loop)
+        asm volatile("v_mov_b32 %0, %1" : "=v"(om[j]) : "v"(xr[j].y));
+        bra_index(j);
+    };
+    auto bra_next = [&]() {
+        xt = bt;
+        bi += 2;
         if (bi == be) {
             if (++bs == nstep) {
                 bs = 0;
@@ -253,10 +288,12 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
             bi = bp[8 * bs];
             be = bp[8 * bs + 1];
         }
-        bra_index();
     };
-    bra_index();
-    bra_load();
+    bra_index(0);
+    bra_index(1);
+    bra_next();
+    bra_load(0);
+    bra_load(1);
 
     for (int t0 = 0; t0 < kk; t0 += 16) {
         ket_rows(t0);
@@ -265,59 +302,74 @@ __global__ __launch_bounds__(KBWG, 4) void kx_block(const KTask *__restrict__ ta
             const O no = (O)func(min(16 * st + l16, ni.nbf - 1)) * 8;   // n past the last repeat it (not used)
             d4 acc[2];
             acc[0] = acc[1] = d4{0.0, 0.0, 0.0, 0.0};
-            kfours(gs, [&](auto N) {
+            auto ket = [&](auto N, auto same) {
                 double d[N];
                 #pragma unroll
                 for (int i = 0; i < N; i++) d[i] = kload(D, pd[i] + no);
                 #pragma unroll
-                for (int i = 0; i < N; i++) {
-                    acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[i][0], has0 >> i & 1 ? d[i] : 0.0, acc[0], 0, 0, 0);
-                    acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[i][1], has1 >> i & 1 ? d[i] : 0.0, acc[1], 0, 0, 0);
+                for (int i = 0; i < N - 1; i++) {
+                    acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[i][0], same || has0 >> i & 1 ? d[i] : 0.0, acc[0], 0, 0, 0);
+                    acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[i][1], same || has1 >> i & 1 ? d[i] : 0.0, acc[1], 0, 0, 0);
                 }
-            });
-            for (int s = KNQ; s < gs; s += 4) {   // entries past the registers
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[N - 1][0], has0 >> (N - 1) & 1 ? d[N - 1] : 0.0, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[N - 1][1], has1 >> (N - 1) & 1 ? d[N - 1] : 0.0, acc[1], 0, 0, 0);
+            };
+            if (gfull >= min(gs, KNQ) - 1) kfours(gs, [&](auto N) { ket(N, std::true_type()); });
+            else kfours(gs, [&](auto N) { ket(N, std::false_type()); });
+            for (int s = KNQ; s < gs; s += KNS) {   // entries past the registers
                 const O to = (O)min(t0 + l16, kk - 1) * Rcs;
-                int4 x[4];
-                double a[4][2], d[4];
+                int4 x[KNS];
+                double a[KNS][2], d[KNS];
                 #pragma unroll
-                for (int u = 0; u < 4; u++) {
+                for (int u = 0; u < KNS; u++) {
                     x[u] = ge[ga + 4 * min(s + u, gs - 1) + kl];
                     if (s + u >= gs) x[u].x = x[u].y = -1;
                 }
                 #pragma unroll
-                for (int u = 0; u < 4; u++) {
+                for (int u = 0; u < KNS; u++) {
                     a[u][0] = kload(R, (O)max(x[u].x, 0) * Rrs + to);
                     a[u][1] = kload(R, (O)max(x[u].y, 0) * Rrs + to);
                     d[u] = kload(D, (O)x[u].z * Dld + no);
                 }
                 #pragma unroll
-                for (int u = 0; u < 4; u++) {
+                for (int u = 0; u < KNS; u++) {
                     acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][0], x[u].x >= 0 ? d[u] : 0.0, acc[0], 0, 0, 0);
                     acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][1], x[u].y >= 0 ? d[u] : 0.0, acc[1], 0, 0, 0);
                 }
             }
-            #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int tl = kl + 4 * r;
-                const bool tv = t0 + tl < kk;   // zero past the last t: what the bra's loads find there does not count
-                *reinterpret_cast<double2 *>(Gt + l16 * KGN + tl * 16 + qw) = make_double2(tv ? acc[0][r] : 0.0, tv ? acc[1][r] : 0.0);
+            if (t0 + 16 > kk) {   // zero past the last t: what the bra's loads find there does not count
+                #pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (t0 + kl + 4 * r >= kk) acc[0][r] = acc[1][r] = 0.0;
             }
+            #pragma unroll
+            for (int r = 0; r < 4; r++)
+                *reinterpret_cast<double2 *>(Gt + l16 * KGN + (4 * kl + r) * 16 + qw) = make_double2(acc[0][r], acc[1][r]);
             __syncthreads();
-            // MFMA u takes the inner indices t = 4 k + u
-            for (int b = b0; b < b1; b++) {
-                double a[4];
+            // MFMA u takes the inner indices t = 4 k + u, which lie at k + 4 u of the
+            // G tile: its 64 values are one run of LDS
+            d4 x;
+            for (int b = b0; b < b1; b += 2) {
+                bra_next();
                 #pragma unroll
-                for (int u = 0; u < 4; u++) a[u] = ol[u];
-                const int mn = om;
-                bra_load();
-                const double *g = Gt + (__builtin_amdgcn_readfirstlane(mn) >> 24) * KGN + kl * 64 + l16;
-                d4 x = d4{0.0, 0.0, 0.0, 0.0};
-                #pragma unroll
-                for (int u = 0; u < 4; u++) x = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], g[16 * u], x, 0, 0, 0);
-                #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int m = __shfl(mn, kl + 4 * r) & KMNONE;   // lane e of the wave holds entry e's
-                    if (m != KMNONE) atomicAdd(&Kb[(m - ml0) * KQ + l16], x[r]);
+                for (int j = 0; j < 2; j++) {
+                    const int nf = __builtin_amdgcn_readfirstlane(om[j]) >> 16;   // local n and flags
+                    if (!(nf & KEMPTY)) {
+                        const double *g = Gt + (nf & 15) * KGN + lane;
+                        if (nf & KFIRST) x = __builtin_amdgcn_mfma_f64_16x16x4f64(ol[j][0], g[0], d4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+                        else x = __builtin_amdgcn_mfma_f64_16x16x4f64(ol[j][0], g[0], x, 0, 0, 0);
+                        #pragma unroll
+                        for (int u = 1; u < 4; u++) x = __builtin_amdgcn_mfma_f64_16x16x4f64(ol[j][u], g[64 * u], x, 0, 0, 0);
+                        if (!(nf & KMORE)) {   // else the next block has the same m
+                            int m[4];
+                            #pragma unroll
+                            for (int r = 0; r < 4; r++) m[r] = __shfl(om[j], kl + 4 * r);   // lane e of the wave holds entry e's
+                            #pragma unroll
+                            for (int r = 0; r < 4; r++)
+                                atomicAdd(reinterpret_cast<double *>(reinterpret_cast<char *>(Kb) + ((m[r] & 0xffff) | xo)), x[r]);
+                        }
+                    }
+                    bra_load(j);
                 }
             }
             __syncthreads();
@@ -460,8 +512,8 @@ struct KPlan {
     std::vector<KGemm> gemms;
     std::vector<KNode> nodes;
     std::vector<int> bfidx, qptr, mptr, bptr, gptr;
-    // bra blocks: 16 (row r, local m | local n within the step << 24) each, the
-    // last row repeated with m = KMNONE past a block's entries
+    // bra blocks: 16 (row r, byte of m in the K block | (local n within the step | flags) << 16) each, the
+    // last row repeated with the sink's byte past a block's entries
     std::vector<int2> qent, ment, brow;
     std::vector<int4> ge;   // ket entries: columns c of the two q (-1: none), p
     std::vector<KTask> block, direct;
@@ -647,7 +699,9 @@ struct KBuilder {
                         int2 &c = at.emplace(e.y, make_int2(-1, -1)).first->second;
                         (j == 0 ? c.x : c.y) = e.x;
                     }
-            for (const auto &e : at) p.e.push_back(make_int4(e.second.x, e.second.y, e.first, 0));
+            for (int both = 1; both >= 0; both--)   // entries that both have come first
+                for (const auto &e : at)
+                    if ((e.second.x >= 0 && e.second.y >= 0) == (both == 1)) p.e.push_back(make_int4(e.second.x, e.second.y, e.first, 0));
         }
         // lengths in fours of the parts for a cut of `cap` fours, longest first
         auto parts = [&](int cap) {
@@ -674,10 +728,13 @@ struct KBuilder {
         for (const auto &g : v) {
             const Pair &p = pairs[g.second];
             P.gptr.push_back((int)P.ge.size());
+            int full = 0;
             for (int k = 0; k < 4 * g.first; k++) {
                 const size_t i = at[g.second]++;
                 P.ge.push_back(i < p.e.size() ? p.e[i] : make_int4(-1, -1, 0, 0));
+                if (full == k && P.ge.back().x >= 0 && P.ge.back().y >= 0) full++;
             }
+            P.gptr.push_back(full / 4);
             P.bfidx.push_back(bfs[p.a]);
             P.bfidx.push_back(p.b >= 0 ? bfs[p.b] : -1);
         }
@@ -720,38 +777,68 @@ struct KBuilder {
         // bra: for each local n the (row, local m) entries, sorted by m; per
         // split of ssz functions m (at most KM, even parts so that no split is
         // a sliver) and step of 16 n, blocks of up to 16 entries dealt to the
-        // eight waves in turn (a wave without one gets an empty block)
+        // eight waves, an even number each (empty ones make up for it)
         std::vector<std::vector<int2>> byn(nb);
         for (int ml = 0; ml < nb; ml++)
             for (const int2 &e : bym[ml]) byn[e.y].push_back(make_int2(e.x, ml));
         kn.nsplit = (nb + KM - 1) / KM;
         kn.ssz = kn.nsplit > 0 ? (nb + kn.nsplit - 1) / kn.nsplit : KM;
         kn.b_ptr = (int)P.bptr.size();
+        int nblk = 0;   // not empty
         for (int sp = 0; sp < kn.nsplit; sp++)
             for (int n0 = 0; n0 < nb; n0 += 16) {
-                struct Blk { int nl, e0, cnt; };
-                std::vector<Blk> wv[8];
-                int turn = 0;
-                for (int nl = n0; nl < std::min(n0 + 16, nb); nl++) {
+                // runs of functions n of one shell, whose lists hold the same m: a
+                // chain takes the same 16 entries of each, in one accumulator
+                struct Chain { int nl, nn, e0, cnt; };
+                std::vector<Chain> ch;
+                auto range = [&](int nl) {   // entries of the split
                     int a = 0, b = 0;
                     while (a < (int)byn[nl].size() && byn[nl][a].y < sp * kn.ssz) a++;
                     for (b = a; b < (int)byn[nl].size() && byn[nl][b].y < (sp + 1) * kn.ssz;) b++;
-                    for (int e = a; e < b; e += 16)
-                        wv[turn++ & 7].push_back(Blk{nl, e, std::min(16, b - e)});
+                    return std::make_pair(a, b);
+                };
+                const int n1 = std::min(n0 + 16, nb);
+                for (int nl = n0, nn; nl < n1; nl += nn) {
+                    const auto r = range(nl);
+                    for (nn = 1; nn < KCHAIN && nl + nn < n1; nn++) {
+                        const auto q = range(nl + nn);
+                        if (bf_shell[bfs[nl + nn]] != bf_shell[bfs[nl]] || q.second - q.first != r.second - r.first) break;
+                        bool same = true;
+                        for (int k = 0; same && k < r.second - r.first; k++)
+                            same = byn[nl + nn][q.first + k].y == byn[nl][r.first + k].y;
+                        if (!same) break;
+                    }
+                    for (int e = r.first; e < r.second; e += 16)
+                        ch.push_back(Chain{nl, nn, e - r.first, std::min(16, r.second - e)});
+                }
+                // to the wave with the fewest blocks, long chains first
+                std::stable_sort(ch.begin(), ch.end(), [](const Chain &x, const Chain &y) { return x.nn > y.nn; });
+                std::vector<Chain> wv[8];
+                int load[8] = {0};
+                for (const Chain &c : ch) {
+                    const int w = (int)(std::min_element(load, load + 8) - load);
+                    load[w] += c.nn;
+                    nblk += c.nn;
+                    wv[w].push_back(c);
                 }
                 for (int w = 0; w < 8; w++) {
                     P.bptr.push_back((int)P.brow.size() / 16);
-                    if (wv[w].empty()) wv[w].push_back(Blk{n0, 0, 0});
-                    for (const Blk &k : wv[w])
-                        for (int e = 0; e < 16; e++) {
-                            const int2 a = k.cnt ? byn[k.nl][k.e0 + std::min(e, k.cnt - 1)] : make_int2(0, 0);
-                            P.brow.push_back(make_int2(a.x, (e < k.cnt ? a.y : KMNONE) | (k.nl - n0) << 24));
+                    if (load[w] == 0 || load[w] % 2) wv[w].push_back(Chain{n0, 1, 0, 0});
+                    if (load[w] == 0) wv[w].push_back(Chain{n0, 1, 0, 0});
+                    for (const Chain &c : wv[w])
+                        for (int k = 0; k < c.nn; k++) {
+                            const int a0 = range(c.nl + k).first + c.e0;
+                            const int nf = (c.nl + k - n0) | (k + 1 < c.nn ? KMORE : 0) | (k == 0 ? KFIRST : 0) | (c.cnt == 0 ? KEMPTY : 0);
+                            for (int e = 0; e < 16; e++) {
+                                const int2 a = c.cnt ? byn[c.nl + k][a0 + std::min(e, c.cnt - 1)] : make_int2(0, 0);
+                                P.brow.push_back(make_int2(a.x, (e < c.cnt ? a.y - sp * kn.ssz : kn.ssz) * KQ * 8 | nf << 16));
+                            }
                         }
                 }
             }
         P.bptr.push_back((int)P.brow.size() / 16);
         // a step of n costs a wave about four MFMAs per bra block
-        column_pairs(kn, bfs, byq, 4.0 * (P.bptr.back() - P.bptr[kn.b_ptr]) / (8.0 * kn.nsplit * ((nb + 15) / 16)));
+        column_pairs(kn, bfs, byq, 4.0 * nblk / (8.0 * kn.nsplit * ((nb + 15) / 16)));
         P.mmax = std::max(P.mmax, kn.ssz);
         P.nmax = std::max(P.nmax, nb);
         P.nodes.push_back(kn);
@@ -869,7 +956,7 @@ struct KBuilder {
             }
             const double reach = std::max({(double)t.m1 * t.Rrs + (double)t.kk * t.Rcs, (double)t.m0 * t.Lld + t.kk + KPAD,
                                            (double)h->num_bf * h->num_bf});
-            if (reach * 8.0 >= 4294967296.0 || ni.nbf > 4096) P.wide = true;
+            if (reach * 8.0 >= 4294967296.0 || ni.nbf > 4096 || t.m0 >= 1 << 24 || t.Lld >= 1 << 21) P.wide = true;
             const double steps = (double)((ni.nbf + 15) / 16) * ((t.kk + 15) / 16);
             order.push_back({steps * (4.0 + (double)t.m1 / nj.nbf + (double)t.m0 / ni.nbf), ti});
         }
@@ -897,7 +984,7 @@ struct KBuilder {
         }
         for (const KNode &n : P.nodes) {
             bool ok = n.bf_off >= 0 && n.bf_off + n.nbf <= (long long)P.bfidx.size() && n.q_ptr + n.nbf < (long long)P.qptr.size() &&
-                      n.m_ptr + n.nbf < (long long)P.mptr.size() && n.g_ptr + n.ngrp < (long long)P.gptr.size() &&
+                      n.m_ptr + n.nbf < (long long)P.mptr.size() && n.g_ptr + 2LL * n.ngrp < (long long)P.gptr.size() &&
                       n.c_off >= 0 && n.c_off + 2LL * n.ngrp <= (long long)P.bfidx.size();
             for (int i = 0; ok && i < n.nbf; i++) ok = P.bfidx[n.bf_off + i] >= 0 && P.bfidx[n.bf_off + i] < nbf;
             for (int i = 0; ok && i < 2 * n.ngrp; i++) ok = P.bfidx[n.c_off + i] >= -1 && P.bfidx[n.c_off + i] < nbf;
@@ -910,11 +997,11 @@ struct KBuilder {
             for (int j = P.qptr[nj.q_ptr]; ok && j < P.qptr[nj.q_ptr + nj.nbf]; j++)
                 ok = P.qent[j].x >= 0 && P.qent[j].x < t.m1 && P.qent[j].y >= 0 && P.qent[j].y < nbf;
             for (int g = 0; ok && g < nj.ngrp; g++) {
-                const int ga = P.gptr[nj.g_ptr + g], gb = P.gptr[nj.g_ptr + g + 1];
-                ok = ga >= 0 && ga <= gb && gb <= (int)P.ge.size() && (gb - ga) % 4 == 0;
-                for (int j = ga; ok && j < gb; j++) {
-                    ok = P.ge[j].z >= 0 && P.ge[j].z < nbf && P.ge[j].x < t.m1 && P.ge[j].y < t.m1;
-                }
+                const int ga = P.gptr[nj.g_ptr + 2 * g], gb = P.gptr[nj.g_ptr + 2 * g + 2], full = P.gptr[nj.g_ptr + 2 * g + 1];
+                ok = ga >= 0 && ga <= gb && gb <= (int)P.ge.size() && (gb - ga) % 4 == 0 && full >= 0 && 4 * full <= gb - ga;
+                for (int j = ga; ok && j < gb; j++)
+                    ok = P.ge[j].z >= 0 && P.ge[j].z < nbf && P.ge[j].x < t.m1 && P.ge[j].y < t.m1 &&
+                         (j >= ga + 4 * full || (P.ge[j].x >= 0 && P.ge[j].y >= 0));
             }
             for (int j = P.mptr[ni.m_ptr]; ok && j < P.mptr[ni.m_ptr + ni.nbf]; j++)
                 ok = P.ment[j].x >= 0 && P.ment[j].x < t.m0 && P.ment[j].y >= 0 && P.ment[j].y < ni.nbf;
@@ -922,15 +1009,20 @@ struct KBuilder {
             // the split (the splits cover every local m)
             const int nst = (ni.nbf + 15) / 16;
             ok = ok && ni.nsplit >= 1 && ni.ssz >= 1 && ni.ssz <= KM && (long long)ni.nsplit * ni.ssz >= ni.nbf && ni.b_ptr >= 0 &&
-                 ni.b_ptr + (long long)ni.nsplit * nst * 8 < (long long)P.bptr.size() && ni.nbf < KMNONE;
+                 ni.b_ptr + (long long)ni.nsplit * nst * 8 < (long long)P.bptr.size();
             for (int k = 0; ok && k < ni.nsplit * nst * 8; k++) {
                 const int sp = k / (nst * 8);
                 const int b0 = P.bptr[ni.b_ptr + k], b1 = P.bptr[ni.b_ptr + k + 1];
-                ok = b0 >= 0 && b0 < b1 && b1 <= (int)(P.brow.size() / 16);
+                ok = b0 >= 0 && b0 < b1 && (b1 - b0) % 2 == 0 && b1 <= (int)(P.brow.size() / 16);
+                const int rows = std::min((sp + 1) * ni.ssz, ni.nbf) - sp * ni.ssz;
                 for (int e = 16 * b0; ok && e < 16 * b1; e++) {
-                    const int m = P.brow[e].y & KMNONE, nl = P.brow[e].y >> 24;
-                    ok = P.brow[e].x >= 0 && P.brow[e].x < t.m0 && nl >= 0 && nl < 16 && nl == P.brow[e & ~15].y >> 24 &&
-                         (m == KMNONE || (m >= sp * ni.ssz && m < std::min((sp + 1) * ni.ssz, ni.nbf)));
+                    const int m = P.brow[e].y & 0xffff, nf = P.brow[e].y >> 16;
+                    ok = P.brow[e].x >= 0 && P.brow[e].x < t.m0 && nf >= 0 && nf < 128 && nf == P.brow[e & ~15].y >> 16 &&
+                         m % (KQ * 8) == 0 && (m / (KQ * 8) < rows || m / (KQ * 8) == ni.ssz);
+                    // a chain begins where none goes on, and goes on in a block of the
+                    // same list with the same m
+                    if (ok && (nf & KMORE)) ok = e + 16 < 16 * b1 && (P.brow[e + 16].y & 0xffff) == m && !(P.brow[e + 16].y >> 16 & (KFIRST | KEMPTY));
+                    if (ok && !(nf & KFIRST)) ok = e >= 16 * b0 + 16 && (P.brow[e - 16].y >> 16 & KMORE);
                 }
             }
             ok = ok && t.Loff >= 0 && t.Loff + (long long)(t.m0 - 1) * t.Lld + t.kk <= size_of(t.Lsrc);
@@ -1019,7 +1111,7 @@ static bool k_upload(H2ERI_p h) {
         !up((void **)&k->direct, P.direct.empty() ? nullptr : P.direct.data(), P.direct.size() * sizeof(KTask)) ||
         !up((void **)&k->gtasks, P.gtasks.empty() ? nullptr : P.gtasks.data(), P.gtasks.size() * sizeof(KGemmTask)))
         return false;
-    const int lds = (KGT + P.mmax * KQ) * 8 + (P.wide ? 0 : P.nmax * 4);   // G tile, K block, functions
+    const int lds = (KGT + (P.mmax + 1) * KQ) * 8 + (P.wide ? 0 : P.nmax * 4);   // G tile, K block, functions
     for (const void *f : {reinterpret_cast<const void *>(&kx_block<unsigned>), reinterpret_cast<const void *>(&kx_block<unsigned long long>)})
         KHIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     // (zeros also between the products, whose rows end where the next begins)
@@ -1050,7 +1142,7 @@ static bool k_run(H2ERI_p h, const double *D_dev, double *K_dev, hipStream_t s) 
     // that of the largest split
     if (!P.block.empty())
         hipLaunchKernelGGL(P.wide ? kx_block<unsigned long long> : kx_block<unsigned>, dim3((unsigned)P.block.size()), dim3(KBWG),
-                           (size_t)(KGT + P.mmax * KQ) * 8 + (size_t)(P.wide ? 0 : P.nmax * 4), s, k->block, k->terms,
+                           (size_t)(KGT + (P.mmax + 1) * KQ) * 8 + (size_t)(P.wide ? 0 : P.nmax * 4), s, k->block, k->terms,
                            k->nodes, k->bfidx, k->gptr, k->ge, k->bptr, k->brow, k->PB, k->CB, k->SC, D_dev, k->KA,
                            P.nacc, nbf);
     if (!P.direct.empty())
