@@ -115,7 +115,7 @@ static const int KGT = 16 * KGN;
 static const int KBWG = 512;    // threads of a block task (8 waves)
 static const int KPAD = 32;     // readable doubles past every operand array
 // Most local functions m of a task (its K block in LDS): 352, the G tile and
-// the node's function offsets take 79,488 bytes, two workgroups per CU; the
+// the node's function offsets take 79,616 bytes, two workgroups per CU; the
 // functions of a larger node are cut into even splits, each of which forms
 // its G again.
 static const int KM = 352;
