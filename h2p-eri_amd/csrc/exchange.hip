@@ -692,16 +692,20 @@ struct KBuilder {
             pairs.push_back(Pair{single[i], best ? single[best] : -1, {}});
         }
         for (Pair &p : pairs) {
-            std::map<int, int2> at;
+            // columns of each partner p, of both functions: more than one where a
+            // shell pair is stored in both orders (or twice)
+            struct Cols { std::vector<int> c[2]; };
+            std::map<int, Cols> at;
             for (int j = 0; j < 2; j++)
                 if ((j == 0 ? p.a : p.b) >= 0)
-                    for (const int2 &e : byq[j == 0 ? p.a : p.b]) {
-                        int2 &c = at.emplace(e.y, make_int2(-1, -1)).first->second;
-                        (j == 0 ? c.x : c.y) = e.x;
-                    }
+                    for (const int2 &e : byq[j == 0 ? p.a : p.b]) at[e.y].c[j].push_back(e.x);
             for (int both = 1; both >= 0; both--)   // entries that both have come first
-                for (const auto &e : at)
-                    if ((e.second.x >= 0 && e.second.y >= 0) == (both == 1)) p.e.push_back(make_int4(e.second.x, e.second.y, e.first, 0));
+                for (const auto &e : at) {
+                    const std::vector<int> &x = e.second.c[0], &y = e.second.c[1];
+                    const size_t nboth = std::min(x.size(), y.size()), n = both ? nboth : std::max(x.size(), y.size());
+                    for (size_t k = both ? 0 : nboth; k < n; k++)
+                        p.e.push_back(make_int4(k < x.size() ? x[k] : -1, k < y.size() ? y[k] : -1, e.first, 0));
+                }
         }
         // lengths in fours of the parts for a cut of `cap` fours, longest first
         auto parts = [&](int cap) {
@@ -989,6 +993,19 @@ struct KBuilder {
             for (int i = 0; ok && i < n.nbf; i++) ok = P.bfidx[n.bf_off + i] >= 0 && P.bfidx[n.bf_off + i] < nbf;
             for (int i = 0; ok && i < 2 * n.ngrp; i++) ok = P.bfidx[n.c_off + i] >= -1 && P.bfidx[n.c_off + i] < nbf;
             if (!ok) { set_error(ERR_ARG, "exchange plan check failed: node lists"); return false; }
+            // the column slots of a function hold each of its entries once
+            std::vector<int> live(nbf, 0);
+            for (int i = 0; i < 2 * n.ngrp; i++) {
+                const int q = P.bfidx[n.c_off + i], g = n.g_ptr + 2 * (i >> 1);
+                for (int j = P.gptr[g]; j < P.gptr[g + 2]; j++) {
+                    const bool has = ((i & 1) ? P.ge[j].y : P.ge[j].x) >= 0;
+                    if (has && q < 0) ok = false;
+                    else if (has) live[q]++;
+                }
+            }
+            for (int i = 0; ok && i < n.nbf; i++)
+                ok = live[P.bfidx[n.bf_off + i]] == P.qptr[n.q_ptr + i + 1] - P.qptr[n.q_ptr + i];
+            if (!ok) { set_error(ERR_ARG, "exchange plan check failed: column slots"); return false; }
         }
         for (const KTerm &t : P.terms) {
             const KNode &ni = P.nodes[t.ni], &nj = P.nodes[t.nj];
