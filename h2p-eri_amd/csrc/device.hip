@@ -1344,6 +1344,7 @@ struct DevPlan {
     int *d_need = nullptr, *d_ctr = nullptr;
     // 16 vectors per pass: element-major copy of the pass's input (N x 16)
     double *Xt = nullptr;
+    size_t bytes = 0;   // device memory held
 };
 
 static const int NWIDTH = 5;   // batch widths: vectors per pass over the matrix data
@@ -1410,6 +1411,7 @@ struct DevState {
     int *ws_ctr = nullptr;
     int *last_noalloc_ctr = nullptr;   // counters of the last allocation-free persistent pass
     JitState *jit = nullptr;           // a BD_JIT handle's on-the-fly state (jit.hip)
+    double pass_bytes = 0;             // bound of one plan's device memory (H2ERI_set_pass_memory; 0: none)
 };
 
 static DevState *dstate(H2ERI_p h) { return (DevState *)h->dev; }
@@ -1428,17 +1430,22 @@ static void free_dev(void *&p) {
     if (p) { (void)hipFree(p); p = nullptr; }
 }
 
-static void release_graph(DevState *d);
-static void release_plan(DevState *d, int i) {
-    release_graph(d);
-    DevPlan &p = d->plans[i];
+// Device memory of a plan; of one that a graph may refer to, release_plan.
+static void free_plan(DevPlan &p) {
     void **ps[] = {(void **)&p.Wv, (void **)&p.d_t64, (void **)&p.d_t32, (void **)&p.d_w64, (void **)&p.d_w32,
                    (void **)&p.d_rt, (void **)&p.d_rsrc, (void **)&p.d_vsrc, (void **)&p.d_q, (void **)&p.d_need,
                    (void **)&p.d_ctr, (void **)&p.Xt};
     for (void **q : ps) free_dev(*q);
     p.ready = false;
     p.q_ready = false;
+    p.bytes = 0;
     p.P = Plan();
+}
+
+static void release_graph(DevState *d);
+static void release_plan(DevState *d, int i) {
+    release_graph(d);
+    free_plan(d->plans[i]);
 }
 
 static void release_plans(DevState *d) {
@@ -2373,6 +2380,21 @@ static int queue_grid(int nv) {
     return e == hipSuccess ? ncu * std::max(per, 1) : 0;
 }
 
+// Device memory of a plan, within the handle's bound.
+static bool plan_alloc(DevState *d, DevPlan &dp, void **dst, const void *src, size_t bytes) {
+    if (bytes == 0) bytes = 64;
+    hipError_t e = hipErrorOutOfMemory;
+    if (d->pass_bytes <= 0 || (double)(dp.bytes + bytes) <= d->pass_bytes) e = hipMalloc(dst, bytes);
+    if (e == hipSuccess) dp.bytes += bytes;
+    if (e == hipSuccess && src) e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        set_error(ERR_DEVICE, "plan upload: %s", hipGetErrorString(e));
+        return false;
+    }
+    return true;
+}
+
 // Queue form of an uploaded plan: built on the host, uploaded, counters zeroed.
 static bool ensure_queue(DevState *d, DevPlan &dp) {
     if (dp.q_ready) return true;
@@ -2381,9 +2403,10 @@ static bool ensure_queue(DevState *d, DevPlan &dp) {
     QPlan Q;
     if (!build_queue(dp.P, dp.P.nv, G, Q)) return false;
     const size_t nq = std::max<size_t>(Q.tasks.size(), 1), nl = Q.need.size();
-    HIP_OK(hipMalloc(&dp.d_q, nq * sizeof(QTask)));
-    HIP_OK(hipMalloc(&dp.d_need, std::max<size_t>(nl, 1) * sizeof(int)));
-    HIP_OK(hipMalloc(&dp.d_ctr, (QC_LISTS + nl) * sizeof(int)));
+    if (!plan_alloc(d, dp, (void **)&dp.d_q, nullptr, nq * sizeof(QTask)) ||
+        !plan_alloc(d, dp, (void **)&dp.d_need, nullptr, std::max<size_t>(nl, 1) * sizeof(int)) ||
+        !plan_alloc(d, dp, (void **)&dp.d_ctr, nullptr, (QC_LISTS + nl) * sizeof(int)))
+        return false;
     if (!Q.tasks.empty()) HIP_OK(hipMemcpy(dp.d_q, Q.tasks.data(), Q.tasks.size() * sizeof(QTask), hipMemcpyHostToDevice));
     if (nl) HIP_OK(hipMemcpy(dp.d_need, Q.need.data(), nl * sizeof(int), hipMemcpyHostToDevice));
     HIP_OK(hipMemset(dp.d_ctr, 0, (QC_LISTS + nl) * sizeof(int)));
@@ -2394,7 +2417,6 @@ static bool ensure_queue(DevState *d, DevPlan &dp) {
     dp.q_grid = std::min(G, std::max(dp.q_n, 1));
     dp.q_est_us = Q.est_us;
     dp.q_ready = true;
-    (void)d;
     return true;
 }
 
@@ -2408,32 +2430,28 @@ static DevPlan *get_plan(H2ERI_p h, int nv) {
     DevState *d = dstate(h);
     DevPlan &dp = d->plans[nv_index(nv)];
     const Tune &c = d->cfg[nv_index(nv)];
-    if (dp.ready) {
-        if (c.executor == 1 && !ensure_queue(d, dp)) return nullptr;
-        return &dp;
-    }
-    if (!build_plan(h, d->st, dp.P, nv, c.tile_bytes, c.nf_schedule, c.executor, c.wave_bytes)) return nullptr;
-    const Plan &P = dp.P;
-    auto alloc_copy = [&](void **dst, const void *src, size_t bytes) -> bool {
-        if (bytes == 0) bytes = 64;
-        hipError_t e = hipMalloc(dst, bytes);
-        if (e == hipSuccess && src) e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
-        if (e != hipSuccess) { set_error(ERR_DEVICE, "plan upload: %s", hipGetErrorString(e)); return false; }
-        return true;
+    auto upload = [&]() -> bool {
+        if (!dp.ready) {
+            if (!build_plan(h, d->st, dp.P, nv, c.tile_bytes, c.nf_schedule, c.executor, c.wave_bytes)) return false;
+            const Plan &P = dp.P;
+            auto alloc_copy = [&](void **dst, const void *src, size_t bytes) -> bool { return plan_alloc(d, dp, dst, src, bytes); };
+            if (!alloc_copy((void **)&dp.Wv, nullptr, (size_t)P.nW * nv * 8)) return false;
+            if (hipMemset(dp.Wv, 0, (size_t)P.nW * nv * 8) != hipSuccess) { set_error(ERR_DEVICE, "workspace memset"); return false; }
+            if (!alloc_copy((void **)&dp.d_t64, P.t64.empty() ? nullptr : P.t64.data(), P.t64.size() * sizeof(BTask))) return false;
+            if (!alloc_copy((void **)&dp.d_t32, P.t32.empty() ? nullptr : P.t32.data(), P.t32.size() * sizeof(BTask))) return false;
+            if (!alloc_copy((void **)&dp.d_w64, P.w64.empty() ? nullptr : P.w64.data(), P.w64.size() * sizeof(BTask))) return false;
+            if (!alloc_copy((void **)&dp.d_w32, P.w32.empty() ? nullptr : P.w32.data(), P.w32.size() * sizeof(BTask))) return false;
+            if (!alloc_copy((void **)&dp.d_rt, P.rt.empty() ? nullptr : P.rt.data(), P.rt.size() * sizeof(RTask))) return false;
+            if (!alloc_copy((void **)&dp.d_rsrc, P.rsrc.empty() ? nullptr : P.rsrc.data(), P.rsrc.size() * sizeof(int))) return false;
+            if (!alloc_copy((void **)&dp.d_vsrc, P.vsrc.empty() ? nullptr : P.vsrc.data(), P.vsrc.size() * sizeof(int))) return false;
+            if (nv == 16 && !alloc_copy((void **)&dp.Xt, nullptr, (size_t)h->krnl_mat_size * 16 * sizeof(double))) return false;
+            dp.ready = true;
+        }
+        return c.executor != 1 || ensure_queue(d, dp);
     };
-    if (!alloc_copy((void **)&dp.Wv, nullptr, (size_t)P.nW * nv * 8)) return nullptr;
-    if (hipMemset(dp.Wv, 0, (size_t)P.nW * nv * 8) != hipSuccess) { set_error(ERR_DEVICE, "workspace memset"); return nullptr; }
-    if (!alloc_copy((void **)&dp.d_t64, P.t64.empty() ? nullptr : P.t64.data(), P.t64.size() * sizeof(BTask))) return nullptr;
-    if (!alloc_copy((void **)&dp.d_t32, P.t32.empty() ? nullptr : P.t32.data(), P.t32.size() * sizeof(BTask))) return nullptr;
-    if (!alloc_copy((void **)&dp.d_w64, P.w64.empty() ? nullptr : P.w64.data(), P.w64.size() * sizeof(BTask))) return nullptr;
-    if (!alloc_copy((void **)&dp.d_w32, P.w32.empty() ? nullptr : P.w32.data(), P.w32.size() * sizeof(BTask))) return nullptr;
-    if (!alloc_copy((void **)&dp.d_rt, P.rt.empty() ? nullptr : P.rt.data(), P.rt.size() * sizeof(RTask))) return nullptr;
-    if (!alloc_copy((void **)&dp.d_rsrc, P.rsrc.empty() ? nullptr : P.rsrc.data(), P.rsrc.size() * sizeof(int))) return nullptr;
-    if (!alloc_copy((void **)&dp.d_vsrc, P.vsrc.empty() ? nullptr : P.vsrc.data(), P.vsrc.size() * sizeof(int))) return nullptr;
-    if (nv == 16 && !alloc_copy((void **)&dp.Xt, nullptr, (size_t)h->krnl_mat_size * 16 * sizeof(double))) return nullptr;
-    dp.ready = true;
-    if (c.executor == 1 && !ensure_queue(d, dp)) return nullptr;
-    return &dp;
+    if (upload()) return &dp;
+    free_plan(dp);   // not complete, so no graph refers to it
+    return nullptr;
 }
 
 // Plan of the next pass for `rem` vectors left (nv_pass); when a pass wider
@@ -2446,7 +2464,6 @@ static DevPlan *pass_plan(H2ERI_p h, int rem) {
         DevPlan *dp = get_plan(h, nv);
         if (dp || !padded || h->BD_JIT || !dstate(h)->st_ready) return dp;
         dstate(h)->no_pad[i] = true;
-        release_plan(dstate(h), i);
         (void)hipGetLastError();
         h2eri_clear_error();
     }
@@ -2999,6 +3016,13 @@ size_t H2ERI_upload(H2ERI_p h) {
     if (!d->ev_join && hipEventCreateWithFlags(&d->ev_join, hipEventDisableTiming) != hipSuccess) { set_error(ERR_DEVICE, "event"); return 0; }
     if (!noalloc_scratch(d->dev)) return 0;
     return d->resident_bytes;
+}
+
+// Bound in bytes of the device memory of one pass width's plan (workspace and
+// task lists); 0: none.  Plans that are there stay.
+void H2ERI_set_pass_memory(H2ERI_p h, const double bytes) {
+    if (!h || !(bytes >= 0)) { set_error(ERR_ARG, "H2ERI_set_pass_memory: bytes >= 0"); return; }
+    dstate_get(h)->pass_bytes = bytes;
 }
 
 void H2ERI_set_phase_timing(H2ERI_p h, const int on) {

@@ -204,6 +204,11 @@ class H2ERI:
         self.lib.H2ERI_set_tile_bytes(self.h, float(nbytes))
         _check(self.lib)
 
+    def set_pass_memory(self, nbytes):
+        """Bound of one pass width's plan on the device (bytes; 0: none)."""
+        self.lib.H2ERI_set_pass_memory(self.h, float(nbytes))
+        _check(self.lib)
+
     def plan_check(self, bits=64):
         """Host-only build and bounds check of the device plan (no GPU needed)."""
         r = self.lib.H2ERI_plan_check(self.h, bits)

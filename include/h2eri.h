@@ -391,6 +391,14 @@ int H2ERI_get_launch_stats(H2ERI_p h2eri, const int max_launch, double *out5);
  * bytes of the algorithmic count. */
 void H2ERI_matvec_bytes(H2ERI_p h2eri, double *out6);
 
+/* Bound in bytes of the device memory that the plan of one batch width
+ * (1, 2, 4, 8, 16 vectors per pass) may take for its workspace and task lists
+ * (additive; 0, the default: what the device has).  A pass that would need
+ * more fails as on a full device, except that a batch whose last vectors would
+ * run in a wider pass then runs them in narrower ones.  Plans that are there
+ * stay. */
+void H2ERI_set_pass_memory(H2ERI_p h2eri, const double bytes);
+
 /* Tile size of the device bi-GEMV tasks in bytes (tuning; re-plans the
  * device layout on the next call). */
 void H2ERI_set_tile_bytes(H2ERI_p h2eri, const double bytes);
