@@ -1379,7 +1379,9 @@ struct DevState {
     double *S64 = nullptr;
     float *S32 = nullptr;
     DevPlan plans[NWIDTH];
-    bool no_pad[NWIDTH] = {false, false, false, false, false};   // widths that did not fit a padded pass (pass_plan)
+    // widths that did not fit a padded pass (pass_plan), until a plan or the
+    // storage is released
+    bool no_pad[NWIDTH] = {false, false, false, false, false};
     // Coulomb and host-pointer staging
     int *d_gidx = nullptr;
     unsigned *d_jmap = nullptr;
@@ -1446,6 +1448,7 @@ static void release_graph(DevState *d);
 static void release_plan(DevState *d, int i) {
     release_graph(d);
     free_plan(d->plans[i]);
+    for (bool &n : d->no_pad) n = false;   // another configuration, or room for another width
 }
 
 static void release_plans(DevState *d) {

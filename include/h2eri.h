@@ -395,8 +395,9 @@ void H2ERI_matvec_bytes(H2ERI_p h2eri, double *out6);
  * (1, 2, 4, 8, 16 vectors per pass) may take for its workspace and task lists
  * (additive; 0, the default: what the device has).  A pass that would need
  * more fails as on a full device, except that a batch whose last vectors would
- * run in a wider pass then runs them in narrower ones.  Plans that are there
- * stay. */
+ * run in a wider pass then runs them in narrower ones, until a setter of
+ * the precision, the executor or the tuning releases a plan.  Plans that are
+ * there stay. */
 void H2ERI_set_pass_memory(H2ERI_p h2eri, const double bytes);
 
 /* Tile size of the device bi-GEMV tasks in bytes (tuning; re-plans the

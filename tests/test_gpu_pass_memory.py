@@ -4,7 +4,7 @@ bitwise the same as those passes alone, and a graph captured before stays."""
 import numpy as np
 import pytest
 
-from conftest import make_synthetic, relerr
+from conftest import make_synthetic
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,25 @@ def test_no_room_keeps_the_graph(executor, tmp_path):
     h.graph_replay(torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert torch.equal(y, _run(h, X[:1].contiguous())[0])
+
+
+@pytest.mark.parametrize("freed", ["precision", "tiles"])
+def test_padding_returns_with_room(freed, tmp_path):
+    import torch
+    h = make_synthetic(tmp_path / "s.rep", 900, 72, leaf=30, max_rank=12, lr_frac=0.4, diag_lr_frac=0.3)
+    X = _batch(h, 9)
+    padded = _run(h, X)   # 16 wide: matrix instructions, other roundings than the narrower passes
+    narrow = torch.cat([_run(h, X[:8].contiguous()), _run(h, X[8:].contiguous())])
+    assert not torch.equal(padded, narrow)
+    h.set_tile_bytes(65536)
+    h.set_tile_bytes(131072)   # the plans go
+    h.set_pass_memory(_bound(h))
+    assert torch.equal(_run(h, X), narrow)
+    h.set_pass_memory(0)
+    if freed == "tiles":
+        h.set_tile_bytes(65536)
+        h.set_tile_bytes(131072)
+    else:
+        h.set_precision(32)
+        h.set_precision(64)
+    assert torch.equal(_run(h, X), padded)
