@@ -1414,6 +1414,7 @@ struct DevState {
     int *last_noalloc_ctr = nullptr;   // counters of the last allocation-free persistent pass
     JitState *jit = nullptr;           // a BD_JIT handle's on-the-fly state (jit.hip)
     double pass_bytes = 0;             // bound of one plan's device memory (H2ERI_set_pass_memory; 0: none)
+    bool no_room = false;              // the last plan that could not be made found too little device memory
 };
 
 static DevState *dstate(H2ERI_p h) { return (DevState *)h->dev; }
@@ -2388,6 +2389,7 @@ static bool plan_alloc(DevState *d, DevPlan &dp, void **dst, const void *src, si
     if (bytes == 0) bytes = 64;
     hipError_t e = hipErrorOutOfMemory;
     if (d->pass_bytes <= 0 || (double)(dp.bytes + bytes) <= d->pass_bytes) e = hipMalloc(dst, bytes);
+    d->no_room = e == hipErrorOutOfMemory;
     if (e == hipSuccess) dp.bytes += bytes;
     if (e == hipSuccess && src) e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -2457,15 +2459,17 @@ static DevPlan *get_plan(H2ERI_p h, int nv) {
     return nullptr;
 }
 
-// Plan of the next pass for `rem` vectors left (nv_pass); when a pass wider
-// than that cannot be planned or held (its workspace), the widest of at most
-// `rem` vectors, from then on.
+// Plan of the next pass for `rem` vectors left (nv_pass); when the workspace
+// of a pass wider than that finds no room on the device or exceeds what a plan
+// can address, the widest of at most `rem` vectors, from then on.
 static DevPlan *pass_plan(H2ERI_p h, int rem) {
     const int nv = nv_pass(rem), i = nv_index(nv);
     const bool padded = nv > rem;
     if (!padded || !dstate_get(h)->no_pad[i]) {
+        if (padded) dstate(h)->no_room = false;
         DevPlan *dp = get_plan(h, nv);
         if (dp || !padded || h->BD_JIT || !dstate(h)->st_ready) return dp;
+        if (!dstate(h)->no_room && h2eri_last_error() != ERR_UNSUPPORTED) return nullptr;
         dstate(h)->no_pad[i] = true;
         (void)hipGetLastError();
         h2eri_clear_error();
