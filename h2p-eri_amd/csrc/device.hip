@@ -1387,7 +1387,8 @@ struct DevState {
     unsigned *d_jmap = nullptr;
     double *d_D = nullptr, *d_J = nullptr, *d_y = nullptr, *d_x = nullptr;
     size_t d_io_len = 0, d_dj_len = 0;   // doubles of d_x / d_y, and of d_D / d_J
-    hipStream_t side = nullptr;         // near-field stream (schedule 2)
+    hipStream_t side = nullptr;         // near-field stream while the caller's stream is captured
+    int near_dev = -1;                  // device whose shared near-field streams the handle uses
     hipGraphExec_t graph = nullptr;     // captured hot-path sequence (H2ERI_graph_capture)
     int graph_kind = -1;                // its kind (0 matvec, 1 Coulomb, 2 exchange)
     bool capturing = false;
@@ -1431,6 +1432,56 @@ static DevState *dstate(H2ERI_p h) { return (DevState *)h->dev; }
 
 static void free_dev(void *&p) {
     if (p) { (void)hipFree(p); p = nullptr; }
+}
+
+// Near-field streams of the staged executor, shared by the handles of a
+// device: one per stream that callers pass.  Passes on one caller stream run
+// one after another, so sharing costs them nothing, and passes on different
+// streams do not wait for each other's near field.  A process has four
+// hardware queues and its streams are dealt onto them: with a stream per
+// handle the seventh handle's near field fell onto its caller's queue and ran
+// after the sweeps instead of beside them ((H2O)16 FP32-stored, one J: 148 us
+// on the other handles, 217 on that one; C10H22 148 and 217).  So there are at
+// most NEAR_MAX of them, beside the caller's; further caller streams share.
+// H2ERI_upload makes the default stream's; the last handle gives all back.  A
+// stream under capture belongs to its capture until that ends: passes on a
+// captured stream fork to the handle's own stream (DevState::side).
+static const int NEAR_MAX = 3, NEAR_DEVICES = 64;
+struct NearPool {
+    int users = 0, n = 0;
+    hipStream_t caller[NEAR_MAX], side[NEAR_MAX];
+};
+static std::mutex g_near_mu;
+static NearPool g_near[NEAR_DEVICES];
+
+static void near_release(DevState *d) {
+    if (d->near_dev < 0) return;
+    std::lock_guard<std::mutex> lk(g_near_mu);
+    NearPool &p = g_near[d->near_dev];
+    d->near_dev = -1;
+    if (--p.users > 0) return;
+    for (int i = 0; i < p.n; i++) (void)hipStreamDestroy(p.side[i]);
+    p.n = 0;
+}
+
+// The near-field stream for passes on caller stream s; without `create` one
+// that is there, if any.
+static bool near_stream(DevState *d, hipStream_t s, bool create, hipStream_t &out) {
+    if (d->near_dev != d->dev) near_release(d);
+    if (d->dev < 0 || d->dev >= NEAR_DEVICES) { set_error(ERR_DEVICE, "near-field stream: device %d", d->dev); return false; }
+    std::lock_guard<std::mutex> lk(g_near_mu);
+    NearPool &p = g_near[d->dev];
+    if (d->near_dev < 0) { p.users++; d->near_dev = d->dev; }
+    for (int i = 0; i < p.n; i++)
+        if (p.caller[i] == s) { out = p.side[i]; return true; }
+    if (p.n < NEAR_MAX && (create || p.n == 0)) {
+        HIP_OK(hipStreamCreateWithFlags(&p.side[p.n], hipStreamNonBlocking));
+        p.caller[p.n++] = s;
+        out = p.side[p.n - 1];
+        return true;
+    }
+    out = p.side[((uintptr_t)s >> 6) % p.n];
+    return true;
 }
 
 // Device memory of a plan; of one that a graph may refer to, release_plan.
@@ -1486,6 +1537,7 @@ void device_release(H2ERI_p h) {
     if (d->ev_join) (void)hipEventDestroy(d->ev_join);
     if (d->ev_base) (void)hipEventDestroy(d->ev_base);
     if (d->side) (void)hipStreamDestroy(d->side);
+    near_release(d);
     delete d;
     h->dev = nullptr;
 }
@@ -2597,14 +2649,22 @@ static bool run_matvec(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, dou
     if (has_side) {
         // near-field launches on their own stream, forked after everything
         // already enqueued on s and joined before the gather
-        if (!d->side) HIP_OK(hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking));
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (s && hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+        hipStream_t side = nullptr;
+        if (cap != hipStreamCaptureStatusNone) {
+            if (!d->side) HIP_OK(hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking));
+            side = d->side;
+        } else if (!near_stream(d, s, !d->ws_Wv, side)) {
+            return false;
+        }
         if (!d->ev_fork) HIP_OK(hipEventCreateWithFlags(&d->ev_fork, hipEventDisableTiming));
         if (!d->ev_join) HIP_OK(hipEventCreateWithFlags(&d->ev_join, hipEventDisableTiming));
         HIP_OK(hipEventRecord(d->ev_fork, s));
-        HIP_OK(hipStreamWaitEvent(d->side, d->ev_fork, 0));
+        HIP_OK(hipStreamWaitEvent(side, d->ev_fork, 0));
         for (const Stage &st : P.stages)
-            if (st.stream == 1 && !launch(st, d->side)) return false;
-        HIP_OK(hipEventRecord(d->ev_join, d->side));
+            if (st.stream == 1 && !launch(st, side)) return false;
+        HIP_OK(hipEventRecord(d->ev_join, side));
     }
     for (const Stage &st : P.stages) {
         if (st.stream != 0) continue;
@@ -3018,6 +3078,8 @@ size_t H2ERI_upload(H2ERI_p h) {
     DevState *d = dstate(h);
     // everything a single-vector pass needs besides its vectors, so that the
     // allocation-free entry point finds it in place
+    hipStream_t near;
+    if (!near_stream(d, nullptr, true, near)) return 0;
     if (!d->side && hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking) != hipSuccess) { set_error(ERR_DEVICE, "stream"); return 0; }
     if (!d->ev_fork && hipEventCreateWithFlags(&d->ev_fork, hipEventDisableTiming) != hipSuccess) { set_error(ERR_DEVICE, "event"); return 0; }
     if (!d->ev_join && hipEventCreateWithFlags(&d->ev_join, hipEventDisableTiming) != hipSuccess) { set_error(ERR_DEVICE, "event"); return 0; }
