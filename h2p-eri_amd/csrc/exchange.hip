@@ -520,9 +520,12 @@ struct KPlan {
     std::vector<KGemmTask> gtasks;
     long long nSC = 0;      // L / R products (computed once)
     int nacc = 1;           // copies of the K accumulators
-    int mmax = 1, nmax = 1; // most functions m of a split, and of a node
+    int mmax = 1, nmax = 1, smax = 1;   // of the row nodes of block terms: most functions m of a split, functions, splits
     bool wide = false;      // 64-bit offsets (kx_block)
     double flops = 0;
+    // LDS of a block task: G tile, K block and, in the 32-bit form, the row
+    // node's functions
+    size_t block_lds() const { return (size_t)(KGT + (mmax + 1) * KQ) * 8 + (wide ? 0 : (size_t)nmax * 4); }
 };
 
 // Default bound of the K accumulators (bytes): workgroups add into one of
@@ -843,8 +846,6 @@ struct KBuilder {
         P.bptr.push_back((int)P.brow.size() / 16);
         // a step of n costs a wave about four MFMAs per bra block
         column_pairs(kn, bfs, byq, 4.0 * nblk / (8.0 * kn.nsplit * ((nb + 15) / 16)));
-        P.mmax = std::max(P.mmax, kn.ssz);
-        P.nmax = std::max(P.nmax, nb);
         P.nodes.push_back(kn);
         node_list[node] = (int)P.nodes.size() - 1;
         return node_list[node];
@@ -958,6 +959,9 @@ struct KBuilder {
                 for (long long e0 = 0; e0 < ne; e0 += KWG / 64) P.direct.push_back(KTask{ti, (int)e0, 0, 0});
                 continue;
             }
+            P.mmax = std::max(P.mmax, ni.ssz);
+            P.nmax = std::max(P.nmax, ni.nbf);
+            P.smax = std::max(P.smax, ni.nsplit);
             const double reach = std::max({(double)t.m1 * t.Rrs + (double)t.kk * t.Rcs, (double)t.m0 * t.Lld + t.kk + KPAD,
                                            (double)h->num_bf * h->num_bf});
             if (reach * 8.0 >= 4294967296.0 || ni.nbf > 4096 || t.m0 >= 1 << 24 || t.Lld >= 1 << 21) P.wide = true;
@@ -1128,7 +1132,7 @@ static bool k_upload(H2ERI_p h) {
         !up((void **)&k->direct, P.direct.empty() ? nullptr : P.direct.data(), P.direct.size() * sizeof(KTask)) ||
         !up((void **)&k->gtasks, P.gtasks.empty() ? nullptr : P.gtasks.data(), P.gtasks.size() * sizeof(KGemmTask)))
         return false;
-    const int lds = (KGT + (P.mmax + 1) * KQ) * 8 + (P.wide ? 0 : P.nmax * 4);   // G tile, K block, functions
+    const int lds = (int)P.block_lds();
     for (const void *f : {reinterpret_cast<const void *>(&kx_block<unsigned>), reinterpret_cast<const void *>(&kx_block<unsigned long long>)})
         KHIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     // (zeros also between the products, whose rows end where the next begins)
@@ -1155,13 +1159,11 @@ static bool k_run(H2ERI_p h, const double *D_dev, double *K_dev, hipStream_t s) 
     D_dev = k->Ds;
     hipLaunchKernelGGL(kx_zero, dim3(zb), dim3(256), 0, s, k->KA, nn2 * 2 * P.nacc);
     KHIP(hipGetLastError());
-    // the blocks add into the accumulators with atomics; the K block's LDS is
-    // that of the largest split
+    // the blocks add into the accumulators with atomics
     if (!P.block.empty())
         hipLaunchKernelGGL(P.wide ? kx_block<unsigned long long> : kx_block<unsigned>, dim3((unsigned)P.block.size()), dim3(KBWG),
-                           (size_t)(KGT + (P.mmax + 1) * KQ) * 8 + (size_t)(P.wide ? 0 : P.nmax * 4), s, k->block, k->terms,
-                           k->nodes, k->bfidx, k->gptr, k->ge, k->bptr, k->brow, k->PB, k->CB, k->SC, D_dev, k->KA,
-                           P.nacc, nbf);
+                           P.block_lds(), s, k->block, k->terms, k->nodes, k->bfidx, k->gptr, k->ge, k->bptr, k->brow,
+                           k->PB, k->CB, k->SC, D_dev, k->KA, P.nacc, nbf);
     if (!P.direct.empty())
         hipLaunchKernelGGL(kx_direct, dim3((unsigned)P.direct.size()), dim3(KWG), 0, s, k->direct, k->terms, k->nodes,
                            k->bfidx, k->qptr, k->qent, k->mptr, k->ment, k->CB, D_dev, k->KA, nbf);
@@ -1264,6 +1266,21 @@ int H2ERI_exchange_plan_check(H2ERI_p h, double *out4) {
         out4[3] = (double)P.nSC + nacc;
     }
     return (int)P.terms.size();
+}
+
+// Shape of the block tasks (host only, tests): out4 = {LDS bytes of a
+// workgroup, most functions of a row node of a block term, most splits of one,
+// 1 when operand offsets take 64 bits}.  Returns 0, -1 on failure.
+int H2ERI_exchange_plan_shape(H2ERI_p h, double *out4) {
+    if (!h || !out4 || !h->U || !h->c_B_blks || !h->c_D_blks) { set_error(ERR_ARG, "exchange_plan_shape: nothing built"); return -1; }
+    KPlan P;
+    KBuilder b(h, P, kstate(h) ? kstate(h)->budget : KACC_BUDGET_DEFAULT);
+    if (!b.build()) return -1;
+    out4[0] = (double)P.block_lds();
+    out4[1] = P.nmax;
+    out4[2] = P.smax;
+    out4[3] = P.wide ? 1.0 : 0.0;
+    return 0;
 }
 
 // Work figures of the exchange plan: out4 = {GEMM flops at upload, terms,

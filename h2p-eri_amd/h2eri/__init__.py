@@ -440,6 +440,13 @@ class H2ERI:
         _check(self.lib)
         return dict(terms=n, **dict(zip(["gemm_flops", "terms_f", "resident_bytes", "scratch_doubles"], out.tolist())))
 
+    def exchange_plan_shape(self):
+        """Shape of the exchange build's block tasks (host only, tests)."""
+        out = np.zeros(4)
+        self.lib.H2ERI_exchange_plan_shape(self.h, _dptr(out))
+        _check(self.lib)
+        return dict(zip(["lds_bytes", "functions", "splits", "wide"], [int(v) for v in out]))
+
     def autotune(self, nv=1, reps=10):
         """Times executors x tile sizes x near-field schedules on the device,
         keeps the best."""

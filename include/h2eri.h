@@ -272,6 +272,11 @@ void H2ERI_set_exchange_scratch(H2ERI_p h2eri, const double bytes);
  * HIP call); out4 as above with out4[2] the bytes it would make resident.
  * Returns the number of block terms, -1 on failure. */
 int H2ERI_exchange_plan_check(H2ERI_p h2eri, double *out4);
+/* Additive (host only, tests): the shape of the exchange build's block tasks:
+ * out4 = {LDS bytes of a workgroup, most functions of a row node of a block
+ * term, most splits of one, 1 when operand offsets take 64 bits}.  0, -1 on
+ * failure. */
+int H2ERI_exchange_plan_shape(H2ERI_p h2eri, double *out4);
 
 /* ------------------------------------------------------------------ */
 /* Additive entry points (no counterpart in the reference).             */
