@@ -119,6 +119,10 @@ static const int KPAD = 32;     // readable doubles past every operand array
 // functions of a larger node are cut into even splits, each of which forms
 // its G again.
 static const int KM = 352;
+static const int KNMAX = 4096;  // most functions of a row node whose list is in LDS (the 32-bit form)
+// LDS of a block task: G tile, K block and, in the 32-bit form, the row node's
+// functions
+static size_t kblock_lds(int m, int n, bool wide) { return (size_t)(KGT + (m + 1) * KQ) * 8 + (wide ? 0 : (size_t)n * 4); }
 // A bra entry: row r, and the byte of m's row in the K block (16 bits; the row
 // past the last is a sink for rows of a block without an entry) under local n
 // (4 bits) and flags of the block.
@@ -523,9 +527,7 @@ struct KPlan {
     int mmax = 1, nmax = 1, smax = 1;   // of the row nodes of block terms: most functions m of a split, functions, splits
     bool wide = false;      // 64-bit offsets (kx_block)
     double flops = 0;
-    // LDS of a block task: G tile, K block and, in the 32-bit form, the row
-    // node's functions
-    size_t block_lds() const { return (size_t)(KGT + (mmax + 1) * KQ) * 8 + (wide ? 0 : (size_t)nmax * 4); }
+    size_t block_lds() const { return kblock_lds(mmax, nmax, wide); }
 };
 
 // Default bound of the K accumulators (bytes): workgroups add into one of
@@ -964,7 +966,7 @@ struct KBuilder {
             P.smax = std::max(P.smax, ni.nsplit);
             const double reach = std::max({(double)t.m1 * t.Rrs + (double)t.kk * t.Rcs, (double)t.m0 * t.Lld + t.kk + KPAD,
                                            (double)h->num_bf * h->num_bf});
-            if (reach * 8.0 >= 4294967296.0 || ni.nbf > 4096 || t.m0 >= 1 << 24 || t.Lld >= 1 << 21) P.wide = true;
+            if (reach * 8.0 >= 4294967296.0 || ni.nbf > KNMAX || t.m0 >= 1 << 24 || t.Lld >= 1 << 21) P.wide = true;
             const double steps = (double)((ni.nbf + 15) / 16) * ((t.kk + 15) / 16);
             order.push_back({steps * (4.0 + (double)t.m1 / nj.nbf + (double)t.m0 / ni.nbf), ti});
         }
@@ -1132,9 +1134,9 @@ static bool k_upload(H2ERI_p h) {
         !up((void **)&k->direct, P.direct.empty() ? nullptr : P.direct.data(), P.direct.size() * sizeof(KTask)) ||
         !up((void **)&k->gtasks, P.gtasks.empty() ? nullptr : P.gtasks.data(), P.gtasks.size() * sizeof(KGemmTask)))
         return false;
-    const int lds = (int)P.block_lds();
+    // one limit for the process: the most any plan asks for, not this one's
     for (const void *f : {reinterpret_cast<const void *>(&kx_block<unsigned>), reinterpret_cast<const void *>(&kx_block<unsigned long long>)})
-        KHIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        KHIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kblock_lds(KM, KNMAX, false)));
     // (zeros also between the products, whose rows end where the next begins)
     KHIP(hipMemset(k->SC, 0, ((size_t)P.nSC + KPAD) * 8));
     // L / R products do not depend on D: computed once at upload
