@@ -541,6 +541,7 @@ struct KState {
     KPlan P;
     bool ready = false;
     double budget = KACC_BUDGET_DEFAULT;   // bytes of the accumulators (H2ERI_set_exchange_scratch)
+    bool wide = false;      // 64-bit offsets whatever the sizes (H2ERI_set_exchange_wide)
     double *PB = nullptr, *CB = nullptr, *SC = nullptr, *KA = nullptr, *D = nullptr, *K = nullptr;
     double *Ds = nullptr;   // the density after screening (the kernels' D)
     int *sbf = nullptr;     // shell_bf_sidx
@@ -580,7 +581,8 @@ struct KBuilder {
     std::vector<long long> pb_off;   // expanded basis of each tree node in PB (-1: none)
     std::vector<int> node_list;      // tree node -> KNode id (-1: not built)
 
-    KBuilder(H2ERI_p h_, KPlan &p_, double budget_) : h(h_), P(p_), budget(budget_) {}
+    KBuilder(H2ERI_p h_, KPlan &p_, const KState *k)
+        : h(h_), P(p_), budget(k ? k->budget : KACC_BUDGET_DEFAULT) { P.wide = k && k->wide; }
 
     int rank_of(int n) const { return h->U[n] ? h->U[n]->ncol : 0; }
     int rows_of(int n) const { return h->mat_cluster[2 * n + 1] - h->mat_cluster[2 * n] + 1; }
@@ -1097,9 +1099,8 @@ static bool k_upload(H2ERI_p h) {
     if (!h->thread_Kmat_workbuf) h->thread_Kmat_workbuf = (void **)new KState();
     KState *k = kstate(h);
     if (k->ready) return true;
-    const double budget = k->budget;
     kstate_release(k);
-    KBuilder b(h, k->P, budget);
+    KBuilder b(h, k->P, k);
     if (!b.build()) return false;
     const KPlan &P = k->P;
     const int nbf = h->num_bf;
@@ -1255,7 +1256,7 @@ void H2ERI_exchange_workbuf_free(H2ERI_p h) {
 int H2ERI_exchange_plan_check(H2ERI_p h, double *out4) {
     if (!h || !h->U || !h->c_B_blks || !h->c_D_blks) { set_error(ERR_ARG, "exchange_plan_check: nothing built"); return -1; }
     KPlan P;
-    KBuilder b(h, P, kstate(h) ? kstate(h)->budget : KACC_BUDGET_DEFAULT);
+    KBuilder b(h, P, kstate(h));
     if (!b.build()) return -1;
     if (out4) {
         const double nn2 = (double)h->num_bf * h->num_bf;
@@ -1276,7 +1277,7 @@ int H2ERI_exchange_plan_check(H2ERI_p h, double *out4) {
 int H2ERI_exchange_plan_shape(H2ERI_p h, double *out4) {
     if (!h || !out4 || !h->U || !h->c_B_blks || !h->c_D_blks) { set_error(ERR_ARG, "exchange_plan_shape: nothing built"); return -1; }
     KPlan P;
-    KBuilder b(h, P, kstate(h) ? kstate(h)->budget : KACC_BUDGET_DEFAULT);
+    KBuilder b(h, P, kstate(h));
     if (!b.build()) return -1;
     out4[0] = (double)P.block_lds();
     out4[1] = P.nmax;
@@ -1307,6 +1308,18 @@ void H2ERI_set_exchange_scratch(H2ERI_p h, const double bytes) {
     device_release_graph_kind(h, 2);
     kstate_release(k);
     k->budget = bytes;
+}
+
+// The block kernel's 64-bit form for every size (on = 1; tests): plans take it
+// by themselves where offsets need it.  Releases the exchange plan.
+void H2ERI_set_exchange_wide(H2ERI_p h, const int on) {
+    if (!h) { set_error(ERR_ARG, "H2ERI_set_exchange_wide: null handle"); return; }
+    if (!h->thread_Kmat_workbuf) h->thread_Kmat_workbuf = (void **)new KState();
+    KState *k = kstate(h);
+    if (k->wide == (on != 0)) return;
+    device_release_graph_kind(h, 2);
+    kstate_release(k);
+    k->wide = on != 0;
 }
 
 }  // extern "C"

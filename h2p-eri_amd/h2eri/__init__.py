@@ -427,6 +427,11 @@ class H2ERI:
         self.lib.H2ERI_set_exchange_scratch(self.h, float(nbytes))
         _check(self.lib)
 
+    def set_exchange_wide(self, on):
+        """The exchange build's 64-bit operand offsets for every size (tests)."""
+        self.lib.H2ERI_set_exchange_wide(self.h, 1 if on else 0)
+        _check(self.lib)
+
     def exchange_stats(self):
         out = np.zeros(4)
         self.lib.H2ERI_exchange_stats(self.h, _dptr(out))

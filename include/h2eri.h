@@ -268,6 +268,11 @@ void H2ERI_exchange_stats(H2ERI_p h2eri, double *out4);
  * at least one copy whatever the bound.  Releases the exchange plan and an
  * exchange graph. */
 void H2ERI_set_exchange_scratch(H2ERI_p h2eri, const double bytes);
+/* Additive (tests): the block kernel's form with 64-bit operand offsets for
+ * every size (on = 1); the default (0) takes it where an operand array or D
+ * reaches 4 GB or a node exceeds the 32-bit form's lists.  Releases the
+ * exchange plan and an exchange graph. */
+void H2ERI_set_exchange_wide(H2ERI_p h2eri, const int on);
 /* Additive: the exchange plan built and bounds-checked on the host only (no
  * HIP call); out4 as above with out4[2] the bytes it would make resident.
  * Returns the number of block terms, -1 on failure. */
