@@ -105,13 +105,20 @@ __device__ __forceinline__ RTask uniform(const RTask &a) {
     return t;
 }
 
-// The pass's external vectors: vector v at v * ld, n of them (the pass is NV
-// wide; the others read as zero and are not written).  ld < 0: an
+// The external vectors of a padded pass (fewer vectors than its width NV):
+// vector v at v * ld, n of them; the others read as zero and are not written.
+// A full pass takes the bare stride: the tests of v < n in it cost 2 to 4% of
+// an 8-vector pass ((H2O)32 staged, FP64: 705 us in place of 663) and 28 more
+// spilled SGPRs in its persistent kernel.  A stride below zero: an
 // element-major copy.
 struct ExtLd {
     long long ld;
     int n;
 };
+__host__ __device__ __forceinline__ long long ext_ld(long long ld) { return ld; }
+__host__ __device__ __forceinline__ long long ext_ld(const ExtLd &e) { return e.ld; }
+__device__ __forceinline__ bool ext_has(long long, int) { return true; }
+__device__ __forceinline__ bool ext_has(const ExtLd &e, int v) { return v < e.n; }
 
 static const int WG = 256;       // threads per workgroup (4 waves)
 // Output elements per reduce task: 1024 / NV values fill the task's 256
@@ -167,14 +174,14 @@ __device__ __forceinline__ void wst(double *p, double v) {
 // threads take values q = tid, tid + WG, ... (contiguous in its
 // NV-interleaved layout), so every thread works for any NV, and each sums
 // the slots in list order with eight loads in flight.  From the external
-// input the threads take elements and read the first ldx.n vectors (a pass
-// wider than the vectors left has zeros in the others).
-template <int NV, bool COH, int NT, int XS = NV>
+// input the threads take elements and read the pass's vectors (zeros beyond
+// the last).
+template <int NV, bool COH, int NT, int XS = NV, typename LD>
 __device__ __forceinline__ void stage_vec(const int *__restrict__ vsrc, int b, int e, int off, int n,
-                                          const double *__restrict__ Wv, const double *__restrict__ X, ExtLd ldx,
+                                          const double *__restrict__ Wv, const double *__restrict__ X, LD ldx,
                                           double *dst, int tid) {
     const int s0 = vsrc[b];
-    if (s0 < 0 && ldx.ld < 0) {   // the external input as an element-major copy (NV values per element)
+    if (s0 < 0 && ext_ld(ldx) < 0) {   // the external input as an element-major copy (NV values per element)
         const double *p = X + (long long)(-s0 - 1 + off) * NV;
         for (int q = tid; q < n * NV; q += NT) dst[XS == NV ? q : (q / NV) * XS + q % NV] = p[q];
         return;
@@ -183,7 +190,7 @@ __device__ __forceinline__ void stage_vec(const int *__restrict__ vsrc, int b, i
         const double *p = X + (long long)(-s0 - 1 + off);
         for (int i = tid; i < n; i += NT) {
             #pragma unroll
-            for (int v = 0; v < NV; v++) dst[i * XS + v] = NV == 1 || v < ldx.n ? p[v * ldx.ld + i] : 0.0;
+            for (int v = 0; v < NV; v++) dst[i * XS + v] = ext_has(ldx, v) ? p[v * ext_ld(ldx) + i] : 0.0;
         }
         return;
     }
@@ -404,9 +411,9 @@ __device__ void coldot_tile(const BTask &t, const T *__restrict__ S, double *__r
 // step (RW).
 template <typename T> struct Dot8 { static const int RC = 4, XS = 10, RW = 4; };
 
-template <typename T, int NV, bool COH, int NT = WG>
+template <typename T, int NV, bool COH, int NT = WG, typename LD>
 __device__ void bgemv_tile_valu(const BTask &task, const T *__restrict__ S, const int *__restrict__ vsrc,
-                                double *__restrict__ Wv, const double *__restrict__ X, ExtLd ldx, double *lds) {
+                                double *__restrict__ Wv, const double *__restrict__ X, LD ldx, double *lds) {
     // At NV = 8 the descriptor stays as loaded: the register allocation of
     // the two tile paths together fits 128 VGPRs only that way (measured on
     // the compiler's output), and the path choice is made uniform below.
@@ -707,7 +714,9 @@ __device__ __forceinline__ double in16_get(const In16 &in, int i, int v, const d
 // Each wave keeps its column sums in registers, one accumulator per group of
 // 16 columns, until the end of the tile; then the four waves add them in LDS
 // in a fixed order.
-template <typename T, bool COH>
+// (LD tells the kernels' copies apart: shared by two persistent kernels the
+// function is called, not inlined, and a pass takes 1.4 times as long.)
+template <typename T, bool COH, typename LD>
 __device__ void mfma_tile16_2s(const BTask &t, const T *__restrict__ base, const int *__restrict__ vsrc,
                                double *__restrict__ Wv, const double *__restrict__ Xt, double *lds) {
     constexpr int NV = 16;
@@ -719,7 +728,7 @@ __device__ void mfma_tile16_2s(const BTask &t, const T *__restrict__ base, const
     const int Cp = (C + 15) & ~15, ng = Cp >> 4;   // groups of 16 columns, at most 4
     double *xin = lds;                                // Cp x 16, zero past C
     double *tr = lds + T16_MAXC * NV + 256 * w;       // this wave's 16 x 16 transposition tile
-    stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, ExtLd{-1, 16}, xin, tid);
+    stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, -1LL, xin, tid);
     for (int q = C * NV + tid; q < Cp * NV; q += WG) xin[q] = 0.0;
     __syncthreads();
     const In16 y = in16_make(vsrc, t.v1b, t.v1e, t.v1off);
@@ -772,7 +781,7 @@ __device__ void mfma_tile16_2s(const BTask &t, const T *__restrict__ base, const
     }
 }
 
-template <typename T, bool COH>
+template <typename T, bool COH, typename LD>
 __device__ void mfma_tile16(const BTask &task, const T *__restrict__ S, const int *__restrict__ vsrc,
                             double *__restrict__ Wv, const double *__restrict__ Xt, double *lds) {
     constexpr int NV = 16;
@@ -783,7 +792,7 @@ __device__ void mfma_tile16(const BTask &task, const T *__restrict__ S, const in
     const int R = t.nrow, C = t.ncol;
     const bool do0 = t.out0 >= 0, do1 = t.out1 >= 0;
     const T *base = S + t.mat;
-    if (do0 && do1) { mfma_tile16_2s<T, COH>(t, base, vsrc, Wv, Xt, lds); return; }
+    if (do0 && do1) { mfma_tile16_2s<T, COH, LD>(t, base, vsrc, Wv, Xt, lds); return; }
     const int cmax = ((C - 1) / VW) * VW;
     // inputs staged in LDS (their slots summed once) when they fit beside
     // each other, padded with zeros to whole groups of 16; otherwise (a row
@@ -794,11 +803,11 @@ __device__ void mfma_tile16(const BTask &task, const T *__restrict__ S, const in
     double *xin = lds;
     double *yin = lds + (st0 ? Cp * NV : 0);
     if (st0) {
-        stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, ExtLd{-1, 16}, xin, tid);
+        stage_vec<NV, COH, WG>(vsrc, t.v0b, t.v0e, t.v0off, C, Wv, Xt, -1LL, xin, tid);
         for (int q = C * NV + tid; q < Cp * NV; q += WG) xin[q] = 0.0;
     }
     if (do1) {
-        stage_vec<NV, COH, WG>(vsrc, t.v1b, t.v1e, t.v1off, R, Wv, Xt, ExtLd{-1, 16}, yin, tid);
+        stage_vec<NV, COH, WG>(vsrc, t.v1b, t.v1e, t.v1off, R, Wv, Xt, -1LL, yin, tid);
         for (int q = R * NV + tid; q < Rp * NV; q += WG) yin[q] = 0.0;
     }
     __syncthreads();
@@ -880,14 +889,14 @@ __device__ void mfma_tile16(const BTask &task, const T *__restrict__ S, const in
 }
 
 // A tile task: the MFMA products at 16 vectors per pass, the VALU tile below.
-template <typename T, int NV, bool COH, int NT = WG>
+template <typename T, int NV, bool COH, int NT = WG, typename LD>
 __device__ __forceinline__ void bgemv_tile(const BTask &task, const T *__restrict__ S, const int *__restrict__ vsrc,
-                                           double *__restrict__ Wv, const double *__restrict__ X, ExtLd ldx,
+                                           double *__restrict__ Wv, const double *__restrict__ X, LD ldx,
                                            double *lds) {
     if constexpr (NV == 16) {
         // X is the element-major copy of the input (the pass's first launch
         // makes it); no wave tiles at 16
-        if constexpr (NT == WG) mfma_tile16<T, COH>(task, S, vsrc, Wv, X, lds);
+        if constexpr (NT == WG) mfma_tile16<T, COH, LD>(task, S, vsrc, Wv, X, lds);
     } else {
         bgemv_tile_valu<T, NV, COH, NT>(task, S, vsrc, Wv, X, ldx, lds);
     }
@@ -898,9 +907,9 @@ __device__ __forceinline__ void bgemv_tile(const BTask &task, const T *__restric
 // group g sums sources g, g + K, ... in order, each thread up to four values
 // with all their loads of four sources in flight; the group sums are added
 // as (g0 + g1) + (g2 + g3), or g0 + g1.
-template <int NV, bool COH>
+template <int NV, bool COH, typename LD>
 __device__ void reduce_task(const RTask &task, const int *__restrict__ src, double *__restrict__ Wv,
-                            double *__restrict__ Y, ExtLd ldy, double *lds) {
+                            double *__restrict__ Y, LD ldy, double *lds) {
     const RTask t = uniform(task);
     const int n = t.len * NV;
     const int K = n <= 64 ? 4 : (n <= 128 ? 2 : 1);
@@ -933,7 +942,7 @@ __device__ void reduce_task(const RTask &task, const int *__restrict__ src, doub
     auto put = [&](int q, double v) {
         if (t.flags & 1) {
             const int i = q / NV, w = q - i * NV;
-            if (NV == 1 || w < ldy.n) Y[w * ldy.ld + t.dst + i] = v;
+            if (ext_has(ldy, w)) Y[w * ext_ld(ldy) + t.dst + i] = v;
         } else {
             wst<COH>(Wv + t.dst * NV + q, v);
         }
@@ -964,14 +973,14 @@ template <int NV> constexpr int waves_per_simd() { return 4; }
 
 // Task b of a staged launch: tiles (FP64, FP32), reduce tasks, then groups of
 // four wave tiles.
-template <int NV>
+template <int NV, typename LD>
 __device__ __forceinline__ void stage_task(int b, const BTask *__restrict__ t64, int n64, const BTask *__restrict__ t32,
                                            int n32, const RTask *__restrict__ rt, int nr, const BTask *__restrict__ w64,
                                            int nw64, const BTask *__restrict__ w32, int nw32,
                                            const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                            const double *__restrict__ S64, const float *__restrict__ S32,
                                            double *__restrict__ Wv, const double *__restrict__ X,
-                                           double *__restrict__ Y, ExtLd ldx, double *lds) {
+                                           double *__restrict__ Y, LD ldx, double *lds) {
     if (b < n64) {
         const BTask t = t64[b];
         bgemv_tile<double, NV, false>(t, S64, vsrc, Wv, X, ldx, lds);
@@ -997,14 +1006,14 @@ __device__ __forceinline__ void stage_task(int b, const BTask *__restrict__ t64,
 }
 
 // One launch per stage: one task per workgroup.
-template <int NV>
+template <int NV, typename LD>
 __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void stage_kernel(const BTask *__restrict__ t64, int n64, const BTask *__restrict__ t32,
                                                    int n32, const RTask *__restrict__ rt, int nr,
                                                    const BTask *__restrict__ w64, int nw64, const BTask *__restrict__ w32,
                                                    int nw32, const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                                    const double *__restrict__ S64, const float *__restrict__ S32,
                                                    double *__restrict__ Wv, const double *__restrict__ X,
-                                                   double *__restrict__ Y, ExtLd ldx) {
+                                                   double *__restrict__ Y, LD ldx) {
     __shared__ double lds[LDS_DOUBLES];
     stage_task<NV>(blockIdx.x, t64, n64, t32, n32, rt, nr, w64, nw64, w32, nw32, vsrc, rsrc, S64, S32, Wv, X, Y, ldx,
                    lds);
@@ -1013,14 +1022,14 @@ __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void stage_kernel(const B
 // A near-field launch with fewer workgroups than tasks (the sweeps' launches
 // on the other stream keep CUs of their own): workgroup g takes tasks
 // g, g + gridDim.x, ...
-template <int NV>
+template <int NV, typename LD>
 __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void stage_loop_kernel(const BTask *__restrict__ t64, int n64, const BTask *__restrict__ t32,
                                                         int n32, const RTask *__restrict__ rt, int nr,
                                                         const BTask *__restrict__ w64, int nw64, const BTask *__restrict__ w32,
                                                         int nw32, const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                                         const double *__restrict__ S64, const float *__restrict__ S32,
                                                         double *__restrict__ Wv, const double *__restrict__ X,
-                                                        double *__restrict__ Y, ExtLd ldx) {
+                                                        double *__restrict__ Y, LD ldx) {
     __shared__ double lds[LDS_DOUBLES];
     const int total = n64 + n32 + nr + (nw64 + 3) / 4 + (nw32 + 3) / 4;
     for (int b = blockIdx.x; b < total; b += gridDim.x) {
@@ -1095,7 +1104,7 @@ __device__ __forceinline__ void wait_vm_stores() { __builtin_amdgcn_s_waitcnt(0x
 
 // GROUP = false: one representation, pointers from the arguments; GROUP =
 // true: QTask::pad_[0] names the molecule whose pointers come from mols.
-template <int NV, bool GROUP>
+template <int NV, bool GROUP, typename LD>
 __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void queue_kernel(const QTask *__restrict__ tasks, int ntask,
                                                       const int *__restrict__ need, int *ctr, int spin_limit,
                                                       const MolPtrs *__restrict__ mols, const BTask *__restrict__ t64,
@@ -1103,7 +1112,7 @@ __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void queue_kernel(const Q
                                                       const int *__restrict__ vsrc, const int *__restrict__ rsrc,
                                                       const double *__restrict__ S64, const float *__restrict__ S32,
                                                       double *__restrict__ Wv, const double *__restrict__ X,
-                                                      double *__restrict__ Y, ExtLd ldx) {
+                                                      double *__restrict__ Y, LD ldx) {
     __shared__ double lds[LDS_DOUBLES];
     __shared__ int s_next[2];
     if (threadIdx.x == 0) s_next[0] = __hip_atomic_fetch_add(ctr + QC_TICKET, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1127,9 +1136,9 @@ __global__ __launch_bounds__(WG, waves_per_simd<NV>()) void queue_kernel(const Q
             __syncthreads();
             if constexpr (GROUP) {
                 const MolPtrs m = mols[q.pad_[0]];
-                if (q.kind == 0) bgemv_tile<double, NV, true>(m.t64[q.idx], m.S64, m.vsrc, m.Wv, m.X, ExtLd{m.ldx, 1}, lds);
-                else if (q.kind == 1) bgemv_tile<float, NV, true>(m.t32[q.idx], m.S32, m.vsrc, m.Wv, m.X, ExtLd{m.ldx, 1}, lds);
-                else reduce_task<NV, true>(m.rt[q.idx], m.rsrc, m.Wv, m.Y, ExtLd{m.ldx, 1}, lds);
+                if (q.kind == 0) bgemv_tile<double, NV, true>(m.t64[q.idx], m.S64, m.vsrc, m.Wv, m.X, m.ldx, lds);
+                else if (q.kind == 1) bgemv_tile<float, NV, true>(m.t32[q.idx], m.S32, m.vsrc, m.Wv, m.X, m.ldx, lds);
+                else reduce_task<NV, true>(m.rt[q.idx], m.rsrc, m.Wv, m.Y, m.ldx, lds);
             } else {
                 if (q.kind == 0) bgemv_tile<double, NV, true>(t64[q.idx], S64, vsrc, Wv, X, ldx, lds);
                 else if (q.kind == 1) bgemv_tile<float, NV, true>(t32[q.idx], S32, vsrc, Wv, X, ldx, lds);
@@ -2427,11 +2436,11 @@ static int queue_grid(int nv) {
         return 0;
     hipError_t e;
     switch (nv) {
-    case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<1, false>, WG, 0); break;
-    case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<2, false>, WG, 0); break;
-    case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<4, false>, WG, 0); break;
-    case 8: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<8, false>, WG, 0); break;
-    default: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<16, false>, WG, 0); break;
+    case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<1, false, long long>, WG, 0); break;
+    case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<2, false, long long>, WG, 0); break;
+    case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<4, false, long long>, WG, 0); break;
+    case 8: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<8, false, long long>, WG, 0); break;
+    default: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<16, false, long long>, WG, 0); break;
     }
     return e == hipSuccess ? ncu * std::max(per, 1) : 0;
 }
@@ -2547,14 +2556,21 @@ static inline int launch_blocks(const Stage &st, const DevState *d, int nv) {
     return (st.stream == 1 && cap > 0) ? std::min(nb, cap) : nb;
 }
 
-template <int NV>
-static void launch_stage(const Stage &st, const DevPlan &dp, DevState *d, const double *X, double *Y, ExtLd ld,
-                         hipStream_t s) {
+template <int NV, typename LD>
+static void launch_stage_ld(const Stage &st, const DevPlan &dp, DevState *d, const double *X, double *Y, LD ld, hipStream_t s) {
     const int nb = stage_blocks(st), grid = launch_blocks(st, d, NV);
-    hipLaunchKernelGGL(grid < nb ? stage_loop_kernel<NV> : stage_kernel<NV>, dim3(grid), dim3(WG), 0, s,
+    hipLaunchKernelGGL((grid < nb ? stage_loop_kernel<NV, LD> : stage_kernel<NV, LD>), dim3(grid), dim3(WG), 0, s,
                        dp.d_t64 + st.t64_beg, st.t64_cnt, dp.d_t32 + st.t32_beg, st.t32_cnt, dp.d_rt + st.r_beg,
                        st.r_cnt, dp.d_w64 + st.w64_beg, st.w64_cnt, dp.d_w32 + st.w32_beg, st.w32_cnt, dp.d_vsrc,
                        dp.d_rsrc, d->S64, d->S32, pass_Wv(d, dp), NV == 16 ? dp.Xt : X, Y, ld);
+}
+// One and two vectors always fill their pass (nv_pass).
+template <int NV>
+static void launch_stage(const Stage &st, const DevPlan &dp, DevState *d, const double *X, double *Y, ExtLd ld,
+                         hipStream_t s) {
+    if constexpr (NV > 2)
+        if (ld.n < NV) { launch_stage_ld<NV>(st, dp, d, X, Y, ld, s); return; }
+    launch_stage_ld<NV>(st, dp, d, X, Y, ld.ld, s);
 }
 
 static void collect_phase_ms(H2ERI_p h, DevState *d);
@@ -2563,11 +2579,17 @@ static void collect_phase_ms(H2ERI_p h, DevState *d);
 // polling, far beyond any dependency of a pass.
 static const int QUEUE_SPIN_LIMIT = 1 << 22;
 
-template <int NV>
-static void launch_queue(const DevPlan &dp, DevState *d, const double *X, double *Y, ExtLd ld, hipStream_t s) {
-    hipLaunchKernelGGL((queue_kernel<NV, false>), dim3(dp.q_grid), dim3(WG), 0, s, dp.d_q, dp.q_n,
+template <int NV, typename LD>
+static void launch_queue_ld(const DevPlan &dp, DevState *d, const double *X, double *Y, LD ld, hipStream_t s) {
+    hipLaunchKernelGGL((queue_kernel<NV, false, LD>), dim3(dp.q_grid), dim3(WG), 0, s, dp.d_q, dp.q_n,
                        dp.d_need, pass_ctr(d, dp), d->spin_limit, (const MolPtrs *)nullptr, dp.d_t64, dp.d_t32, dp.d_rt,
                        dp.d_vsrc, dp.d_rsrc, d->S64, d->S32, pass_Wv(d, dp), NV == 16 ? dp.Xt : X, Y, ld);
+}
+template <int NV>
+static void launch_queue(const DevPlan &dp, DevState *d, const double *X, double *Y, ExtLd ld, hipStream_t s) {
+    if constexpr (NV > 2)
+        if (ld.n < NV) { launch_queue_ld<NV>(dp, d, X, Y, ld, s); return; }
+    launch_queue_ld<NV>(dp, d, X, Y, ld.ld, s);
 }
 
 // One pass of the persistent executor on stream s (reset + queue launch).
@@ -3367,7 +3389,7 @@ void *H2ERI_group_create(const int nh, H2ERI_p *handles, const double *const *X_
     std::vector<MolPtrs> mols(nh);
     int dev = 0, ncu = 0, per = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue_kernel<1, true>, WG, 0) != hipSuccess) {
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (queue_kernel<1, true, long long>), WG, 0) != hipSuccess) {
         set_error(ERR_DEVICE, "H2ERI_group_create: occupancy query failed");
         delete g;
         return nullptr;
@@ -3442,10 +3464,10 @@ int H2ERI_group_matvec(void *group, void *stream) {
     }
     hipLaunchKernelGGL(queue_reset_kernel, dim3((std::max(g->q_nlist, QC_LISTS) + 255) / 256), dim3(256), 0, s, g->d_ctr,
                        g->q_nlist);
-    hipLaunchKernelGGL((queue_kernel<1, true>), dim3(g->q_grid), dim3(WG), 0, s, g->d_q, g->q_n, g->d_need,
+    hipLaunchKernelGGL((queue_kernel<1, true, long long>), dim3(g->q_grid), dim3(WG), 0, s, g->d_q, g->q_n, g->d_need,
                        g->d_ctr, QUEUE_SPIN_LIMIT, g->d_mols, (const BTask *)nullptr, (const BTask *)nullptr,
                        (const RTask *)nullptr, (const int *)nullptr, (const int *)nullptr, (const double *)nullptr,
-                       (const float *)nullptr, (double *)nullptr, (const double *)nullptr, (double *)nullptr, ExtLd{0, 1});
+                       (const float *)nullptr, (double *)nullptr, (const double *)nullptr, (double *)nullptr, 0LL);
     if (hipGetLastError() != hipSuccess) { set_error(ERR_DEVICE, "H2ERI_group_matvec: launch failed"); return -1; }
     return 0;
 }
