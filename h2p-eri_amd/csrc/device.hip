@@ -1258,6 +1258,7 @@ struct Storage {
     std::vector<MatRef> U;
     std::vector<BlkRef> B, D;
     double bytes_U = 0, bytes_B = 0, bytes_D = 0;   // algorithmic (U counted twice)
+    int n_blk = 0;   // B and D blocks stored
 
     MatRef store(const double *src, int nrow, int ncol, bool fp32) {
         MatRef m;
@@ -1280,6 +1281,7 @@ struct Storage {
     BlkRef store_blk(H2E_dense_mat_p b, bool fp32, double &bytes) {
         BlkRef r;
         if (!b || b->nrow == 0 || b->ncol == 0) return r;
+        n_blk++;
         const double esz = fp32 ? 4.0 : 8.0;
         if (b->ld >= 0) {
             r.M = store(b->data, b->nrow, b->ncol, fp32);
@@ -2520,18 +2522,40 @@ static DevPlan *get_plan(H2ERI_p h, int nv) {
     return nullptr;
 }
 
-// Plan of the next pass for `rem` vectors left (nv_pass); when the workspace
+// Bytes of stored blocks (U among them) per B or D block below which five
+// vectors of the staged executor run as 4 + 1.
+static const double SMALL_BLOCK = 128.0 * 1024.0;
+
+// Width of the next pass for `rem` vectors left: nv_pass, except that five
+// vectors of a representation of small blocks (globular molecules) run as
+// 4 + 1 in the staged executor.  Its 8-vector tiles pay for eight vectors
+// there, and the matrix data they save are few: (H2O)8 to (H2O)64, 26 to 61 KB
+// per block, take 0.87 to 0.98 of the padded pass's time as 4 + 1 ((H2O)12
+// FP64 287 us for 322, (H2O)40 FP32-stored 1,113 for 1,236); (H2O)10 and
+// alkanes, 198 KB and more, 1.04 to 1.94 times it; the persistent executor,
+// 1.1 times and more.  Six vectors are even (0.97 to 1.06) on small blocks.
+static int pass_width(H2ERI_p h, int rem) {
+    const int nv = nv_pass(rem);
+    if (rem != 5 || h->BD_JIT) return nv;
+    const DevState *d = dstate(h);
+    const double bytes = 0.5 * d->st.bytes_U + d->st.bytes_B + d->st.bytes_D;
+    return d->cfg[nv_index(nv)].executor == 0 && bytes < SMALL_BLOCK * d->st.n_blk ? 4 : nv;
+}
+
+// Plan of the next pass for `rem` vectors left (pass_width); when the workspace
 // of a pass wider than that finds no room on the device or exceeds what a plan
 // can address, the widest of at most `rem` vectors, from then on.
 static DevPlan *pass_plan(H2ERI_p h, int rem) {
-    const int nv = nv_pass(rem), i = nv_index(nv);
+    if (!upload_storage(h)) return nullptr;
+    const int nv = pass_width(h, rem), i = nv_index(nv);
     const bool padded = nv > rem;
-    if (!padded || !dstate_get(h)->no_pad[i]) {
-        if (padded) dstate(h)->no_room = false;
+    DevState *d = dstate(h);
+    if (!padded || !d->no_pad[i]) {
+        d->no_room = false;
         DevPlan *dp = get_plan(h, nv);
-        if (dp || !padded || h->BD_JIT || !dstate(h)->st_ready) return dp;
-        if (!dstate(h)->no_room && h2eri_last_error() != ERR_UNSUPPORTED) return nullptr;
-        dstate(h)->no_pad[i] = true;
+        if (dp || !padded || h->BD_JIT) return dp;
+        if (!d->no_room && h2eri_last_error() != ERR_UNSUPPORTED) return nullptr;
+        d->no_pad[i] = true;
         (void)hipGetLastError();
         h2eri_clear_error();
     }
@@ -2722,7 +2746,7 @@ static void collect_phase_ms(H2ERI_p h, DevState *d) {
     h->timers[MV_VOP_TIMER_IDX] += d->phase_ms[PH_GATHER] * 1e-3;
 }
 
-// Batched device matvec: nvec vectors, processed in passes of 16, 8, 4, 2, 1.
+// Batched device matvec: nvec vectors, in the passes that pass_plan chooses.
 static bool matvec_multi_dev_impl(H2ERI_p h, int nvec, const double *X, double *Y, hipStream_t s) {
     if (h->BD_JIT) {   // timed like the stored form: the reference's phase timer slots
         if (!upload_storage(h)) return false;
