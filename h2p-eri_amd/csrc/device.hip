@@ -1445,6 +1445,13 @@ static void free_dev(void *&p) {
     if (p) { (void)hipFree(p); p = nullptr; }
 }
 
+// Whether a caller captures stream s.
+static bool captured(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+    return cap != hipStreamCaptureStatusNone;
+}
+
 // Near-field streams of the staged executor, shared by the handles of a
 // device: one per stream that callers pass.  Passes on one caller stream run
 // one after another, so sharing costs them nothing, and passes on different
@@ -2544,13 +2551,17 @@ static int pass_width(H2ERI_p h, int rem) {
 
 // Plan of the next pass for `rem` vectors left (pass_width); when the workspace
 // of a pass wider than that finds no room on the device or exceeds what a plan
-// can address, the widest of at most `rem` vectors, from then on.
-static DevPlan *pass_plan(H2ERI_p h, int rem) {
+// can address, the widest of at most `rem` vectors, from then on; also while
+// the caller captures stream s, when no plan can be made, and the wider one is
+// not there.
+static DevPlan *pass_plan(H2ERI_p h, int rem, hipStream_t s) {
     if (!upload_storage(h)) return nullptr;
     const int nv = pass_width(h, rem), i = nv_index(nv);
     const bool padded = nv > rem;
     DevState *d = dstate(h);
-    if (!padded || !d->no_pad[i]) {
+    const DevPlan &p = d->plans[i];
+    const bool there = p.ready && (d->cfg[i].executor != 1 || p.q_ready);
+    if (!padded || there || !(d->no_pad[i] || captured(s))) {
         d->no_room = false;
         DevPlan *dp = get_plan(h, nv);
         if (dp || !padded || h->BD_JIT) return dp;
@@ -2695,10 +2706,8 @@ static bool run_matvec(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, dou
     if (has_side) {
         // near-field launches on their own stream, forked after everything
         // already enqueued on s and joined before the gather
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (s && hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
         hipStream_t side = nullptr;
-        if (cap != hipStreamCaptureStatusNone) {
+        if (captured(s)) {
             if (!d->side) HIP_OK(hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking));
             side = d->side;
         } else if (!near_stream(d, s, !d->ws_Wv, side)) {
@@ -2770,7 +2779,7 @@ static bool matvec_multi_dev_impl(H2ERI_p h, int nvec, const double *X, double *
     int done = 0;
     while (done < nvec) {
         const int rem = nvec - done;
-        DevPlan *dp = pass_plan(h, rem);
+        DevPlan *dp = pass_plan(h, rem, s);
         if (!dp) return false;
         const int n = std::min(dp->P.nv, rem);
         if (!run_matvec(h, dstate(h), *dp, X + done * N, Y + done * N, n, s)) return false;
@@ -3057,7 +3066,7 @@ int H2ERI_graph_capture(H2ERI_p h, const int kind, const int n, const double *in
         if (!upload_storage(h)) return -1;
         for (int done = 0; done < n;) {
             const int rem = n - done;
-            const DevPlan *dp = pass_plan(h, rem);
+            const DevPlan *dp = pass_plan(h, rem, nullptr);
             if (!dp) return -1;
             done += std::min(dp->P.nv, rem);
         }
