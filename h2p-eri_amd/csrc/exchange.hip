@@ -568,6 +568,7 @@ static void kstate_release(KState *k) {
                    (void **)&k->block, (void **)&k->direct, (void **)&k->gtasks, (void **)&k->Ds, (void **)&k->sbf};
     for (void **p : ps) kfree(*p);
     k->ready = false;
+    k->resident = 0;
     k->P = KPlan();
 }
 
@@ -1263,9 +1264,20 @@ int H2ERI_exchange_plan_check(H2ERI_p h, double *out4) {
         out4[0] = P.flops;
         out4[1] = (double)P.terms.size();
         const double nacc = 2.0 * P.nacc * nn2;
-        out4[2] = 8.0 * ((double)P.PB.size() + (double)P.CB.size() + (double)P.nSC + nacc + 3.0 * nn2) +
-                  4.0 * ((double)P.bfidx.size() + P.qptr.size() + P.mptr.size() + P.gptr.size() + P.bptr.size()) +
-                  8.0 * ((double)P.qent.size() + P.ment.size() + P.brow.size()) + 16.0 * (double)P.ge.size();
+        // as k_upload: operands and their padding, accumulators, D, K and the
+        // screened D, lists, terms, tasks (an empty array takes 64 bytes)
+        const double operands = (double)P.PB.size() + (double)P.CB.size() + (double)P.nSC + 3.0 * KPAD;
+        out4[2] = 8.0 * (operands + nacc + 3.0 * nn2);
+        auto add = [&](size_t n, size_t size) { out4[2] += n > 0 ? (double)n * (double)size : 64.0; };
+        for (const auto *v : {&P.bfidx, &P.qptr, &P.mptr, &P.gptr, &P.bptr}) add(v->size(), sizeof(int));
+        for (const auto *v : {&P.qent, &P.ment, &P.brow}) add(v->size(), sizeof(int2));
+        add(P.ge.size(), sizeof(int4));
+        add(P.terms.size(), sizeof(KTerm));
+        add(P.gemms.size(), sizeof(KGemm));
+        add(P.nodes.size(), sizeof(KNode));
+        add(P.gtasks.size(), sizeof(KGemmTask));
+        for (const auto *v : {&P.block, &P.direct}) add(v->size(), sizeof(KTask));
+        add((size_t)h->nshell + 1, sizeof(int));
         out4[3] = (double)P.nSC + nacc;
     }
     return (int)P.terms.size();
