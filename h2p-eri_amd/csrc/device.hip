@@ -107,7 +107,7 @@ __device__ __forceinline__ RTask uniform(const RTask &a) {
 
 // The external vectors of a padded pass (fewer vectors than its width NV):
 // vector v at v * ld, n of them; the others read as zero and are not written.
-// A full pass takes the bare stride: the tests of v < n in it cost 2 to 4% of
+// A full pass takes the bare stride: the tests of v < n in it cost 2 to 6% of
 // an 8-vector pass ((H2O)32 staged, FP64: 705 us in place of 663) and 28 more
 // spilled SGPRs in its persistent kernel.  A stride below zero: an
 // element-major copy.
@@ -115,10 +115,7 @@ struct ExtLd {
     long long ld;
     int n;
 };
-__host__ __device__ __forceinline__ long long ext_ld(long long ld) { return ld; }
-__host__ __device__ __forceinline__ long long ext_ld(const ExtLd &e) { return e.ld; }
-__device__ __forceinline__ bool ext_has(long long, int) { return true; }
-__device__ __forceinline__ bool ext_has(const ExtLd &e, int v) { return v < e.n; }
+template <typename LD> constexpr bool is_padded() { return std::is_same_v<LD, ExtLd>; }
 
 static const int WG = 256;       // threads per workgroup (4 waves)
 // Output elements per reduce task: 1024 / NV values fill the task's 256
@@ -181,7 +178,10 @@ __device__ __forceinline__ void stage_vec(const int *__restrict__ vsrc, int b, i
                                           const double *__restrict__ Wv, const double *__restrict__ X, LD ldx,
                                           double *dst, int tid) {
     const int s0 = vsrc[b];
-    if (s0 < 0 && ext_ld(ldx) < 0) {   // the external input as an element-major copy (NV values per element)
+    long long ld;
+    if constexpr (is_padded<LD>()) ld = ldx.ld;
+    else ld = ldx;
+    if (s0 < 0 && ld < 0) {   // the external input as an element-major copy (NV values per element)
         const double *p = X + (long long)(-s0 - 1 + off) * NV;
         for (int q = tid; q < n * NV; q += NT) dst[XS == NV ? q : (q / NV) * XS + q % NV] = p[q];
         return;
@@ -190,7 +190,10 @@ __device__ __forceinline__ void stage_vec(const int *__restrict__ vsrc, int b, i
         const double *p = X + (long long)(-s0 - 1 + off);
         for (int i = tid; i < n; i += NT) {
             #pragma unroll
-            for (int v = 0; v < NV; v++) dst[i * XS + v] = ext_has(ldx, v) ? p[v * ext_ld(ldx) + i] : 0.0;
+            for (int v = 0; v < NV; v++) {
+                if constexpr (is_padded<LD>()) dst[i * XS + v] = v < ldx.n ? p[(long long)v * ld + i] : 0.0;
+                else dst[i * XS + v] = p[(long long)v * ld + i];
+            }
         }
         return;
     }
@@ -942,7 +945,11 @@ __device__ void reduce_task(const RTask &task, const int *__restrict__ src, doub
     auto put = [&](int q, double v) {
         if (t.flags & 1) {
             const int i = q / NV, w = q - i * NV;
-            if (ext_has(ldy, w)) Y[w * ext_ld(ldy) + t.dst + i] = v;
+            if constexpr (is_padded<LD>()) {
+                if (w < ldy.n) Y[(long long)w * ldy.ld + t.dst + i] = v;
+            } else {
+                Y[(long long)w * ldy + t.dst + i] = v;
+            }
         } else {
             wst<COH>(Wv + t.dst * NV + q, v);
         }
@@ -1369,7 +1376,11 @@ static inline bool nv_valid(int nv) { return nv == 1 || nv == 2 || nv == 4 || nv
 // / 0.34 / 0.40 / 0.50 / 0.68, C100H202 1.51 / - / 2.02 / 2.73 / 3.39, (H2O)64
 // 0.73 / - / 1.08 / 1.80 / 2.38: 3 vectors as 4 take 0.40 in place of 0.63,
 // 5 as 8 0.50 (2.73, 1.80) in place of 0.70 (3.53, 1.81), 9 as 16 0.68
-// (3.39, 2.38) in place of 0.79 (4.24, 2.53).
+// (3.39, 2.38) in place of 0.79 (4.24, 2.53).  Untuned, staged, from H2O to
+// (H2O)64 and C3H8 to C50H102, both precisions, the passes that add up to 3 /
+// 6 / 7 / 9 to 15 vectors take 1.07 to 1.66 / 0.97 to 2.08 / 1.28 to 2.9 /
+// 0.98 to 2.8 times the padded one; persistent 1.1 times and more; five
+// vectors: pass_width.
 static inline int nv_pass(int rem) { return rem > 8 ? 16 : (rem > 4 ? 8 : (rem > 2 ? 4 : rem)); }
 
 // Tuning configuration of one batch width.
