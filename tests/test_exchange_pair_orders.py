@@ -54,3 +54,19 @@ def test_exchange_sums_every_row(twice, tmp_path):
     D = M.density(atoms, 41, M.rng_for(96))
     print(f"exchange with repeated pairs: {h.nbf} functions, twice {twice}", flush=True)
     assert relerr(h.build_exchange(D), oracle_bind.Oracle(p).exchange(D)) < 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("twice", [False, True])
+def test_coulomb_sums_every_row(twice, tmp_path):
+    from h2eri import molecules as M
+    p = str(tmp_path / "r.rep")
+    h, atoms = _with_repeated_pairs(p, twice)
+    o = oracle_bind.Oracle(p)
+    o.lib.orc_set_threads(1)   # its threads add rows of one element of J without a lock
+    Ds = np.stack([M.density(atoms, 41, M.rng_for(97 + k)) for k in range(5)])
+    Js = h.build_coulomb_multi(Ds)
+    ref = [o.coulomb(D) for D in Ds]
+    o.lib.orc_set_threads(0)
+    for J, R in zip(Js, ref):
+        assert relerr(J, R) < 1e-12
