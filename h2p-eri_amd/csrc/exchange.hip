@@ -192,15 +192,19 @@ __device__ __forceinline__ void kfours(int n, F f) {
 // What bounds it: FP64 MFMA issue together with VALU issue, which it does not
 // overlap: an MFMA takes 64 cycles of its SIMD, at most 62 TFLOP/s on this
 // card, and every VALU instruction beside it adds about two (twelve per MFMA:
-// 44 TFLOP/s).  C30H62 issues 193 GFLOP of MFMAs, half of them padding (the
-// entries of an n come in sixteens, those of a q in fours): 3.1 ms of the 5.15.
+// 44 TFLOP/s).  C30H62 issues 189 GFLOP of MFMAs, half of them padding (the
+// entries of an n come in sixteens, those of a q in fours): 3.05 ms of the
+// 5.15, the MFMA units busy in 48% of the cycles.  (H2O)64, whose ranks of
+// about 13 fill a step of 16 t badly, issues 1,073 GFLOP for 460: 42% of its
+// 33.3 ms.
 // So the loops are kept short of VALU work: fours that both functions have
 // meet their D operands unmasked, rows without an entry add into a sink
 // instead of being masked, K block bytes and flags are in the lists.  Masks,
 // index arithmetic and register copies in the loops: 5.50 ms.
-// What is left beside it: a wave waits at a step's two barriers for the one
-// with most work (0.6 ms), the loads of a new t (0.2) and the LDS atomics
-// (0.15).  Operand latency is covered: rows padded to whole 128-byte lines
+// What is left beside it, from timing builds of the 5.50 ms form: a wave waits
+// at a step's two barriers for the one with most work (0.6 ms), the loads of a
+// new t (0.2) and the LDS atomics (0.15).  Operand latency is covered there:
+// rows padded to whole 128-byte lines
 // (5.55 ms), a second block in flight (5.52) and the next step's D in
 // registers (5.63) changed nothing or cost.  16 waves per CU (128 VGPRs, two
 // workgroups by LDS): 40 entries in registers spill (5.86 ms against 5.64).

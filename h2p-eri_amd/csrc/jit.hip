@@ -378,9 +378,8 @@ __host__ __device__ inline void jit_density(const JitView &v, int c) {
 }
 
 // One thread per centre, workgroups of one order, the highest (and slowest)
-// first.  The E tables of order 4 take 256 VGPRs, two waves per SIMD; the
-// centres are too few to use more (C30H62: 77,249, 1,207 waves of the
-// 2,048 that fit).
+// first.  The E tables of order 4 take 256 VGPRs and 30 AGPRs, so one wave per
+// SIMD: 1,024 fit, C30H62 has 1,236 (77,249 centres; 31 us).
 __global__ void __launch_bounds__(256) jit_density_kernel(JitView v) {
     int b = blockIdx.x, L = JIT_OMAX;
     for (; L > 0; L--) {
@@ -465,7 +464,8 @@ __host__ __device__ inline void jit_rows_any(const JitView &v, int e, int sub) {
     }
 }
 // Eight lanes per entry; entries are sorted by class, so a wave's eight
-// entries take one path.
+// entries take one path.  256 VGPRs and 86 AGPRs, one wave per SIMD (C30H62:
+// 3,584 waves, 28 us).
 static const int JIT_RLANES = 8;
 __global__ void __launch_bounds__(256) jit_rows_kernel(JitView v, int nout) {
     const int i = (blockIdx.x * 256 + threadIdx.x) / JIT_RLANES;
@@ -474,10 +474,16 @@ __global__ void __launch_bounds__(256) jit_rows_kernel(JitView v, int nout) {
 }
 
 // The potential kernels, bound by FP64 vector issue: C30H62 has 5.4e8 pairs
-// of centres (1.08e9 primitive quartets), 45 to 250 vector instructions each,
-// 1.2 ms at one instruction per SIMD and four cycles; the three launches take
-// 2.1 ms together, in place of 255 ms when every quartet formed its Cartesian
-// components.  One wave per task, lanes over bra centres (their
+// of centres (1.08e9 primitive quartets) at 45 (s-s) to about 2,000 (order 4
+// with 4) vector instructions, 104 on average (8.8e8 of whole waves, idle
+// lanes among them): 1.5 ms at one per SIMD and four cycles.  The three
+// launches take 1.18 + 0.63 + 0.20 ms (total orders <= 2, 3 and 4, >= 5), in
+// place of 255 ms when every quartet formed its Cartesian components.
+// Counters: vector instructions issue in 86%, 77% and 54% of their SIMD
+// cycles, 70%, 82% and 87% of them FP64 arithmetic.  The last one keeps 474
+// registers (one wave per SIMD, so latency shows) and moves 114 VGPRs through
+// AGPRs; the first loses 16% of its LDS cycles to bank conflicts of the
+// table.  One wave per task, lanes over bra centres (their
 // exponent, position and potential in registers), a loop over the ket
 // centres, which are the same for every lane: their data come through scalar
 // loads and feed the FMAs from scalar registers.  A task whose centres fill

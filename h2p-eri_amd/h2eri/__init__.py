@@ -423,7 +423,7 @@ class H2ERI:
         _check(self.lib)
 
     def set_exchange_scratch(self, nbytes):
-        """Bound of the exchange build's intermediate G (bytes); the terms run in chunks that fit it."""
+        """Bound of the exchange build's K accumulators (bytes): up to four copies of (K1, K_diag), at least one."""
         self.lib.H2ERI_set_exchange_scratch(self.h, float(nbytes))
         _check(self.lib)
 
