@@ -60,7 +60,9 @@ def log(*a):
 # ---------------------------------------------------------------------------
 def pass_widths(n):
     """Widths of the passes of a batched call of n vectors (16 per pass, the
-    last vectors in the narrowest of 1, 2, 4, 8, 16 that holds them)."""
+    last vectors in the narrowest of 1, 2, 4, 8, 16 that holds them; five of a
+    representation of small blocks, which the staged executor runs as 4 + 1,
+    count as one pass)."""
     out = []
     while n > 0:
         w = 16 if n > 8 else 8 if n > 4 else 4 if n > 2 else n

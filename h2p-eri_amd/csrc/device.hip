@@ -2549,9 +2549,10 @@ static const double SMALL_BLOCK = 128.0 * 1024.0;
 // 4 + 1 in the staged executor.  Its 8-vector tiles pay for eight vectors
 // there, and the matrix data they save are few: (H2O)8 to (H2O)64, 26 to 61 KB
 // per block, take 0.87 to 0.98 of the padded pass's time as 4 + 1 ((H2O)12
-// FP64 287 us for 322, (H2O)40 FP32-stored 1,113 for 1,236); (H2O)10 and
-// alkanes, 198 KB and more, 1.04 to 1.94 times it; the persistent executor,
-// 1.1 times and more.  Six vectors are even (0.97 to 1.06) on small blocks.
+// FP64 287 us for 322, (H2O)40 FP32-stored 1,113 for 1,236; (H2O)6 1.08 and
+// (H2O)32 1.01 and 1.07); (H2O)10 and alkanes, 198 KB and more, 1.04 to 1.94
+// times it; the persistent executor, 1.1 times and more.  Six vectors are even
+// (0.97 to 1.06) on small blocks.
 static int pass_width(H2ERI_p h, int rem) {
     const int nv = nv_pass(rem);
     if (rem != 5 || h->BD_JIT) return nv;
