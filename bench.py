@@ -524,7 +524,8 @@ def single_workload(args):
 def jit_measure(torch, stream, cfg=1, reps=3, host_compare=True):
     """The on-the-fly form (BD_JIT = 1: B and D evaluated from the shell
     pairs in every matvec) on C30H62 at reltol 1e-6: ms per FP64 matvec
-    (HIP events, device vectors), with the integral work of one matvec."""
+    (HIP events, device vectors), with the integral values its blocks hold (the
+    Hermite form applies them without forming them)."""
     import numpy as np
 
     import h2eri
@@ -550,7 +551,7 @@ def jit_measure(torch, stream, cfg=1, reps=3, host_compare=True):
         ms.append(e0.elapsed_time(e1))
     best = min(ms)
     log(f"[bench] on-the-fly B/D ({M.workload_name(cfg)}): {best:.1f} ms per matvec, "
-        f"{st['eri_values'] / best / 1e6:.2f} G integrals/s")
+        f"blocks of {st['eri_values'] / best / 1e6:.2f} G integrals/s")
     rec = {"workload": f"{M.workload_name(cfg)} cc-pVDZ, reltol {reltol:g}", "krnl_mat_size": hj.n,
            "ms_per_matvec": round(best, 3), "ms_all": [round(m, 3) for m in ms],
            "integrals_per_matvec": st["eri_values"], "shell_quartets_per_matvec": st["quartets"],
@@ -601,8 +602,8 @@ def jit_host_compare(torch, stream, cfg=0, reps=3):
             "cpu_threads": threads, "gpu_ms_per_matvec": round(min(ms), 3),
             "ratio": round(cpu_s * 1e3 / min(ms), 1),
             "note": "CPU: the host integral engine evaluating the dense B and D blocks (B and D construction "
-                    "timers of a dense build); GPU: one on-the-fly matvec, which evaluates the same blocks "
-                    "from both sides and applies them"}
+                    "timers of a dense build); GPU: one on-the-fly matvec, which applies the same blocks "
+                    "from both sides through Hermite potentials, without forming them"}
 
 
 def exchange_measure(h, torch, D, D_dev, stream):

@@ -522,7 +522,8 @@ int H2ERI_plan_emulate(H2ERI_p h2eri, const int ub_bits, const int nv, const dou
 int H2ERI_jit_emulate(H2ERI_p h2eri, const double *x, double *y);
 
 /* Work of one BD_JIT matvec, counted on the host: out4 = {tasks, shell
- * quartets, primitive quartets, integral values}.  Returns 0, -1 on failure. */
+ * quartets, primitive quartets, integral values of the blocks applied (no
+ * integral is formed)}.  Returns 0, -1 on failure. */
 int H2ERI_jit_stats(H2ERI_p h2eri, double *out4);
 
 /* Host verification of the persistent executor's queue (no HIP call, tests
