@@ -1463,53 +1463,120 @@ static bool captured(hipStream_t s) {
     return cap != hipStreamCaptureStatusNone;
 }
 
-// Near-field streams of the staged executor, shared by the handles of a
-// device: one per stream that callers pass.  Passes on one caller stream run
-// one after another, so sharing costs them nothing, and passes on different
-// streams do not wait for each other's near field.  A process has four
-// hardware queues and its streams are dealt onto them: with a stream per
-// handle the seventh handle's near field fell onto its caller's queue and ran
-// after the sweeps instead of beside them ((H2O)16 FP32-stored, one J: 148 us
-// on the other handles, 217 on that one; C10H22 148 and 217).  So there are at
-// most NEAR_MAX of them, beside the caller's; further caller streams share.
-// H2ERI_upload makes the default stream's; the last handle gives all back.  A
-// stream under capture belongs to its capture until that ends: passes on a
-// captured stream fork to the handle's own stream (DevState::side).
-static const int NEAR_MAX = 3, NEAR_DEVICES = 64;
+// Near-field streams of the staged executor: a few per device, shared by its
+// handles.  Passes on one caller stream run one after another, so sharing costs
+// them nothing.  A process has four hardware queues onto which its streams are
+// dealt, and a near field on its caller's queue runs after the sweeps instead
+// of beside them: with a stream per handle that was the seventh handle's lot
+// ((H2O)16 FP32-stored, one J: 148 us on the other handles, 217 on that one;
+// C10H22 148 and 217), with one per caller stream that of the first stream a
+// program made after its handle.  So the first pass on a caller stream tries a
+// near-field stream out: a kernel on the caller's waits, at most NEAR_WAIT, for
+// one on the near-field stream, which cannot start before it on the same
+// queue; later passes read the answer when it is there and take the next
+// near-field stream if need be.  The host waits for nothing.  A stream under
+// capture belongs to its capture until that ends: passes on a captured stream
+// fork to the handle's own stream (DevState::side).  The last handle of a
+// device gives everything back.
+static const int NEAR_MAX = 3, NEAR_CALLERS = 16, NEAR_DEVICES = 64;
+static const long long NEAR_WAIT = 20000;   // ticks of 10 ns
+__global__ void near_wait_kernel(const int *flag, int gen, int *seen) {
+    const long long t0 = wall_clock64();
+    int ok = 0;
+    while (!ok && wall_clock64() - t0 < NEAR_WAIT)
+        ok = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= gen;
+    __hip_atomic_store(seen, 2 * gen + ok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ void near_set_kernel(int *flag, int gen) {
+    __hip_atomic_store(flag, gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+struct NearCaller {
+    hipStream_t s;
+    int pick;       // its near-field stream
+    int left;       // streams not tried yet
+    int gen;        // number of the trial under way, 0: none
+};
 struct NearPool {
-    int users = 0, n = 0;
-    hipStream_t caller[NEAR_MAX], side[NEAR_MAX];
+    int users = 0, n = 0, ncall = 0, next = 0, gen = 0;
+    hipStream_t side[NEAR_MAX];
+    NearCaller c[NEAR_CALLERS];
+    int *flag = nullptr, *seen = nullptr;   // per caller: on the device, in host memory
 };
 static std::mutex g_near_mu;
 static NearPool g_near[NEAR_DEVICES];
+
+static void near_free(NearPool &p) {
+    (void)hipDeviceSynchronize();   // a trial may be under way
+    for (int i = 0; i < p.n; i++) (void)hipStreamDestroy(p.side[i]);
+    if (p.flag) (void)hipFree(p.flag);
+    if (p.seen) (void)hipHostFree(p.seen);
+    p = NearPool();
+}
 
 static void near_release(DevState *d) {
     if (d->near_dev < 0) return;
     std::lock_guard<std::mutex> lk(g_near_mu);
     NearPool &p = g_near[d->near_dev];
     d->near_dev = -1;
-    if (--p.users > 0) return;
-    for (int i = 0; i < p.n; i++) (void)hipStreamDestroy(p.side[i]);
-    p.n = 0;
+    if (--p.users == 0) near_free(p);
 }
 
-// The near-field stream for passes on caller stream s; without `create` one
-// that is there, if any.
-static bool near_stream(DevState *d, hipStream_t s, bool create, hipStream_t &out) {
-    if (d->near_dev != d->dev) near_release(d);
-    if (d->dev < 0 || d->dev >= NEAR_DEVICES) { set_error(ERR_DEVICE, "near-field stream: device %d", d->dev); return false; }
+static bool near_make(NearPool &p) {
+    for (; p.n < NEAR_MAX; p.n++) HIP_OK(hipStreamCreateWithFlags(&p.side[p.n], hipStreamNonBlocking));
+    HIP_OK(hipMalloc(&p.flag, NEAR_CALLERS * sizeof(int)));
+    HIP_OK(hipMemset(p.flag, 0, NEAR_CALLERS * sizeof(int)));
+    HIP_OK(hipHostMalloc((void **)&p.seen, NEAR_CALLERS * sizeof(int)));
+    for (int i = 0; i < NEAR_CALLERS; i++) p.seen[i] = 0;
+    HIP_OK(hipDeviceSynchronize());
+    return true;
+}
+
+// The device's near-field streams, for handle d until it is released.
+static bool near_prepare(DevState *d) {
+    if (d->near_dev == d->dev) return true;
+    near_release(d);
+    if (d->dev < 0 || d->dev >= NEAR_DEVICES) { set_error(ERR_DEVICE, "near-field streams: device %d", d->dev); return false; }
     std::lock_guard<std::mutex> lk(g_near_mu);
     NearPool &p = g_near[d->dev];
-    if (d->near_dev < 0) { p.users++; d->near_dev = d->dev; }
-    for (int i = 0; i < p.n; i++)
-        if (p.caller[i] == s) { out = p.side[i]; return true; }
-    if (p.n < NEAR_MAX && (create || p.n == 0)) {
-        HIP_OK(hipStreamCreateWithFlags(&p.side[p.n], hipStreamNonBlocking));
-        p.caller[p.n++] = s;
-        out = p.side[p.n - 1];
-        return true;
+    if (p.users == 0 && !near_make(p)) { near_free(p); return false; }
+    p.users++;
+    d->near_dev = d->dev;
+    return true;
+}
+
+// The near-field stream for a pass on caller stream s (not under capture).
+static bool near_stream(DevState *d, hipStream_t s, hipStream_t &out) {
+    if (!near_prepare(d)) return false;
+    std::lock_guard<std::mutex> lk(g_near_mu);
+    NearPool &p = g_near[d->dev];
+    int i = 0;
+    while (i < p.ncall && p.c[i].s != s) i++;
+    if (i == p.ncall) {
+        if (p.ncall < NEAR_CALLERS) p.ncall++;
+        else i = p.next, p.next = (p.next + 1) % NEAR_CALLERS;
+        p.c[i].s = s;
+        p.c[i].pick = i % NEAR_MAX;
+        p.c[i].left = NEAR_MAX;
+        p.c[i].gen = 0;
     }
-    out = p.side[((uintptr_t)s >> 6) % p.n];
+    NearCaller &c = p.c[i];
+    bool trial = c.left == NEAR_MAX && c.gen == 0;
+    const int seen = __atomic_load_n(&p.seen[i], __ATOMIC_RELAXED);
+    if (c.gen && seen >> 1 == c.gen) {
+        if (!(seen & 1) && c.left > 0) {   // on the caller's queue
+            c.pick = (c.pick + 1) % NEAR_MAX;
+            trial = true;
+        }
+        c.gen = 0;
+    }
+    if (trial) {
+        c.left--;
+        c.gen = ++p.gen;
+        hipLaunchKernelGGL(near_wait_kernel, dim3(1), dim3(1), 0, s, p.flag + i, c.gen, p.seen + i);
+        hipLaunchKernelGGL(near_set_kernel, dim3(1), dim3(1), 0, p.side[c.pick], p.flag + i, c.gen);
+        HIP_OK(hipGetLastError());
+    }
+    out = p.side[c.pick];
     return true;
 }
 
@@ -2722,7 +2789,7 @@ static bool run_matvec(H2ERI_p h, DevState *d, DevPlan &dp, const double *X, dou
         if (captured(s)) {
             if (!d->side) HIP_OK(hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking));
             side = d->side;
-        } else if (!near_stream(d, s, !d->ws_Wv, side)) {
+        } else if (!near_stream(d, s, side)) {
             return false;
         }
         if (!d->ev_fork) HIP_OK(hipEventCreateWithFlags(&d->ev_fork, hipEventDisableTiming));
@@ -3145,8 +3212,7 @@ size_t H2ERI_upload(H2ERI_p h) {
     DevState *d = dstate(h);
     // everything a single-vector pass needs besides its vectors, so that the
     // allocation-free entry point finds it in place
-    hipStream_t near;
-    if (!near_stream(d, nullptr, true, near)) return 0;
+    if (!near_prepare(d)) return 0;
     if (!d->side && hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking) != hipSuccess) { set_error(ERR_DEVICE, "stream"); return 0; }
     if (!d->ev_fork && hipEventCreateWithFlags(&d->ev_fork, hipEventDisableTiming) != hipSuccess) { set_error(ERR_DEVICE, "event"); return 0; }
     if (!d->ev_join && hipEventCreateWithFlags(&d->ev_join, hipEventDisableTiming) != hipSuccess) { set_error(ERR_DEVICE, "event"); return 0; }

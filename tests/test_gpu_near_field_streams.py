@@ -1,8 +1,8 @@
-"""The near field's stream is shared by the handles of a process: J of a
-handle takes the same time whichever of many handles it is (a stream per handle
-shares a hardware queue with its caller on some of them, 1.45 times the time),
-and handles on several streams, in several threads and beside a capture keep
-their results."""
+"""The near field's streams are shared by the handles of a process: J of a
+handle takes the same time whichever of many handles it is and whichever stream
+it is called on (a near-field stream that shares its caller's hardware queue
+takes 1.45 times the time), and handles on several streams, in several threads
+and beside a capture keep their results."""
 import threading
 import time
 
@@ -47,6 +47,28 @@ def test_every_handle_is_as_fast(rep):
         J0 = J if J0 is None else J0
         assert torch.equal(J, J0)
     print("J of one density, ms by handle:", " ".join(f"{m:.3f}" for m in ms), flush=True)
+    assert max(ms) < 1.2 * float(np.median(ms))
+
+
+def test_every_stream_is_as_fast(rep):
+    import h2eri
+    import torch
+    D = torch.from_numpy(rep[1]).to("cuda:0")
+    J = torch.empty_like(D)
+    h = h2eri.H2ERI.load(rep[0])
+    h.upload()
+    ms = []
+    for st in [torch.cuda.default_stream()] + [torch.cuda.Stream() for _ in range(7)]:
+        best = 1e9
+        for _ in range(8):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(50):
+                h.build_coulomb_dev(D.data_ptr(), J.data_ptr(), st.cuda_stream)
+            torch.cuda.synchronize()
+            best = min(best, (time.perf_counter() - t) / 50 * 1e3)
+        ms.append(best)
+    print("J of one density, ms by caller stream:", " ".join(f"{m:.3f}" for m in ms), flush=True)
     assert max(ms) < 1.2 * float(np.median(ms))
 
 
